@@ -203,17 +203,6 @@ __device__ __forceinline__ double lane_value(double v, int src) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// one lane-pair stage of the pivot search: keep the larger value, the
-// smaller row-major index on ties
-template <int S>
-__device__ __forceinline__ void pivot_stage(double &big, int &best) {
-  const double pb = partner<S>(big);
-  const int pi = partner<S>(best);
-  const bool t = (pb > big) | ((pb == big) & (pi < best));
-  big = t ? pb : big;
-  best = t ? pi : best;
-}
-
 constexpr int kSmallThreads = 256;       // 4 workgroup partials per thread
 
 // an instance of a batch has ended: fold it into the summary, which is done
@@ -245,78 +234,200 @@ __device__ __forceinline__ double sum_partials(const double *__restrict__ src, i
   return s;
 }
 
-// Gauss-Jordan of k_diis_small: columns per lane (8 groups of lanes, n1 <= 25)
-constexpr int kGJCols = 4;
+// largest 32-bit value over the wave (the DPP combines of wave_sum)
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
+  v = max(v, partner_u32<5>(v));
+  v = max(v, partner_u32<4>(v));
+  v = max(v, partner_u32<3>(v));
+  v = max(v, partner_u32<2>(v));
+  v = max(v, partner_u32<1>(v));
+  v = max(v, partner_u32<0>(v));
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+}
 
-// the columns of wave W's two groups, W + 8 j (lanes 0..31) and W + 4 + 8 j
-// (lanes 32..63), of row lane & 31; lane L < kB holds row L of B in a
-// (static register indices; the upper half takes its row from lane L - 32)
-template <int W>
-__device__ __forceinline__ void group_columns(const double (&a)[kB], double (&g)[kGJCols]) {
+// max(|a|, |b|) (fmax would first quieten each operand)
+__device__ __forceinline__ double max_abs(double a, double b) {
+  double m;
+  asm("v_max_f64 %0, |%1|, |%2|" : "=v"(m) : "v"(a), "v"(b));
+  return m;
+}
+
+// Gauss-Jordan with full pivoting on the bordered system of k_diis_small,
+// n1 <= 2 J rows, by one wave without barriers.  Lane L works on row
+// r = L & 31 and on the columns 2 j + (L >> 5), j < J; lane r < kB holds row r
+// in a on entry.  A row exchange of the reference is an exchange of two `pos`
+// values (a lane's current row index); the right-hand side e_1 is bv.
+//   Pivot: the largest |a(j, k)| over the rows and columns not yet pivoted,
+// first in row-major order of the current indices on ties, as the reference's
+// nested loops pick it.  Each lane takes the maximum of its own columns and
+// the first column that has it; then the high words meet in six 32-bit
+// lane-pair stages, and only where several lanes share the largest high word
+// do the low words and the row-major codes (pos * 32 + column) follow.  A
+// pivoted column holds the in-place inverse, which neither later pivots nor
+// the solution read: it becomes zero, which is never a pivot, and stays zero,
+// the pivot rows' entries being zero there too.
+//   The pivot row reaches the other lanes through LDS (in issue order within
+// the wave, no barrier).  The update a - pc * dum keeps the reference's two
+// roundings: `keep` is 1, and 0 with dum = -1 on the pivot row, whose result
+// is pc itself.
+//   Bound by the issue of one wave, about 250 instructions a step at J = 13.
+// One wave rather than four: with four (four columns to a lane) every step
+// held a workgroup barrier, an exchange of candidates through LDS and two
+// six-stage reductions of 64-bit values.  Average launch of k_diis_small, four
+// waves -> one wave and its loads unchained: 15.5 -> 9.8 us at 60 atoms (up
+// to 22 rows), 20.9 -> 13.7 us at 2000 atoms (up to 25), 19.2 -> 12.6 us on a
+// batch of 64 molecules.
+template <int J>
+__device__ __forceinline__ bool eliminate(const double (&a)[kB], int n1, double *rowbuf,
+                                          double &bv, int &pos) {
+#pragma clang fp contract(off)
+  constexpr int JP = J <= 4 ? 4 : J <= 8 ? 8 : 16;
+  typedef double Row __attribute__((ext_vector_type(JP)));
+  const int lane = lane_id(), r = lane & 31, half = lane >> 5;
+  Row g;
 #pragma unroll
-  for (int j = 0; j < kGJCols; ++j) {
-    constexpr int lo0 = W, hi0 = W + 4;
-    const int lo = lo0 + 8 * j, hi = hi0 + 8 * j;
-    const double vl = (lo < kB) ? a[lo < kB ? lo : 0] : 0.0;
-    const double vh = partner<0>((hi < kB) ? a[hi < kB ? hi : 0] : 0.0);
-    g[j] = (lane_id() < 32) ? vl : vh;
+  for (int j = 0; j < JP; ++j) g[j] = 0.0;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const double lo = a[2 * j];
+    const double hi = partner<0>(2 * j + 1 < kB ? a[2 * j + 1 < kB ? 2 * j + 1 : 0] : 0.0);
+    const double v = half ? hi : lo;
+    g[j] = (r < n1 && 2 * j + half < n1) ? v : 0.0;
   }
+  bv = (r == 0) ? 1.0 : 0.0;
+  pos = r;
+  bool rowlive = r < n1;
+  for (int it = 0; it < n1; ++it) {
+    // the lane's largest value and its first column
+    double m[J];
+#pragma unroll
+    for (int j = 0; j < J; j += 2) m[j] = max_abs(g[j], j + 1 < J ? g[j + 1] : g[j]);
+#pragma unroll
+    for (int w = 2; w < J; w *= 2)
+#pragma unroll
+      for (int j = 0; j + w < J; j += 2 * w) m[j] = max_abs(m[j], m[j + w]);
+    const double big = rowlive ? m[0] : 0.0;
+    int jc = 0;
+#pragma unroll
+    for (int j = J - 1; j >= 0; --j) jc = (fabs(g[j]) == big) ? j : jc;
+    const int code = pos * 32 + 2 * jc + half;
+    // every lane inverts its own candidate while the search goes on
+    const double rec = 1.0 / big;
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(big);
+    const unsigned hi = (unsigned)(bits >> 32), lo = (unsigned)bits;
+    const unsigned mhi = wave_max_u32(hi);
+    unsigned long long cand = __ballot(hi == mhi);
+    if (__popcll(cand) > 1) {
+      const unsigned mlo = wave_max_u32(hi == mhi ? lo : 0u);
+      const bool tie = (hi == mhi) & (lo == mlo);
+      if (mhi == 0u && mlo == 0u) return false;   // nothing left above zero
+      cand = __ballot(tie);
+      if (__popcll(cand) > 1) {
+        const unsigned first = wave_max_u32(tie ? ~(unsigned)code : 0u);
+        cand = __ballot(tie && ~(unsigned)code == first);
+      }
+    }
+    const int src = __builtin_amdgcn_readfirstlane(__ffsll(cand) - 1);
+    const int best = __builtin_amdgcn_readlane(code, src);
+    const int lr = src & 31, hc = src >> 5;
+    const int irow = best >> 5, icol = best & 31, jj = icol >> 1;
+    // the pivot column: the multipliers a(j, icol) of all rows, in both halves
+    const double col = g[jj];
+    const double d = lane_value(col, src);
+    if (d == 0.0) return false;
+    g[jj] = (half == hc) ? 0.0 : col;
+    const bool prow = r == lr;
+    if (prow) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) rowbuf[half * 16 + j] = g[j];
+    }
+    wave_lds_sync();
+    const unsigned long long cb = (unsigned long long)__double_as_longlong(col);
+    const auto sl = __builtin_amdgcn_permlane32_swap((unsigned)cb, (unsigned)cb, false, false);
+    const auto sh = __builtin_amdgcn_permlane32_swap((unsigned)(cb >> 32), (unsigned)(cb >> 32),
+                                                     false, false);
+    // (the swap of a register with itself leaves the lower half's values in
+    // the first result and the upper half's in the second, in all lanes)
+    const unsigned long long db = ((unsigned long long)(hc ? sh[1] : sh[0]) << 32) |
+                                  (hc ? sl[1] : sl[0]);
+    const double dum = prow ? -1.0 : __longlong_as_double((long long)db);
+    const double keep = prow ? 0.0 : 1.0;
+    const double pinv = __builtin_copysign(lane_value(rec, src), d);
+    double pr[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) pr[j] = rowbuf[half * 16 + j];
+    wave_lds_sync();
+    pos = prow ? icol : (pos == icol ? irow : pos);
+    rowlive = rowlive & !prow;
+    const double bp = lane_value(bv, lr) * pinv;
+    bv = __builtin_fma(bv, keep, -(bp * dum));
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const double pc = pr[j] * pinv;
+      g[j] = __builtin_fma(g[j], keep, -(pc * dum));
+    }
+  }
+  return true;
 }
 
 __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
-    int diis_max, int nbj, const int *__restrict__ jboff, const int *__restrict__ eboff,
-    const int *__restrict__ soff, int ninst, int maxit, Systems sys) {
+    int diis_max, int nbj, int nbe, int nsph_all, const int *__restrict__ jboff,
+    const int *__restrict__ eboff, const int *__restrict__ soff, int ninst, int maxit,
+    Systems sys) {
 #pragma clang fp contract(off)
   const SysArgs &q0 = sys.s[blockIdx.y];
   const int inst = blockIdx.x;
   DiisState *__restrict__ st = q0.st + inst;
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
-  // every state word and map entry of the iteration, loaded together
+  // Every state word, the rows of B and the workgroup partials are loaded at
+  // once, none behind a test of another (a launch is a chain of memory round
+  // trips of about 0.7 us each): the block ranges of a single system come
+  // with the launch, and the partials of Gram dots that do not exist yet are
+  // read and not used.
   const int done = st->done;
   const double tol = st->tol;
   int nmat = st->nmat;
   const int it0 = st->it;
   const bool pending = st->pending_norm != 0;
-  const int jb = jboff[inst], eb = eboff[inst];
-  const int nblk = jboff[inst + 1] - jb, nblk_e = eboff[inst + 1] - eb;
-  const int nsph = soff[inst + 1] - soff[inst];
-  if (done) return;
+  int jb = 0, eb = 0, nblk = nbj, nblk_e = nbe, nsph = nsph_all;
+  if (ninst > 1) {
+    jb = jboff[inst];
+    eb = eboff[inst];
+    nblk = jboff[inst + 1] - jb;
+    nblk_e = eboff[inst + 1] - eb;
+    nsph = soff[inst + 1] - soff[inst];
+  }
   DiisState *sum = ninst > 1 ? q0.st + ninst : nullptr;
-  const double *__restrict__ part = q0.part + jb;
-  const double *__restrict__ part_e = q0.part_e + eb;
-  // lane r: row r of B and logical slot r, in flight with the partial sums
+  // lane r: row r of B and logical slot r
   double a[kB];
 #pragma unroll
-  for (int c = 0; c < kB; ++c) a[c] = (lane < kB) ? st->b[lane * kB + c] : 0.0;
-  int myslot = (lane < diis_max) ? st->slot[lane] : 0;
-  const int lastslot = st->slot[nmat - 1];
+  for (int c = 0; c < kB; ++c) a[c] = st->b[min(lane, kB - 1) * kB + c];
+  int myslot = st->slot[min(lane, kDiisMax - 1)];
   __shared__ double red[kPartStride + 1];
-  const int off = (nmat >= diis_max) ? 10 : 0;
-  const int ndot = nmat - off - 1;
   // Gram-row dot products and the increment norm of the previous iteration
   // (value 26): eight consecutive lanes share a value, each sums every eighth
   // workgroup partial, so that all loads are in flight together, and the
   // eight partial sums meet in three lane-pair stages within the group
   {
     const int q = tid / kTPQ, r = tid % kTPQ;
-    double s = 0.0;
-    if (q <= kPartStride) {
-      const bool need = (q < ndot || q == kDiisMax) || (q == kPartStride && pending);
-      if (need) {
-        const double *src = (q == kPartStride) ? part_e : part + (size_t)q * nbj;
-        const int nb = (q == kPartStride) ? nblk_e : nblk;
-        if (max(nblk, nblk_e) <= kTPQ * 8)
-          s = sum_partials<8>(src, nb, r);
-        else
-          s = sum_partials<32>(src, nb, r);
-      }
-    }
+    const bool norm_row = q >= kPartStride;
+    const double *src = norm_row ? q0.part_e + eb : q0.part + jb + (size_t)q * nbj;
+    const int nb = norm_row ? nblk_e : nblk;
+    double s;
+    if (max(nblk, nblk_e) <= kTPQ * 8)
+      s = sum_partials<8>(src, nb, r);
+    else
+      s = sum_partials<32>(src, nb, r);
     s += partner<3>(s);
     s += partner<4>(s);
     s += partner<5>(s);
     if (r == 0 && q <= kPartStride) red[q] = s;
   }
   __syncthreads();
+  if (done) return;
+  const int off = (nmat >= diis_max) ? 10 : 0;
+  const int ndot = nmat - off - 1;
+  const int lastslot = __builtin_amdgcn_readlane(myslot, __builtin_amdgcn_readfirstlane(nmat - 1));
   if (pending) {
     // rms of the per-sphere norms and the convergence test of the previous
     // iteration (rmsvec, jacobi_diis.f90:405-438; jacobi_diis.f90:153-156),
@@ -336,7 +447,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
     }
     if (stop) return;
   }
-  // B update, by every wave alike (wave 0 persists it)
+  // the bordered system is one wave's work from here on
+  if (wave != 0) return;
+  // B update
   {
   // lane i + 1 keeps dot i; every lane keeps the self dot
   const int qi = (lane >= 1 && lane <= kDiisMax) ? lane - 1 : 0;
@@ -385,166 +498,27 @@ __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
     }
   }
   }
-  if (wave == 0) {
-    // persist B and the slot map; k_extrap leaves this iteration's norm
-    if (lane < kB) {
+  // persist B and the slot map; k_extrap leaves this iteration's norm
+  if (lane < kB) {
 #pragma unroll
-      for (int c = 0; c < kB; ++c) st->b[lane * kB + c] = a[c];
-    }
-    if (lane < diis_max) st->slot[lane] = myslot;
-    if (lane == 0) {
-      st->pending_norm = 1;
-      q0.newslot[inst] = lastslot;
-    }
+    for (int c = 0; c < kB; ++c) st->b[lane * kB + c] = a[c];
+  }
+  if (lane < diis_max) st->slot[lane] = myslot;
+  if (lane == 0) {
+    st->pending_norm = 1;
+    q0.newslot[inst] = lastslot;
   }
 
-  // Gauss-Jordan with full pivoting on B, n1 = nmat + 1, by all four waves
-  // and both halves of each: lane L works on row r = L & 31 (its current row
-  // index is `pos`: the reference's row exchange becomes an exchange of two
-  // pos values) and on the columns G, G + 8, G + 16, G + 24 of its group
-  // G = wave + 4 (L >> 5); the right-hand side e_1 travels with wave 0.
-  // Columns already pivoted hold the in-place inverse, which neither the
-  // later pivots nor the solution read, so what they receive does not
-  // matter; the arithmetic on every live element is the reference's.  A
-  // candidate is coded row * 32 + column (n1 <= 25), which orders candidates
-  // row-major as the reference's nested loops do; the pivot is the largest
-  // value (an exact max), then the smallest code among its ties.
-  // Per step and wave: its candidate, the lane holding that row, the signed
-  // pivot value and the whole column it lies in, double-buffered so that
-  // one barrier per step suffices.
-  constexpr int kNW = kSmallThreads / kWave;
-  constexpr int kNone = 0x7fffffff;
-  struct alignas(16) Cand {
-    double v, d;   // |pivot| (-1: none) and the signed pivot
-    int k, l;      // candidate code and the lane holding its row
-  };
-  __shared__ Cand cand[2][kNW];
-  __shared__ double ccol[2][kNW][32];
+  // the register count of a lane follows the system's size
+  __shared__ __align__(16) double rowbuf[32];
   const int n1 = nmat + 1;
-  const int r = lane & 31, half = lane >> 5;
-  double g[kGJCols];
-  switch (__builtin_amdgcn_readfirstlane(wave)) {
-    case 0: group_columns<0>(a, g); break;
-    case 1: group_columns<1>(a, g); break;
-    case 2: group_columns<2>(a, g); break;
-    default: group_columns<3>(a, g); break;
-  }
-  const int grp = wave + 4 * half;
-#pragma unroll
-  for (int j = 0; j < kGJCols; ++j)
-    if (!(r < n1 && grp + 8 * j < n1)) g[j] = 0.0;
-  double bv = (lane == 0) ? 1.0 : 0.0;
-  int pos = r;
-  unsigned int live = (n1 >= 32) ? 0xffffffffu : ((1u << n1) - 1u);   // columns not pivoted
-  bool ok = true;
-  for (int it = 0; it < n1; ++it) {
-    const int buf = it & 1;
-    // pivot: largest |a(j, k)| > 0 over rows and columns not pivoted, first
-    // in row-major order of the current row indices on ties
-    const bool rowlive = r < n1 && ((live >> pos) & 1u);
-    double big = -1.0;
-    int best = kNone;
-#pragma unroll
-    for (int j = 0; j < kGJCols; ++j) {
-      const int c = grp + 8 * j;
-      const double v = (rowlive && c < n1 && ((live >> c) & 1u)) ? fabs(g[j]) : -1.0;
-      const bool t = v > big;   // columns ascend: the first one wins ties
-      big = t ? v : big;
-      best = t ? pos * 32 + c : best;
-    }
-    if (!(big > 0.0)) best = kNone;
-    {
-      double m = big;
-      m = fmax(m, partner<0>(m));
-      m = fmax(m, partner<1>(m));
-      m = fmax(m, partner<2>(m));
-      m = fmax(m, partner<3>(m));
-      m = fmax(m, partner<4>(m));
-      m = fmax(m, partner<5>(m));
-      int key = (big == m) ? best : kNone;
-      key = min(key, partner<0>(key));
-      key = min(key, partner<1>(key));
-      key = min(key, partner<2>(key));
-      key = min(key, partner<3>(key));
-      key = min(key, partner<4>(key));
-      key = min(key, partner<5>(key));
-      big = m;
-      best = __builtin_amdgcn_readfirstlane(key);
-    }
-    {
-      // the column of this wave's candidate (the multipliers a(j, icol) if
-      // it wins), held by the half of its group, and, from the lane holding
-      // its row there, the signed pivot
-      const int cc = best & 31;
-      const int jj = (best == kNone) ? 0 : (cc >> 3);
-      const int hc = (best == kNone) ? 0 : ((cc >> 2) & 1);
-      double v = 0.0;
-#pragma unroll
-      for (int j = 0; j < kGJCols; ++j) v = (j == jj) ? g[j] : v;
-      if (half == hc) ccol[buf][wave][r] = v;
-      int lr = __ffsll((unsigned long long)__ballot(lane < n1 && pos == (best >> 5))) - 1;
-      lr = max(lr, 0);
-      const double dv = lane_value(v, lr + 32 * hc);
-      if (lane == 0) cand[buf][wave] = Cand{big, dv, best, lr};
-    }
-    __syncthreads();
-    Cand cw[kNW];
-#pragma unroll
-    for (int w = 0; w < kNW; ++w) cw[w] = cand[buf][w];
-    double m = cw[0].v;
-#pragma unroll
-    for (int w = 1; w < kNW; ++w) m = fmax(m, cw[w].v);
-    best = kNone;
-    int win = 0;
-#pragma unroll
-    for (int w = 0; w < kNW; ++w) {
-      const bool t = (cw[w].v == m) & (cw[w].k < best);
-      best = t ? cw[w].k : best;
-      win = t ? w : win;
-    }
-    best = __builtin_amdgcn_readfirstlane(best);
-    win = __builtin_amdgcn_readfirstlane(win);
-    if (best == kNone) { ok = false; break; }
-    double d = cw[0].d;
-    int lr = cw[0].l;
-#pragma unroll
-    for (int w = 1; w < kNW; ++w) {
-      d = (win == w) ? cw[w].d : d;
-      lr = (win == w) ? cw[w].l : lr;
-    }
-    lr = __builtin_amdgcn_readfirstlane(lr);
-    const int irow = best >> 5, icol = best & 31;
-    if (!((live >> icol) & 1u) || d == 0.0) { ok = false; break; }
-    // each row's multiplier a(j, icol) and the pivot row's values in this
-    // lane's columns, read before the pivot row is scaled
-    const double dum = ccol[buf][win][r];
-    const int src = lr + 32 * half;
-    double pr[kGJCols];
-#pragma unroll
-    for (int j = 0; j < kGJCols; ++j) pr[j] = __shfl(g[j], src, kWave);
-    const double pinv = 1.0 / d;
-    // the lane holding row irow becomes pivot row icol
-    if (irow != icol) {
-      int np = pos;
-      if (r < n1 && pos == icol) np = irow;
-      if (r == lr) np = icol;
-      pos = np;
-    }
-    live &= ~(1u << icol);
-    // scale the pivot row (a(icol, :) * pivinv) and eliminate column icol
-    // from the other rows, in every column of the lane (no branch)
-#pragma unroll
-    for (int j = 0; j < kGJCols; ++j) {
-      const double pc = pr[j] * pinv;
-      const double el = g[j] - pc * dum;
-      g[j] = (r == lr) ? pc : el;
-    }
-    if (wave == 0) {
-      const double bp = lane_value(bv, lr) * pinv;
-      bv = (r == lr) ? bp : bv - bp * dum;
-    }
-  }
-  if (wave != 0) return;
+  double bv;
+  int pos;
+  bool ok;
+  if (n1 <= 8) ok = eliminate<4>(a, n1, rowbuf, bv, pos);
+  else if (n1 <= 14) ok = eliminate<7>(a, n1, rowbuf, bv, pos);
+  else if (n1 <= 20) ok = eliminate<10>(a, n1, rowbuf, bv, pos);
+  else ok = eliminate<13>(a, n1, rowbuf, bv, pos);
   if (ok) {
     if (lane < n1 && pos >= 1) st->coef[pos - 1] = bv;
   }
@@ -1029,8 +1003,8 @@ int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
     if (diis_max > 0) {
       TimedLaunch tl(h, DDX_K_DIIS, s);
       hipExtLaunchKernelGGL(k_diis_small, dim3(ninst, count), dim3(kSmallThreads), 0, s, tl.b,
-                            tl.e, 0, diis_max, nbj, h->jboff.p, h->eboff.p, h->soff.p, ninst,
-                            l0.max_iter, sys);
+                            tl.e, 0, diis_max, nbj, nbe, h->n, h->jboff.p, h->eboff.p, h->soff.p,
+                            ninst, l0.max_iter, sys);
       DDX_HIP(hipGetLastError());
     }
     {
