@@ -83,6 +83,7 @@ struct DiisState {
   int ok;                   // converged
   int singular;             // DIIS resets from a singular B
   int pending_norm;         // the last k_extrap left increment-norm partials
+  int cur;                  // physical slot of logical index nmat - 1, the next vector's
   int slot[kDiisMax];       // logical history index -> physical slot
   int ncoef;                // coefficients valid in coef[] (0: keep Jacobi step)
   int remaining;            // batch summary only: instances not yet done

@@ -157,6 +157,90 @@ __device__ __forceinline__ int wave_max_int(int v) {
   return v;
 }
 
+// List length per lane after s halvings of n values.
+__host__ __device__ constexpr int reduced_len(int n, int s) {
+  return s == 0 ? n : reduced_len((n + 1) / 2, s - 1);
+}
+
+// 64-bit value of the partner lane of stage S of wave_reduce_split (S >= 2):
+// mirror within 16 lanes, mirror within 8, then quad swaps by 2 and by 1
+template <int S>
+__device__ __forceinline__ double dpp_partner(double v) {
+  constexpr int ctrl = S == 2 ? 0x140 : S == 3 ? 0x141 : S == 4 ? 0x4E : 0xB1;
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), ctrl, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), ctrl, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Stage S of a reduce-scatter across the wave: each lane splits its list of
+// N values into halves x = v[0, H) and y = v[H, N), pairs with a lane that
+// differs in lane bit 5 - S (and holds the same columns), keeps one half
+// (bit clear: x, set: y) and adds the partner's copy of that half.  Stage 0
+// pairs lanes 32 apart and stage 1 lanes 16 apart by the gfx950 row swaps,
+// stages 2..5 use DPP.  After six stages each lane holds the wave sums of
+// columns base .. base + len - 1.
+// FP32 values move as one 32-bit word.
+template <int S>
+__device__ __forceinline__ float dpp_partner(float v) {
+  constexpr int ctrl = S == 2 ? 0x140 : S == 3 ? 0x141 : S == 4 ? 0x4E : 0xB1;
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, false));
+}
+
+template <int S, int N, typename R>
+__device__ __forceinline__ void wave_reduce_split(R *v, int &base, int &len) {
+  constexpr int H = (N + 1) / 2;
+  const bool side = (lane_id() >> (5 - S)) & 1;
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    const R x = v[k];
+    const R y = (k + H < N) ? v[k + H] : R(0);
+    if constexpr (S < 2 && sizeof(R) == 4) {
+      const unsigned xb = __float_as_uint(x), yb = __float_as_uint(y);
+      unsigned nxb, nyb;
+      if constexpr (S == 0) {
+        auto r = __builtin_amdgcn_permlane32_swap(xb, yb, false, false);
+        nxb = r[0]; nyb = r[1];
+      } else {
+        auto r = __builtin_amdgcn_permlane16_swap(xb, yb, false, false);
+        nxb = r[0]; nyb = r[1];
+      }
+      v[k] = __uint_as_float(nxb) + __uint_as_float(nyb);
+    } else if constexpr (S < 2) {
+      const long long bx = __double_as_longlong(x), by = __double_as_longlong(y);
+      const unsigned xl = (unsigned)(bx & 0xffffffffll), xh = (unsigned)(bx >> 32);
+      const unsigned yl = (unsigned)(by & 0xffffffffll), yh = (unsigned)(by >> 32);
+      unsigned nxl, nyl, nxh, nyh;
+      if constexpr (S == 0) {
+        auto rl = __builtin_amdgcn_permlane32_swap(xl, yl, false, false);
+        auto rh = __builtin_amdgcn_permlane32_swap(xh, yh, false, false);
+        nxl = rl[0]; nyl = rl[1]; nxh = rh[0]; nyh = rh[1];
+      } else {
+        auto rl = __builtin_amdgcn_permlane16_swap(xl, yl, false, false);
+        auto rh = __builtin_amdgcn_permlane16_swap(xh, yh, false, false);
+        nxl = rl[0]; nyl = rl[1]; nxh = rh[0]; nyh = rh[1];
+      }
+      // the swap leaves, in every lane, its own half and the partner's copy
+      // of it, one in each register
+      const double nx = __longlong_as_double(((long long)nxh << 32) | nxl);
+      const double ny = __longlong_as_double(((long long)nyh << 32) | nyl);
+      v[k] = nx + ny;
+    } else {
+      const double keep = side ? y : x;
+      const double send = side ? x : y;
+      v[k] = keep + dpp_partner<S>(send);
+    }
+  }
+  if (side) {
+    base += H;
+    len = len > H ? len - H : 0;
+  } else {
+    len = len < H ? len : H;
+  }
+  if constexpr (S < 5) wave_reduce_split<S + 1, H, R>(v, base, len);
+}
+
 // number of set ballot bits below this lane
 __device__ __forceinline__ int ballot_prefix(unsigned long long b) {
   unsigned long long below = (lane_id() == 0) ? 0ull : (~0ull >> (64 - lane_id()));

@@ -74,6 +74,15 @@ __device__ __forceinline__ double widen_late(float v) {
   return (double)v;
 }
 
+// x_new = D^-1 (rhs - y) and the residual x_new - x of that rounded x_new (no
+// fused multiply-subtract: both kernels that call it give the same bits)
+__device__ __forceinline__ void jacobi_step(double facl, double rhs, double y, double x,
+                                            double &xn, double &dx) {
+#pragma clang fp contract(off)
+  xn = facl * (rhs - y);
+  dx = xn - x;
+}
+
 // E is the storage type of the residual history: double, or float in mixed
 // precision, where the history only steers the extrapolation coefficients.
 // Each residual is rounded to E once and that rounded value enters every dot
@@ -148,8 +157,9 @@ __global__ __launch_bounds__(kJThreads) void k_jacobi(size_t nn, int nylm, int d
       if (q0.acc) yk += q0.yacc[k];
       q0.yacc[k] = yk;
     }
-    double xn = facl[lm] * (rhs[k] - yk);
-    const E er = (E)(xn - x[k]);
+    double xn, dx;
+    jacobi_step(facl[lm], rhs[k], yk, x[k], xn, dx);
+    const E er = (E)dx;
     const double e = (double)er;
     xo[k] = xn;
     if (eo) {
@@ -176,6 +186,168 @@ __global__ __launch_bounds__(kJThreads) void k_jacobi(size_t nn, int nylm, int d
   const int q = threadIdx.x;
   if (q < ndot || q == kDiisMax)
     part[(size_t)q * nbj + blockIdx.x] =
+        (wpart[0][q] + wpart[1][q]) + (wpart[2][q] + wpart[3][q]);
+}
+
+// element at a 32-bit byte offset of a wave-uniform base
+template <typename T>
+__device__ __forceinline__ T load_at(const void *base, unsigned bytes) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
+}
+
+// the largest number of Gram dots of an iteration: nmat stays below diis_max
+// or drops by ten
+constexpr int kMaxDots = kDiisMax - 2;
+
+// One thread's two elements of k_jacobi_two: history residuals (H of them,
+// those past ndot re-read slot 0 and meet only unread sums), operator image,
+// Jacobi step, stores, and its shares of the Gram dots, self dot last.
+template <typename E, int H>
+__device__ __forceinline__ void jacobi_two_elements(
+    const SysArgs &a, unsigned nn, unsigned nylm, const unsigned (&k)[2], const bool (&live)[2],
+    const unsigned (&lm)[2], const int (&s0)[2], const int (&s1)[2], const double (&rhs)[2],
+    const double (&x)[2], const double (&f)[2], const unsigned (&slot)[kMaxDots], unsigned cur,
+    bool done, double (&acc)[kMaxDots + 1]) {
+  E ev[2][H];
+#pragma unroll
+  for (int q = 0; q < H; ++q)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      ev[i][q] = load_at<E>(a.ed, (slot[q] * nn + k[i]) * (unsigned)sizeof(E));
+  double y[2] = {0.0, 0.0}, ya[2] = {0.0, 0.0};
+  const bool add = a.yacc && a.acc;
+  if (add) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) ya[i] = a.yacc[k[i]];
+  }
+  if (a.yp) {
+    // sums over the segments in order, the loads of eight segments of both
+    // elements in flight together (past the last one: read again, not added)
+    const int n0 = s1[0] - s0[0], n1 = s1[1] - s0[1];
+    for (int j = 0; j < max(n0, n1); j += 8) {
+      double v[2][8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        v[0][t] = a.yp[(size_t)(s0[0] + max(min(j + t, n0 - 1), 0)) * nylm + lm[0]];
+        v[1][t] = a.yp[(size_t)(s0[1] + max(min(j + t, n1 - 1), 0)) * nylm + lm[1]];
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        if (j + t < n0) y[0] += v[0][t];
+        if (j + t < n1) y[1] += v[1][t];
+      }
+    }
+  } else {
+    double v[2][kProjSplit];
+#pragma unroll
+    for (int j = 0; j < kProjSplit; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) v[i][j] = a.y[(size_t)min(j, a.ny - 1) * nn + k[i]];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      y[i] = v[i][0];
+#pragma unroll
+      for (int j = 1; j < kProjSplit; ++j)
+        if (j < a.ny) y[i] += v[i][j];
+    }
+  }
+  E *__restrict__ eo = reinterpret_cast<E *>(a.ed) + (size_t)cur * nn;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if (!live[i]) continue;
+    if (add) y[i] += ya[i];
+    double xn, dx;
+    jacobi_step(f[i], rhs[i], y[i], x[i], xn, dx);
+    const E er = (E)dx;
+    const double e = (double)er;
+    if (!done) {
+      if (a.yacc) a.yacc[k[i]] = y[i];
+      a.xd[(size_t)cur * nn + k[i]] = xn;
+      eo[k[i]] = er;
+    }
+#pragma unroll
+    for (int q = 0; q < H; ++q) acc[q] += (double)ev[i][q] * e;
+    acc[kMaxDots] += e * e;
+  }
+}
+
+// k_jacobi for one system of at most 512 elements per workgroup, two per
+// thread: the same sums, arranged for latency.  Such a launch (under 700
+// workgroups at 2000 atoms) is a chain of memory round trips of 0.7 us and
+// more, not of bytes:
+//  * the workgroup's range comes from its index (the block map's formula) and
+//    the next vector's slot from the state, instead of a map's load each;
+//  * all pointers are read from the argument block at once;
+//  * what does not depend on the DIIS state (segment ranges, right-hand side,
+//    iterate) loads while the state does, then both elements' history and
+//    segment shares together, without a branch between their loads;
+//  * the 24 wave sums meet in one reduce-scatter (the lane pairs of wave_sum,
+//    the same bits) instead of one six-stage sum each.
+// Average launch of k_jacobi -> this kernel: 12.5 -> 5.8 us at 60 atoms, 18.9 ->
+// 7.7 us at 200 atoms and lmax 10, 12.1 -> 7.7 us at 1000, 14.8 -> 12.5 us at
+// 2000 atoms (lmax 8).
+template <typename E>
+__global__ __launch_bounds__(kJThreads) void k_jacobi_two(unsigned nn, unsigned nylm,
+                                                          int diis_max, unsigned nbj,
+                                                          const double *__restrict__ facl,
+                                                          Systems sys) {
+  const SysArgs a = sys.s[blockIdx.y];
+  asm volatile("" ::"s"(a.rhs), "s"(a.y), "s"(a.yp), "s"(a.segoff), "s"(a.x), "s"(a.ed),
+               "s"(a.st), "s"(a.yacc), "s"(a.part), "s"(facl));
+  const DiisState *__restrict__ st = a.st;
+  __shared__ double wpart[kJThreads / kWave][kMaxDots + 1];
+  const bool done = st->done != 0;
+  const int nmat = st->nmat;
+  const unsigned cur = (unsigned)st->cur;
+  int all[kDiisMax];
+#pragma unroll
+  for (int q = 0; q < kDiisMax; ++q) all[q] = st->slot[q];
+  const unsigned end = nn * (blockIdx.x + 1) / nbj;
+  unsigned k[2], lm[2];
+  bool live[2];
+  double rhs[2], x[2], f[2];
+  int s0[2], s1[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    k[i] = nn * blockIdx.x / nbj + threadIdx.x + i * kJThreads;
+    live[i] = k[i] < end;
+    if (!live[i]) k[i] = end - 1;   // a duplicate whose results are dropped
+    const unsigned c = k[i] / nylm;
+    lm[i] = k[i] - c * nylm;
+    rhs[i] = a.rhs[k[i]];
+    x[i] = a.x[k[i]];
+    f[i] = facl[lm[i]];
+    s0[i] = a.segoff[c];
+    s1[i] = a.segoff[c + 1];
+  }
+  const int off = nmat >= diis_max ? 10 : 0, ndot = nmat - off - 1;
+  unsigned slot[kMaxDots];
+#pragma unroll
+  for (int q = 0; q < kMaxDots; ++q) {
+    const int s = off ? all[q + 10 < kDiisMax ? q + 10 : 0] : all[q];
+    slot[q] = (unsigned)(q < ndot ? s : all[0]);
+  }
+  double acc[kMaxDots + 1];
+#pragma unroll
+  for (int q = 0; q <= kMaxDots; ++q) acc[q] = 0.0;
+  // the loads of a thread follow the history's depth
+  if (ndot <= 8)
+    jacobi_two_elements<E, 8>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, done, acc);
+  else if (ndot <= 16)
+    jacobi_two_elements<E, 16>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, done, acc);
+  else
+    jacobi_two_elements<E, kMaxDots>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, done,
+                                     acc);
+  const int wave = threadIdx.x / kWave;
+  int base = 0, len = kMaxDots + 1;
+  wave_reduce_split<0, kMaxDots + 1, double>(acc, base, len);
+  static_assert(reduced_len(kMaxDots + 1, 6) == 1, "one value per lane");
+  if (len > 0) wpart[wave][base] = acc[0];
+  __syncthreads();
+  if (done) return;
+  const int q = threadIdx.x;
+  if (q < ndot || q == kMaxDots)
+    a.part[(size_t)(q == kMaxDots ? kDiisMax : q) * nbj + blockIdx.x] =
         (wpart[0][q] + wpart[1][q]) + (wpart[2][q] + wpart[3][q]);
 }
 
@@ -522,7 +694,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
   if (ok) {
     if (lane < n1 && pos >= 1) st->coef[pos - 1] = bv;
   }
+  const int cur = __builtin_amdgcn_readlane(myslot, ok ? __builtin_amdgcn_readfirstlane(nmat) : 0);
   if (lane == 0) {
+    st->cur = cur;
     if (!ok) {
       st->nmat = 1;
       st->ncoef = 0;
@@ -668,6 +842,7 @@ __global__ void k_diis_init(int ninst, double tol, DiisState *__restrict__ st) {
   if (t < kDiisMax) d->slot[t] = t;
   if (t == 0) {
     d->nmat = 1;
+    d->cur = 0;
     d->it = 0;
     d->done = 0;
     d->ok = q < ninst ? 0 : 1;
@@ -953,6 +1128,16 @@ int solve_begin(ddx_handle *h, Lane &ln, int star, int diis_max, double tol, con
 }
 
 namespace {
+// Whether k_jacobi_two takes a system: one instance, DIIS on, block ranges of
+// at most 512 elements whose bounds and history offsets fit 32 bits (up to
+// 524 288 elements: 6400 atoms at lmax 8).  Past that a workgroup's threads
+// take more than two elements and the launch is bound by its bytes; a batch's
+// blocks need their map.
+bool jacobi_two_fits(const ddx_handle *h, size_t nn, int diis_max) {
+  return h->ninst == 1 && diis_max > 0 && nn <= 2 * (size_t)kJThreads * h->nbj &&
+         nn * (h->nbj + 1) < (1ull << 32) && nn * kDiisMax * sizeof(double) < (1ull << 32);
+}
+
 // `nr` rounds of one solve, or of a direct and an adjoint solve in lockstep
 int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
   Lane &l0 = *lanes[0];
@@ -992,12 +1177,17 @@ int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
     {
       TimedLaunch tl(h, DDX_K_JACOBI, s);
       // mixed precision keeps the residual history in FP32
-      if (l0.incr)
-        hipExtLaunchKernelGGL(k_jacobi<float>, dim3(nbj, count), dim3(kJThreads), 0, s, tl.b, tl.e,
-                              0, nn, h->nylm, diis_max, h->jblk.p, nbj, h->facl.p, sys);
-      else
-        hipExtLaunchKernelGGL(k_jacobi<double>, dim3(nbj, count), dim3(kJThreads), 0, s, tl.b,
-                              tl.e, 0, nn, h->nylm, diis_max, h->jblk.p, nbj, h->facl.p, sys);
+      const auto launch = [&](auto two, auto one) {
+        if (jacobi_two_fits(h, nn, diis_max))
+          hipExtLaunchKernelGGL(two, dim3(nbj, count), dim3(kJThreads), 0, s, tl.b, tl.e, 0,
+                                (unsigned)nn, (unsigned)h->nylm, diis_max, (unsigned)nbj,
+                                h->facl.p, sys);
+        else
+          hipExtLaunchKernelGGL(one, dim3(nbj, count), dim3(kJThreads), 0, s, tl.b, tl.e, 0, nn,
+                                h->nylm, diis_max, h->jblk.p, nbj, h->facl.p, sys);
+      };
+      if (l0.incr) launch(k_jacobi_two<float>, k_jacobi<float>);
+      else launch(k_jacobi_two<double>, k_jacobi<double>);
     }
     DDX_HIP(hipGetLastError());
     if (diis_max > 0) {

@@ -9,6 +9,11 @@
   size.  Tolerance: one unit of the last printed digit, or 5% below 1e-6 (the
   Gram dots are summed in another order, and the late increments carry that
   rounding).
+* test_single_system_equals_batch_of_two: a single system's latency-ordered
+  solver kernels against the general kernels, which a batch takes: both
+  solutions bit for bit, at one and several workgroups, with a workgroup's
+  second element per thread absent, partial and full.  (At these sizes every
+  sweep worker has one unit, so the operators' sums are split alike.)
 """
 import numpy as np
 import pytest
@@ -30,3 +35,25 @@ def test_increment_norms_of_every_iteration(name):
     unit = 10.0 ** (np.floor(np.log10(ref)) - 3)
     tol = np.where(ref >= 1e-6, unit, np.maximum(unit, 5e-2 * ref))
     assert np.all(np.abs(got - ref) <= 1.01 * tol), (got, ref)
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+@pytest.mark.parametrize("n,lmax,ngrid", [(1, 6, 110), (2, 0, 26), (4, 6, 110), (10, 6, 110),
+                                          (11, 6, 110), (21, 6, 110), (40, 10, 302),
+                                          (3, 16, 302), (150, 8, 194)])
+def test_single_system_equals_batch_of_two(n, lmax, ngrid, mixed):
+    from ddpcm_amd.ddx import DDCosmo, DDCosmoBatch
+    from ddpcm_amd.inputs import synthetic_input
+    d = synthetic_input(n, 77 + n, lmax, ngrid)
+    x, y, z, r = d.bohr()
+    q = d.charge if n > 1 else np.array([1.0])
+    h = DDCosmo(x, y, z, r, lmax, ngrid)
+    b = DDCosmoBatch([x, x], [y, y], [z, z], [r, r], lmax, ngrid)
+    for v in (h, b):
+        v.set_precision(mixed)
+    e, f = h.energy_forces(q)
+    eb, fb = b.energy_forces([q, q])
+    for name in ("sigma", "s"):
+        one, two = h.get(name), b.get(name)
+        assert np.array_equal(one, two[:n]) and np.array_equal(one, two[n:]), name
+    assert e == eb[0] == eb[1]
