@@ -207,7 +207,7 @@ __device__ __forceinline__ void jacobi_two_elements(
     const SysArgs &a, unsigned nn, unsigned nylm, const unsigned (&k)[2], const bool (&live)[2],
     const unsigned (&lm)[2], const int (&s0)[2], const int (&s1)[2], const double (&rhs)[2],
     const double (&x)[2], const double (&f)[2], const unsigned (&slot)[kMaxDots], unsigned cur,
-    bool done, double (&acc)[kMaxDots + 1]) {
+    double (&acc)[kMaxDots + 1]) {
   E ev[2][H];
 #pragma unroll
   for (int q = 0; q < H; ++q)
@@ -260,11 +260,9 @@ __device__ __forceinline__ void jacobi_two_elements(
     jacobi_step(f[i], rhs[i], y[i], x[i], xn, dx);
     const E er = (E)dx;
     const double e = (double)er;
-    if (!done) {
-      if (a.yacc) a.yacc[k[i]] = y[i];
-      a.xd[(size_t)cur * nn + k[i]] = xn;
-      eo[k[i]] = er;
-    }
+    if (a.yacc) a.yacc[k[i]] = y[i];
+    a.xd[(size_t)cur * nn + k[i]] = xn;
+    eo[k[i]] = er;
 #pragma unroll
     for (int q = 0; q < H; ++q) acc[q] += (double)ev[i][q] * e;
     acc[kMaxDots] += e * e;
@@ -327,24 +325,26 @@ __global__ __launch_bounds__(kJThreads) void k_jacobi_two(unsigned nn, unsigned 
     const int s = off ? all[q + 10 < kDiisMax ? q + 10 : 0] : all[q];
     slot[q] = (unsigned)(q < ndot ? s : all[0]);
   }
+  // (keeps the loads above ahead of the test)
+  asm volatile("" ::"v"(rhs[0]), "v"(rhs[1]), "v"(x[0]), "v"(x[1]), "v"(f[0]), "v"(f[1]),
+               "v"(s0[0]), "v"(s0[1]), "v"(s1[0]), "v"(s1[1]));
+  if (done) return;
   double acc[kMaxDots + 1];
 #pragma unroll
   for (int q = 0; q <= kMaxDots; ++q) acc[q] = 0.0;
   // the loads of a thread follow the history's depth
   if (ndot <= 8)
-    jacobi_two_elements<E, 8>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, done, acc);
+    jacobi_two_elements<E, 8>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, acc);
   else if (ndot <= 16)
-    jacobi_two_elements<E, 16>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, done, acc);
+    jacobi_two_elements<E, 16>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, acc);
   else
-    jacobi_two_elements<E, kMaxDots>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, done,
-                                     acc);
+    jacobi_two_elements<E, kMaxDots>(a, nn, nylm, k, live, lm, s0, s1, rhs, x, f, slot, cur, acc);
   const int wave = threadIdx.x / kWave;
   int base = 0, len = kMaxDots + 1;
   wave_reduce_split<0, kMaxDots + 1, double>(acc, base, len);
   static_assert(reduced_len(kMaxDots + 1, 6) == 1, "one value per lane");
   if (len > 0) wpart[wave][base] = acc[0];
   __syncthreads();
-  if (done) return;
   const int q = threadIdx.x;
   if (q < ndot || q == kMaxDots)
     a.part[(size_t)(q == kMaxDots ? kDiisMax : q) * nbj + blockIdx.x] =
@@ -808,6 +808,106 @@ __global__ __launch_bounds__(kJThreads) void k_extrap(int nylm, size_t nn, int d
   if (threadIdx.x == 0) part[blockIdx.x] = tot;
 }
 
+// x_new = sum_i c_i x_i of one element: the history values of the C >= ncoef
+// newest slots are loaded together (those past ncoef re-read slot 0 and are
+// not added).
+template <int C>
+__device__ __forceinline__ double extrapolate(const double *__restrict__ xd, unsigned nn,
+                                              unsigned k, const unsigned (&slot)[kDiisMax],
+                                              const double (&coef)[kDiisMax], int ncoef) {
+  double v[C];
+#pragma unroll
+  for (int q = 0; q < C; ++q)
+    v[q] = load_at<double>(xd, (slot[q] * nn + k) * (unsigned)sizeof(double));
+  double xn = 0.0;
+#pragma unroll
+  for (int q = 0; q < C; ++q)
+    if (q < ncoef) xn = xn + coef[q] * v[q];
+  return xn;
+}
+
+// k_extrap for one system whose workgroups stage all their spheres at once
+// (at most kExtrapTerms elements, 64 spheres), one element per thread of 512:
+// the same sums, arranged for latency as k_jacobi_two is.  The workgroup's
+// spheres come from its index, the slots and coefficients load with the state
+// and beside the iterate, the history without a branch between its loads, and
+// the serial sum of a sphere's norm terms reads LDS eight terms ahead of its
+// additions.  512 threads for the usual 200..480 elements: two elements to
+// each of 256 threads took 198 registers and two rounds of workgroups at 2000
+// atoms.  Average launch of k_extrap -> this kernel: 9.2 -> 4.6 us at 60 atoms,
+// 12.1 -> 6.9 us at 200 atoms and lmax 10, 13.2 -> 9.0 us at 1000, 15.7 -> 14.2
+// us at 2000 atoms (lmax 8; near its bytes there).
+constexpr int kExtrapThreads = 512;
+
+__global__ __launch_bounds__(kExtrapThreads) void k_extrap_one(
+    unsigned n, unsigned nylm, unsigned nn, unsigned nbe, const double *__restrict__ invl1,
+    const double *__restrict__ cf, Systems sys) {
+  const SysArgs a = sys.s[blockIdx.y];
+  asm volatile("" ::"s"(a.x), "s"(a.xs), "s"(a.xd), "s"(a.st), "s"(a.inc), "s"(a.newslot),
+               "s"(a.part_e), "s"(invl1), "s"(cf));
+  const DiisState *__restrict__ st = a.st;
+  __shared__ double terms[kExtrapTerms];
+  const bool done = st->done != 0;
+  const int ncoef = st->ncoef;
+  const unsigned newest = (unsigned)*a.newslot;
+  unsigned slot[kDiisMax];
+  double coef[kDiisMax];
+#pragma unroll
+  for (int q = 0; q < kDiisMax; ++q) {
+    slot[q] = (unsigned)st->slot[q];
+    coef[q] = st->coef[q];
+  }
+#pragma unroll
+  for (int q = 0; q < kDiisMax; ++q) slot[q] = __builtin_amdgcn_readfirstlane((int)slot[q]);
+  if (done) return;
+  const unsigned c0 = n * blockIdx.x / nbe, c1 = n * (blockIdx.x + 1) / nbe;
+  const unsigned ne = (c1 - c0) * nylm, e0 = c0 * nylm;
+  const bool xs_inc = a.xs_inc != 0;
+  for (unsigned j = threadIdx.x; j < ne; j += kExtrapThreads) {
+    const unsigned k = e0 + j, lm = k % nylm;
+    const double x = a.x[k], il = invl1[lm], cl = cf[lm];
+    double xn;
+    if (ncoef == 0)   // the plain Jacobi step
+      xn = a.xd[(size_t)newest * nn + k];
+    else if (ncoef <= 8)
+      xn = extrapolate<8>(a.xd, nn, k, slot, coef, ncoef);
+    else if (ncoef <= 16)
+      xn = extrapolate<16>(a.xd, nn, k, slot, coef, ncoef);
+    else
+      xn = extrapolate<kDiisMax - 1>(a.xd, nn, k, slot, coef, ncoef);
+    const double inc = xn - x;
+    a.x[k] = xn;
+    if (a.xs) a.xs[k] = cl * (xs_inc ? inc : xn);
+    if (a.inc) a.inc[k] = inc;
+    terms[j] = il * inc * inc;
+  }
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  double usq = 0.0;
+  if (threadIdx.x < c1 - c0) {
+    const double *t = terms + threadIdx.x * nylm;
+    const int last = (int)nylm - 1;
+    double sq = 0.0, ahead[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ahead[i] = t[min(i, last)];
+    for (int l = 0; l <= last; l += 8) {
+      double v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i] = ahead[i];
+        ahead[i] = t[min(l + 8 + i, last)];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (l + i <= last) sq += v[i];
+    }
+    const double u = sqrt(sq);
+    usq += u * u;
+  }
+  usq = wave_sum(usq);
+  if (threadIdx.x == 0) a.part_e[blockIdx.x] = usq;
+}
+
 // rms of the per-sphere norms and the convergence test (rmsvec,
 // jacobi_diis.f90:405-438; jacobi_diis.f90:153-156)
 __global__ __launch_bounds__(kWave) void k_norm(const int *__restrict__ eboff,
@@ -1138,6 +1238,13 @@ bool jacobi_two_fits(const ddx_handle *h, size_t nn, int diis_max) {
          nn * (h->nbj + 1) < (1ull << 32) && nn * kDiisMax * sizeof(double) < (1ull << 32);
 }
 
+// Whether k_extrap_one takes a system: as k_jacobi_two, with every workgroup's
+// spheres staged at once.
+bool extrap_one_fits(const ddx_handle *h, size_t nn, int diis_max) {
+  const int most = (h->n + h->nbe - 1) / h->nbe;   // spheres of a workgroup
+  return jacobi_two_fits(h, nn, diis_max) && most <= kWave && most * h->nylm <= kExtrapTerms;
+}
+
 // `nr` rounds of one solve, or of a direct and an adjoint solve in lockstep
 int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
   Lane &l0 = *lanes[0];
@@ -1199,8 +1306,13 @@ int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
     }
     {
       TimedLaunch tl(h, DDX_K_EXTRAP, s);
-      hipExtLaunchKernelGGL(k_extrap, dim3(nbe, count), dim3(kJThreads), 0, s, tl.b, tl.e, 0,
-                            h->nylm, nn, diis_max, h->eblk.p, invl1, h->cf.p, sys);
+      if (extrap_one_fits(h, nn, diis_max))
+        hipExtLaunchKernelGGL(k_extrap_one, dim3(nbe, count), dim3(kExtrapThreads), 0, s, tl.b, tl.e, 0,
+                              (unsigned)h->n, (unsigned)h->nylm, (unsigned)nn, (unsigned)nbe,
+                              invl1, h->cf.p, sys);
+      else
+        hipExtLaunchKernelGGL(k_extrap, dim3(nbe, count), dim3(kJThreads), 0, s, tl.b, tl.e, 0,
+                              h->nylm, nn, diis_max, h->eblk.p, invl1, h->cf.p, sys);
     }
     DDX_HIP(hipGetLastError());
     if (diis_max == 0) {
