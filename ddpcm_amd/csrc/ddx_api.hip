@@ -344,7 +344,7 @@ int create(ddx_handle **out, int n, int count, const int *nsph, const double *x,
   for (Lane &ln : h->lane)
     if (hipHostMalloc((void **)&ln.h_diis, sizeof(DiisState), hipHostMallocDefault) !=
             hipSuccess ||
-        hipHostMalloc((void **)&ln.h_head, 8 * sizeof(int), hipHostMallocDefault) != hipSuccess) {
+        hipHostGetDevicePointer((void **)&ln.d_rec, ln.h_diis, 0) != hipSuccess) {
       set_error("hipHostMalloc failed");
       return fail(DDX_ERR_ALLOC);
     }
@@ -439,10 +439,8 @@ int ddx_batch_init(ddx_handle **out, int count, const int *nsph, const double *x
 int ddx_free(ddx_handle *h) {
   if (!h) return DDX_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  for (Lane &ln : h->lane) {
+  for (Lane &ln : h->lane)
     if (ln.h_diis) (void)hipHostFree(ln.h_diis);
-    if (ln.h_head) (void)hipHostFree(ln.h_head);
-  }
   for (auto &e : h->gev)
     if (e) (void)hipEventDestroy(e);
   drop_round_graphs(h);

@@ -162,8 +162,10 @@ struct Lane {
   DevArray<int> misc;             // per instance: slot of the newest vector
   DevArray<int> res;              // per instance: iterations, ok (after the solve)
   std::vector<int> h_res;         // host copy of res (batches)
-  DiisState *h_diis = nullptr;  // pinned host mirror of diis
-  int *h_head = nullptr;        // pinned: two copies of (nmat, it, done, ok), one per group
+  // pinned host record of the solve: the kernel that ends a single system's
+  // solve writes it, ok and hist there and then done; of a batch only done
+  // (the summary state is copied afterwards).  d_rec: its device address.
+  DiisState *h_diis = nullptr, *d_rec = nullptr;
   // the solve in flight (solve_begin .. solve_end)
   int serial = -1, star = 0, diis_max = 0, max_iter = 0, rounds = 0, enqueued = 0, group = 3;
   double tol = 0.0;

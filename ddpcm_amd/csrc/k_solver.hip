@@ -59,6 +59,7 @@ struct SysArgs {
   double *inc;               // the last increment x_new - x (null: not kept)
   int xs_inc;                // xs = cf inc instead of cf x (the next round applies
                              //   the FP32 operator to the increment)
+  DiisState *rec;            // the host's record of the solve (pinned host memory)
 };
 struct Systems {
   SysArgs s[2];
@@ -377,13 +378,37 @@ __device__ __forceinline__ double lane_value(double v, int src) {
 
 constexpr int kSmallThreads = 256;       // 4 workgroup partials per thread
 
-// an instance of a batch has ended: fold it into the summary, which is done
-// when the last instance is
-__device__ __forceinline__ void instance_done(DiisState *sum, int it, int ok) {
-  if (!sum) return;
-  atomicMax(&sum->it, it);
-  atomicAnd(&sum->ok, ok);
-  if (atomicSub(&sum->remaining, 1) == 1) sum->done = 1;
+// Tells the host, which polls the record, that the solve has ended.  Once per
+// solve: a copy of the state's header after every second round cost two
+// copy kernels (2.3 us each at 60 atoms, 4 us at 2000) in the round's chain.
+__device__ __forceinline__ void post_done(DiisState *rec) {
+  __threadfence_system();
+  __hip_atomic_store(&rec->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// An instance has ended with iteration it0, by one whole wave.  A batch's is
+// folded into the summary, which is done when the last instance is; a single
+// system's results go to the host's record.
+__device__ __forceinline__ void instance_done(DiisState *sum, const DiisState *st, DiisState *rec,
+                                              int it0, double norm, int ok) {
+  if (sum) {
+    if (lane_id() != 0) return;
+    atomicMax(&sum->it, it0 + 1);
+    atomicAnd(&sum->ok, ok);
+    if (atomicSub(&sum->remaining, 1) == 1) {
+      sum->done = 1;
+      post_done(rec);
+    }
+    return;
+  }
+  for (int q = lane_id(); q <= min(it0, kMaxIter); q += kWave)
+    rec->hist[q] = q == it0 ? norm : st->hist[q];
+  if (lane_id() == 0) {
+    rec->it = it0 + 1;
+    rec->ok = ok;
+  }
+  __threadfence_system();   // the whole wave's stores before lane 0's flag
+  if (lane_id() == 0) post_done(rec);
 }
 
 // lanes per summed value in the Gram-row reduction of k_diis_small
@@ -612,11 +637,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
       st->norm = norm;
       st->ok = norm < tol;
       st->pending_norm = 0;
-      if (stop) {
-        st->done = 1;
-        instance_done(sum, it0 + 1, norm < tol);
-      }
+      if (stop) st->done = 1;
     }
+    if (stop && wave == 0) instance_done(sum, st, q0.rec, it0, norm, norm < tol);
     if (stop) return;
   }
   // the bordered system is one wave's work from here on
@@ -921,17 +944,19 @@ __global__ __launch_bounds__(kWave) void k_norm(const int *__restrict__ eboff,
   double s = 0.0;
   for (int b = eboff[inst] + threadIdx.x; b < eboff[inst + 1]; b += kWave) s += part[b];
   s = wave_sum(s);
+  const double norm = sqrt(s / (double)(soff[inst + 1] - soff[inst]));
+  const int it = st->it;
+  const bool stop = norm < tol || it + 1 >= maxit;
   if (threadIdx.x == 0) {
-    double norm = sqrt(s / (double)(soff[inst + 1] - soff[inst]));
-    int it = st->it;
     if (it <= kMaxIter) st->hist[it] = norm;
     st->it = it + 1;
     st->norm = norm;
     st->ok = norm < tol;
-    st->done = (norm < tol) || (it + 1 >= maxit);
-    if (st->done) instance_done(ninst > 1 ? sys.s[blockIdx.y].st + ninst : nullptr, it + 1,
-                                norm < tol);
+    st->done = stop;
   }
+  if (stop)
+    instance_done(ninst > 1 ? sys.s[blockIdx.y].st + ninst : nullptr, st, sys.s[blockIdx.y].rec,
+                  it, norm, norm < tol);
 }
 
 // fresh states for the ninst instances and the summary of a batch
@@ -1160,6 +1185,7 @@ SysArgs sys_args(const ddx_handle *h, Lane &ln) {
   // an increment round reads xs = cf inc, which k_extrap writes as well
   a.inc = (ln.incr && ln.star) ? ln.inc.p : nullptr;
   a.xs_inc = 0;
+  a.rec = ln.d_rec;
   return a;
 }
 
@@ -1217,6 +1243,7 @@ int solve_begin(ddx_handle *h, Lane &ln, int star, int diis_max, double tol, con
   ln.enqueued = 0;
   ln.group = 3;
   ln.active = true;
+  ln.h_diis->done = 0;   // (no kernel of an earlier solve writes it any more)
 
   const int nst = h->ninst > 1 ? h->ninst + 1 : 1;
   hipLaunchKernelGGL(k_diis_init, dim3(nst), dim3(kWave), 0, ln.stream, h->ninst, tol,
@@ -1392,10 +1419,9 @@ void drop_round_graphs(ddx_handle *h) {
   h->round_graphs.clear();
 }
 
-// Enqueues the next group of rounds and the copy of each lane's state header
-// (nmat, it, done, ok) into slot `slot` of its pinned h_head, marked by
-// h->gev[slot].  The first group of a solve (3 rounds) runs eagerly and
-// makes every buffer the rounds use; eager groups after it have 2 rounds.
+// Enqueues the next group of rounds, its end marked by h->gev[slot].  The
+// first group of a solve (3 rounds) runs eagerly and makes every buffer the
+// rounds use; eager groups after it are single rounds.
 // With graphs on (and no kernel timer) each later group is one launch of a
 // captured graph of kGraphRounds rounds, which covers the rest of a typical
 // solve; the rounds after convergence return at once.
@@ -1417,10 +1443,7 @@ int solve_enqueue(ddx_handle *h, Lane *const *lanes, int count, int slot) {
     DDX_TRY(enqueue_rounds(h, lanes, count, nr));
   h->tag_solve = -1;
   h->tag_round = 0;
-  l0.group = 2;
-  for (int k = 0; k < count; ++k)
-    DDX_HIP(hipMemcpyAsync(lanes[k]->h_head + 4 * slot, solve_gate(h, *lanes[k]), 4 * sizeof(int),
-                           hipMemcpyDeviceToHost, s));
+  l0.group = 1;
   DDX_HIP(hipEventRecord(h->gev[slot], s));
   return DDX_OK;
 }
@@ -1438,50 +1461,73 @@ int solve_end(ddx_handle *h, Lane &ln, int *n_iter, int *ok, std::vector<double>
   return DDX_OK;
 }
 
+namespace {
+bool lanes_done(Lane *const *lanes, int count) {
+  for (int k = 0; k < count; ++k)
+    if (!*(volatile int *)&lanes[k]->h_diis->done) return false;
+  return true;
+}
+
+// Enqueues groups of rounds until the lanes' records say done or all rounds
+// have run.  Two groups are in flight: while one runs, the next is already
+// queued behind it, so the device does not wait for the host, and the host
+// sees the end of a solve within the group that brought it (the one queued
+// after it returns at once).  Of the graph groups only the first runs ahead
+// (behind the eager first group): a later one would mostly repeat finished
+// rounds.
+int run_groups(ddx_handle *h, Lane *const *lanes, int count) {
+  int head = 0, queued = 0, groups = 0;
+  while (!lanes_done(lanes, count)) {
+    const bool more = lanes[0]->enqueued < lanes[0]->rounds;
+    if (more && (queued == 0 || (queued == 1 && (!h->use_graphs || groups == 1)))) {
+      DDX_TRY(solve_enqueue(h, lanes, count, (head + queued) & 1));
+      ++queued;
+      ++groups;
+      continue;
+    }
+    if (queued == 0) break;
+    // poll the record beside the group's event for about a millisecond,
+    // then sleep on the event
+    hipError_t e = hipErrorNotReady;
+    for (int spin = 0; spin < 1000 && e == hipErrorNotReady; ++spin) {
+      if (lanes_done(lanes, count)) return DDX_OK;
+      e = hipEventQuery(h->gev[head]);
+    }
+    if (e == hipErrorNotReady) e = hipEventSynchronize(h->gev[head]);
+    DDX_HIP(e);
+    head ^= 1;
+    --queued;
+  }
+  return DDX_OK;
+}
+}  // namespace
+
 int solve_run(ddx_handle *h, Lane *const *lanes, int count) {
   const int serial = h->solve_serial++;
   for (int k = 0; k < count; ++k) lanes[k]->serial = serial;
-  // one eager group always runs ahead: while the host waits for the state
-  // of group k, group k + 1 is already queued behind it, so the device does
-  // not wait for the host between groups (a group queued after convergence
-  // returns at once).  Of the graph groups only the first runs ahead (behind
-  // the eager first group): a later one would mostly repeat finished rounds.
-  int cur = 0, queued = 1, groups = 1;
-  DDX_TRY(solve_enqueue(h, lanes, count, cur));
-  while (true) {
-    if (lanes[0]->enqueued < lanes[0]->rounds && queued == 1 &&
-        (!h->use_graphs || groups == 1)) {
-      DDX_TRY(solve_enqueue(h, lanes, count, cur ^ 1));
-      ++queued;
-      ++groups;
-    }
-    DDX_HIP(hipEventSynchronize(h->gev[cur]));
-    --queued;
-    bool all = true;
-    for (int k = 0; k < count; ++k) all = all && lanes[k]->h_head[4 * cur + 2] != 0;
-    if (all) break;
-    if (queued == 0) {
-      if (lanes[0]->enqueued >= lanes[0]->rounds) break;
-      DDX_TRY(solve_enqueue(h, lanes, count, cur ^ 1));
-      ++queued;
-      ++groups;
-    }
-    cur ^= 1;
+  const int rc = run_groups(h, lanes, count);
+  if (rc != DDX_OK) {
+    // no kernel of this solve may write its record once another one starts
+    (void)hipStreamSynchronize(lanes[0]->stream);
+    return rc;
   }
-  for (int k = 0; k < count; ++k) {
-    Lane &ln = *lanes[k];
-    DDX_HIP(hipMemcpyAsync(ln.h_diis, solve_gate(h, ln), sizeof(DiisState),
-                           hipMemcpyDeviceToHost, ln.stream));
-    if (h->ninst > 1) {
-      hipLaunchKernelGGL(k_diis_results, dim3((h->ninst + 255) / 256), dim3(256), 0, ln.stream,
-                         h->ninst, ln.max_iter, ln.diis.p, ln.res.p);
-      DDX_HIP(hipGetLastError());
-      ln.h_res.resize(2 * (size_t)h->ninst);
-      DDX_HIP(hipMemcpyAsync(ln.h_res.data(), ln.res.p, 2 * sizeof(int) * h->ninst,
+  // a single system's record is complete; a batch's states are copied
+  if (h->ninst > 1 || !lanes_done(lanes, count)) {
+    for (int k = 0; k < count; ++k) {
+      Lane &ln = *lanes[k];
+      DDX_HIP(hipMemcpyAsync(ln.h_diis, solve_gate(h, ln), sizeof(DiisState),
                              hipMemcpyDeviceToHost, ln.stream));
+      if (h->ninst > 1) {
+        hipLaunchKernelGGL(k_diis_results, dim3((h->ninst + 255) / 256), dim3(256), 0, ln.stream,
+                           h->ninst, ln.max_iter, ln.diis.p, ln.res.p);
+        DDX_HIP(hipGetLastError());
+        ln.h_res.resize(2 * (size_t)h->ninst);
+        DDX_HIP(hipMemcpyAsync(ln.h_res.data(), ln.res.p, 2 * sizeof(int) * h->ninst,
+                               hipMemcpyDeviceToHost, ln.stream));
+      }
     }
+    DDX_HIP(hipStreamSynchronize(lanes[0]->stream));
   }
-  DDX_HIP(hipStreamSynchronize(lanes[0]->stream));
   // launches of rounds after a solve's last iteration returned at once:
   // drop them from the timers
   int it[2] = {0, 0}, itmax = 0;
