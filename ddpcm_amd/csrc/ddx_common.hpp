@@ -244,7 +244,8 @@ struct ddx_handle {
   // triples grouped by the sphere that contains the point
   ddx::DevArray<int> paircnt, pairoff;
   // sweep work: units of 64 triples per container, segments per container
-  ddx::DevArray<int> ucnt, uoff, segcnt, segoff;
+  ddx::DevArray<int> ucnt, uoff, toff, segcnt, segoff;
+  ddx::DevArray<int4> wstart;       // where each worker's range starts (k_worker_start)
   int nunit = 0, nworker = 0, nseg_cap = 0;
   int ncu = 0;                      // compute units of the device
   ddx::DevArray<double4> tgeo;    // (cos theta, sin theta, cos phi, sin phi)

@@ -383,12 +383,42 @@ __global__ __launch_bounds__(kSetupThreads) void k_triple_geo(
 // A launch of the sweep hands contiguous ranges of units to a fixed number
 // of workers; a segment is the part of one worker's range inside one
 // container, and each segment leaves one partial L* S vector.
+// toff: first triple of each container (n + 1 entries).
 __global__ void k_unit_count(int n, const int *__restrict__ inl, const int *__restrict__ pairoff,
-                             int *__restrict__ ucnt) {
+                             int *__restrict__ ucnt, int *__restrict__ toff) {
   int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n) return;
-  int t = pairoff[inl[c + 1]] - pairoff[inl[c]];
-  ucnt[c] = (t + kWave - 1) / kWave;
+  const int b = pairoff[inl[c]], e = pairoff[inl[c + 1]];
+  ucnt[c] = (e - b + kWave - 1) / kWave;
+  toff[c] = b;
+  if (c == n - 1) toff[n] = e;
+}
+
+// Where each sweep worker starts: (container, unit, segment, triple) of its
+// first unit, worker w's being floor(w U / G), and the end of the last one's
+// range (G + 1 entries).  Made once per setup: found by every worker of every
+// sweep, the container was a binary search of dependent loads (11 of them at
+// 2000 spheres, 17 in the 512-molecule batch) ahead of the first triple.
+__global__ void k_worker_start(int n, const int *__restrict__ uoff, const int *__restrict__ segoff,
+                               const int *__restrict__ toff, long long U, long long G,
+                               int4 *__restrict__ wstart) {
+  const long long w = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (w > G) return;
+  const int u0 = (int)(w * U / G);
+  if (w == G) {
+    wstart[w] = make_int4(n, u0, 0, 0);
+    return;
+  }
+  int lo = 0, hi = n;   // uoff[lo] <= u0 < uoff[hi]: the last c with uoff[c] <= u0
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (uoff[mid] <= u0) lo = mid;
+    else hi = mid;
+  }
+  const int b = uoff[lo];
+  int seg = segoff[lo];
+  if (u0 > b) seg += 1 + (int)(w - (((long long)b + 1) * G + U - 1) / U);
+  wstart[w] = make_int4(lo, u0, seg, toff[lo] + (u0 - b) * kWave);
 }
 
 // segments per container: its first unit starts one, and so does every
@@ -535,8 +565,9 @@ int run_setup(ddx_handle *h) {
   }
   DDX_TRY(h->ucnt.reserve(n + 1));
   DDX_TRY(h->uoff.reserve(n + 1));
+  DDX_TRY(h->toff.reserve(n + 1));
   hipLaunchKernelGGL(k_unit_count, dim3((n + 255) / 256), dim3(256), 0, s, n, h->inl.p,
-                     h->pairoff.p, h->ucnt.p);
+                     h->pairoff.p, h->ucnt.p, h->toff.p);
   DDX_HIP(hipGetLastError());
   DDX_TRY(scan_exclusive(h->ucnt.p, h->uoff.p, n, h->scan_tmp, s));
   int nunit = 0;
@@ -582,6 +613,12 @@ int run_setup(ddx_handle *h) {
   DDX_HIP(hipGetLastError());
   DDX_TRY(scan_exclusive(h->segcnt.p, h->segoff.p, n, h->scan_tmp, s));
   h->nseg_cap = (int)G + n;   // segments: at most one per container plus one per worker
+  DDX_TRY(h->wstart.reserve((size_t)G + 1));
+  if (G > 0) {
+    hipLaunchKernelGGL(k_worker_start, dim3((unsigned)((G + 256) / 256)), dim3(256), 0, s, n,
+                       h->uoff.p, h->segoff.p, h->toff.p, (long long)nunit, G, h->wstart.p);
+    DDX_HIP(hipGetLastError());
+  }
 
   h->have_geo32 = false;   // the float copies are remade on their next use
   h->fmm.lists_ok = false;  // as are the near lists of the far-field sums

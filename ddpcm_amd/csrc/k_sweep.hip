@@ -459,49 +459,37 @@ __device__ __forceinline__ void sweep_chunk(
 // accumulators and the two-deep load pipeline without spilling)
 template <typename R, int LMAX, bool DIR, bool ADJ>
 __global__ __launch_bounds__(kWave * kSweepWaves, 2) void k_sweep(
-    long long U, long long G, const int *__restrict__ uoff, const int *__restrict__ segoff,
-    const int *__restrict__ inl, const int *__restrict__ pairoff, int n,
+    int G, const int4 *__restrict__ wstart, const int *__restrict__ uoff,
+    const int *__restrict__ segoff, const int *__restrict__ toff,
     const typename Geo<R>::G4 *__restrict__ tgeo,
     const typename Geo<R>::G2 *__restrict__ ttw,
     const int *__restrict__ tslot, const int *__restrict__ tp, const double *__restrict__ Xs,
     R *__restrict__ rw, int spare, const R *__restrict__ xiw, const double *__restrict__ cf,
     double *__restrict__ yp, const DiisState *__restrict__ gdir,
     const DiisState *__restrict__ gadj, const int *__restrict__ inst, int ninst) {
-  const bool dir = DIR && !(gdir && gdir->done);
-  const bool adj = ADJ && !(gadj && gadj->done);
-  if (!dir && !adj) return;
   constexpr int NY = (LMAX + 1) * (LMAX + 1);
   // (the wave index through readfirstlane: the compiler does not see that
   // threadIdx.x / 64 is uniform across a wave, and every quantity below
   // would otherwise live in vector registers and load per lane)
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-  const long long w = (long long)blockIdx.x * kSweepWaves + wave;
+  const int w = (int)blockIdx.x * kSweepWaves + wave;
   if (w >= G) return;
-  const int u0 = (int)(w * U / G), u1 = (int)((w + 1) * U / G);
-  // container of unit u0: the last c with uoff[c] <= u0
-  int lo = 0, hi = n;   // uoff[lo] <= u0 < uoff[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (uoff[mid] <= u0) lo = mid;
-    else hi = mid;
-  }
-  int c = lo;
-  while (uoff[c + 1] <= u0) ++c;   // skip containers without triples
-  // global index of this worker's first segment
-  int seg = segoff[c];
-  if (u0 > uoff[c]) {
-    const long long wlo = (((long long)uoff[c] + 1) * G + U - 1) / U;
-    seg += 1 + (int)(w - wlo);
-  }
-  for (int u = u0; u < u1;) {
-    while (uoff[c + 1] <= u) {
+  const int4 at = wstart[w];
+  const int u1 = wstart[w + 1].y;
+  const bool dir = DIR && !(gdir && gdir->done);
+  const bool adj = ADJ && !(gadj && gadj->done);
+  if (!dir && !adj) return;
+  int c = at.x, seg = at.z, beg = at.w;
+  for (int u = at.y; u < u1;) {
+    int uc = uoff[c + 1];
+    while (uc <= u) {   // on to the next container (some hold no triples)
       ++c;
+      uc = uoff[c + 1];
       seg = segoff[c];
+      beg = toff[c];
     }
-    const int ue = min(u1, uoff[c + 1]);
-    const int cb = pairoff[inl[c]], ce = pairoff[inl[c + 1]];
-    const int beg = cb + (u - uoff[c]) * kWave;
-    const int end = min(ce, cb + (ue - uoff[c]) * kWave);
+    const int ue = min(u1, uc);
+    const int end = min(toff[c + 1], beg + (ue - u) * kWave);
     double *ys = yp + (size_t)seg * NY;
     bool dc = dir, ac = adj;
     if (inst) {
@@ -524,7 +512,6 @@ __global__ __launch_bounds__(kWave * kSweepWaves, 2) void k_sweep(
         sweep_chunk<R, LMAX, false, true>(c, beg, end, tgeo, ttw, tslot, tp, Xs, rw, spare, xiw, cf, ys);
     }
     u = ue;
-    ++seg;
   }
 }
 
@@ -725,9 +712,8 @@ int launch_sweep(ddx_handle *h, hipStream_t s, const double *Xs, R *rw, const R 
   hipExtLaunchKernelGGL((k_sweep<R, LMAX, DIR, ADJ>),
                         dim3((h->nworker + kSweepWaves - 1) / kSweepWaves),
                         dim3(kWave * kSweepWaves), 0, s, tl.b,
-                        tl.e, 0, (long long)h->nunit, (long long)h->nworker, h->uoff.p,
-                        h->segoff.p, h->inl.p, h->pairoff.p, h->n, tgeo, ttw,
-                        h->tslot.p, h->tp.p, Xs, rw, (int)h->ntri, xiw, h->cf.p, yp, gdir, gadj,
+                        tl.e, 0, h->nworker, h->wstart.p, h->uoff.p, h->segoff.p, h->toff.p, tgeo,
+                        ttw, h->tslot.p, h->tp.p, Xs, rw, (int)h->ntri, xiw, h->cf.p, yp, gdir, gadj,
                         h->ninst > 1 ? h->inst.p : nullptr, h->ninst);
   DDX_HIP(hipGetLastError());
   return DDX_OK;
