@@ -36,6 +36,63 @@ int download(double *dst, const double *src, size_t n, hipStream_t s) {
 
 int sync(ddx_handle *h) {
   DDX_HIP(hipStreamSynchronize(h->stream));
+  h->stage_busy = false;
+  return DDX_OK;
+}
+
+// (x, y, z, r) and charges of n spheres from the pinned stage (5 n values:
+// x, y, z, r, q) to the device arrays; without q (only the first 4 n) or
+// without sph (only the charges)
+__global__ void k_unstage(int n, const double *__restrict__ in, double4 *__restrict__ sph,
+                          double *__restrict__ q) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (sph) sph[i] = make_double4(in[i], in[n + i], in[2 * n + i], in[3 * n + i]);
+  if (q) q[i] = in[4 * (size_t)n + i];
+}
+
+// the results of a run into pinned host memory
+__global__ void k_export(int ne, const double *__restrict__ e, int nf,
+                         const double *__restrict__ f, double *__restrict__ out) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < ne) out[k] = e[k];
+  else if (k - ne < nf) out[k] = f[k - ne];
+}
+
+// A call's inputs travel through pinned memory of the handle, read by one
+// kernel on the stream, with no copy call and no wait (a pageable copy of a
+// few hundred bytes holds the caller for about 15 us).
+int stage_inputs(ddx_handle *h, const double *x, const double *y, const double *z,
+                 const double *r, const double *charge) {
+  const size_t n = h->n;
+  if (h->stage_busy) DDX_TRY(sync(h));
+  double *st = h->h_stage;
+  if (x) {
+    std::memcpy(st, x, n * sizeof(double));
+    std::memcpy(st + n, y, n * sizeof(double));
+    std::memcpy(st + 2 * n, z, n * sizeof(double));
+    std::memcpy(st + 3 * n, r, n * sizeof(double));
+    DDX_TRY(h->sph.reserve(n));
+  }
+  if (charge) {
+    std::memcpy(st + 4 * n, charge, n * sizeof(double));
+    DDX_TRY(h->charge.reserve(n));
+  }
+  hipLaunchKernelGGL(k_unstage, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream,
+                     (int)n, h->d_stage, x ? h->sph.p : nullptr, charge ? h->charge.p : nullptr);
+  DDX_HIP(hipGetLastError());
+  h->stage_busy = true;
+  return DDX_OK;
+}
+
+// the time of the last setup, once its events have passed
+int read_setup_time(ddx_handle *h) {
+  if (!h->setup_timed) return DDX_OK;
+  DDX_HIP(hipEventSynchronize(h->ev[6]));
+  float ms = 0.f;
+  DDX_HIP(hipEventElapsedTime(&ms, h->ev[0], h->ev[6]));
+  h->stats.ms_setup = ms;
+  h->setup_timed = false;
   return DDX_OK;
 }
 
@@ -46,22 +103,19 @@ double tol_of(int iconv) {
 }
 
 int set_geometry(ddx_handle *h, const double *x, const double *y, const double *z,
-                 const double *r) {
-  std::vector<double4> sph(h->n);
+                 const double *r, const double *charge) {
   for (int i = 0; i < h->n; ++i) {
     if (!(r[i] > 0.0)) {
       set_error("radius of sphere %d is not positive", i + 1);
       return DDX_ERR_ARG;
     }
-    sph[i] = make_double4(x[i], y[i], z[i], r[i]);
     h->rmax = i == 0 || r[i] > h->rmax ? r[i] : h->rmax;
   }
   h->h_x.assign(x, x + h->n);
   h->h_y.assign(y, y + h->n);
   h->h_z.assign(z, z + h->n);
   h->h_r.assign(r, r + h->n);
-  DDX_TRY(upload(h->sph, sph.data(), h->n, h->stream));
-  return sync(h);
+  return stage_inputs(h, x, y, z, r, charge);
 }
 
 // Start of the direct solve L X = g (rhs in h->rhs, X in h->sigma) on a lane,
@@ -169,6 +223,7 @@ int reserve_vectors(ddx_handle *h) {
 // charges uploaded.  main.f90:178-265.
 int pipeline(ddx_handle *h) {
   hipStream_t s = h->stream;
+  h->results_ok = false;
   DDX_TRY(reserve_vectors(h));
   DDX_TRY(h->phi.reserve((size_t)h->ncav + 1));
   DDX_TRY(h->zeta.reserve((size_t)h->ncav + 1));
@@ -230,7 +285,13 @@ int pipeline(ddx_handle *h) {
     DDX_TRY(field_forces_contract(h, h->charge.p, h->zeta.p, h->fx.p));
     DDX_HIP(hipEventRecord(h->ev[5], s));
   }
+  const int nf = h->igrad ? 3 * h->n : 0;
+  hipLaunchKernelGGL(k_export, dim3((unsigned)((h->ninst + nf + 255) / 256)), dim3(256), 0, s,
+                     h->ninst, h->energy.p, nf, h->fx.p, h->d_out);
+  DDX_HIP(hipGetLastError());
   DDX_TRY(sync(h));
+  h->results_ok = true;
+  DDX_TRY(read_setup_time(h));
   // with forces the two solves run together: ms_direct covers both and
   // ms_adjoint is zero
   float ms = 0.f;
@@ -255,14 +316,13 @@ int pipeline(ddx_handle *h) {
   return DDX_OK;
 }
 
+// (its time is read once the events have passed: here nothing waits)
 int timed_setup(ddx_handle *h) {
   DDX_HIP(hipEventRecord(h->ev[0], h->stream));
   DDX_TRY(run_setup(h));
   DDX_HIP(hipEventRecord(h->ev[6], h->stream));
-  DDX_TRY(sync(h));
-  float ms = 0.f;
-  DDX_HIP(hipEventElapsedTime(&ms, h->ev[0], h->ev[6]));
-  h->stats.ms_setup = ms;
+  h->stage_busy = false;   // run_setup has waited for its counts, past the inputs
+  h->setup_timed = true;
   return DDX_OK;
 }
 
@@ -341,13 +401,35 @@ int create(ddx_handle **out, int n, int count, const int *nsph, const double *x,
       set_error("hipEventCreate failed");
       return fail(DDX_ERR_HIP);
     }
-  for (Lane &ln : h->lane)
-    if (hipHostMalloc((void **)&ln.h_diis, sizeof(DiisState), hipHostMallocDefault) !=
-            hipSuccess ||
-        hipHostGetDevicePointer((void **)&ln.d_rec, ln.h_diis, 0) != hipSuccess) {
+  // one pinned allocation (each is a call of tens of microseconds): the
+  // lanes' records, the setup's counts, a call's inputs, the results
+  {
+    const size_t rec = (sizeof(DiisState) + 63) / 64 * 64, cnt = 64;
+    static_assert(kSetupCounts * sizeof(int) <= 64, "the counts fit their line");
+    const size_t in = 5 * (size_t)n * sizeof(double);
+    const size_t res = (3 * (size_t)n + count) * sizeof(double);
+    char *hp = nullptr, *dp = nullptr;
+    if (hipHostMalloc((void **)&hp, 2 * rec + cnt + in + res, hipHostMallocDefault) !=
+        hipSuccess) {
       set_error("hipHostMalloc failed");
       return fail(DDX_ERR_ALLOC);
     }
+    h->h_pinned = hp;
+    if (hipHostGetDevicePointer((void **)&dp, hp, 0) != hipSuccess) {
+      set_error("hipHostGetDevicePointer failed");
+      return fail(DDX_ERR_HIP);
+    }
+    for (int k = 0; k < 2; ++k) {
+      h->lane[k].h_diis = (DiisState *)(hp + k * rec);
+      h->lane[k].d_rec = (DiisState *)(dp + k * rec);
+    }
+    h->h_counts = (int *)(hp + 2 * rec);
+    h->d_counts = (int *)(dp + 2 * rec);
+    h->h_stage = (double *)(hp + 2 * rec + cnt);
+    h->d_stage = (double *)(dp + 2 * rec + cnt);
+    h->h_out = (double *)(hp + 2 * rec + cnt + in);
+    h->d_out = (double *)(dp + 2 * rec + cnt + in);
+  }
   for (auto &e : h->gev)
     if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
       set_error("hipEventCreate failed");
@@ -399,7 +481,9 @@ int create(ddx_handle **out, int n, int count, const int *nsph, const double *x,
                       hipSuccess ? DDX_OK : DDX_ERR_HIP))
       return fail(rc);
   }
-  if ((rc = set_geometry(h, x, y, z, rvdw)) || (rc = timed_setup(h))) return fail(rc);
+  if ((rc = set_geometry(h, x, y, z, rvdw, nullptr)) || (rc = timed_setup(h)) ||
+      (rc = sync(h)) || (rc = read_setup_time(h)))
+    return fail(rc);
   *out = h;
   return DDX_OK;
 }
@@ -439,8 +523,7 @@ int ddx_batch_init(ddx_handle **out, int count, const int *nsph, const double *x
 int ddx_free(ddx_handle *h) {
   if (!h) return DDX_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  for (Lane &ln : h->lane)
-    if (ln.h_diis) (void)hipHostFree(ln.h_diis);
+  if (h->h_pinned) (void)hipHostFree(h->h_pinned);
   for (auto &e : h->gev)
     if (e) (void)hipEventDestroy(e);
   drop_round_graphs(h);
@@ -539,7 +622,7 @@ int ddx_get_neighbours(const ddx_handle *hc, int *inl, int *nl) {
 int ddx_mkrhs(ddx_handle *h, const double *charge, double *phi, double *psi) {
   if (!h || !charge || !phi || !psi) return DDX_ERR_ARG;
   DDX_TRY(reserve_vectors(h));
-  DDX_TRY(upload(h->charge, charge, h->n, h->stream));
+  DDX_TRY(stage_inputs(h, nullptr, nullptr, nullptr, nullptr, charge));
   DDX_TRY(h->phi.reserve((size_t)h->ncav + 1));
   if (use_fmm(h))
     DDX_TRY(fmm_potential(h, h->charge.p, h->phi.p, nullptr));
@@ -587,6 +670,7 @@ int ddx_cosmo(ddx_handle *h, int star, int cart, const double *phi, const double
               const double *psi, double *sigma, double *esolv) {
   if (!h || !psi || !sigma) return DDX_ERR_ARG;
   DDX_TRY(single(h, "ddx_cosmo"));
+  h->results_ok = false;
   hipStream_t s = h->stream;
   size_t nn = (size_t)h->nylm * h->n;
   DDX_TRY(reserve_vectors(h));
@@ -617,6 +701,7 @@ int ddx_cosmo(ddx_handle *h, int star, int cart, const double *phi, const double
 int ddx_forces_dd(ddx_handle *h, const double *phi, const double *sigma, const double *s_adj,
                   double *fx) {
   if (!h || !phi || !sigma || !s_adj || !fx) return DDX_ERR_ARG;
+  h->results_ok = false;
   hipStream_t s = h->stream;
   size_t nn = (size_t)h->nylm * h->n;
   DDX_TRY(reserve_vectors(h));
@@ -719,11 +804,10 @@ int ddx_get_history(const ddx_handle *h, int star, int cap, double *norms, int *
 int ddx_upload(ddx_handle *h, const double *x, const double *y, const double *z,
                const double *rvdw, const double *charge) {
   if (!h || !x || !y || !z || !rvdw || !charge) return DDX_ERR_ARG;
-  DDX_TRY(set_geometry(h, x, y, z, rvdw));
-  DDX_TRY(upload(h->charge, charge, h->n, h->stream));
+  DDX_TRY(set_geometry(h, x, y, z, rvdw, charge));
   h->have_charge = true;
   h->have_setup = false;
-  return sync(h);
+  return DDX_OK;
 }
 
 int ddx_run(ddx_handle *h) {
@@ -744,6 +828,11 @@ int ddx_result(ddx_handle *h, double *esolv, double *fx) {
 
 int ddx_batch_result(ddx_handle *h, double *esolv, double *fx) {
   if (!h) return DDX_ERR_ARG;
+  if (h->results_ok) {   // the last pipeline left them in pinned memory
+    if (esolv) std::memcpy(esolv, h->h_out, h->ninst * sizeof(double));
+    if (fx && h->igrad) std::memcpy(fx, h->h_out + h->ninst, 3 * (size_t)h->n * sizeof(double));
+    return DDX_OK;
+  }
   if (esolv) DDX_TRY(download(esolv, h->energy.p, h->ninst, h->stream));
   if (fx && h->igrad) DDX_TRY(download(fx, h->fx.p, 3 * (size_t)h->n, h->stream));
   return sync(h);
@@ -757,7 +846,7 @@ int ddx_energy_forces(ddx_handle *h, const double *charge, double *esolv, double
 
 int ddx_batch_energy_forces(ddx_handle *h, const double *charge, double *esolv, double *fx) {
   if (!h || !charge || !esolv) return DDX_ERR_ARG;
-  DDX_TRY(upload(h->charge, charge, h->n, h->stream));
+  DDX_TRY(stage_inputs(h, nullptr, nullptr, nullptr, nullptr, charge));
   h->have_charge = true;
   if (!h->have_setup) DDX_TRY(timed_setup(h));
   const int rc = pipeline(h);
@@ -893,6 +982,7 @@ int ddx_kernel_timer_read(ddx_handle *h, int kernel, int *launches, double *tota
 
 int ddx_get_stats(const ddx_handle *h, ddx_stats *st) {
   if (!h || !st) return DDX_ERR_ARG;
+  DDX_TRY(read_setup_time(const_cast<ddx_handle *>(h)));
   *st = h->stats;
   return DDX_OK;
 }

@@ -24,6 +24,10 @@ constexpr int kUnitsPerWorker = 12;    // units of 64 triples per sweep worker (
 // unit ranges end at different times (four to a workgroup: 6% slower)
 constexpr int kSweepWaves = 1;
 
+// the setup's counts in pinned memory: neighbour pairs, largest degree,
+// triples, exposed points, sweep units
+enum { kCntPairs, kCntDegree, kCntTriples, kCntCav, kCntUnits, kSetupCounts };
+
 void set_error(const char *fmt, ...);
 
 #define DDX_HIP(call)                                                        \
@@ -230,7 +234,7 @@ struct ddx_handle {
   ddx::DevArray<double> charge;
 
   // neighbours, and the spatial hash that finds them
-  ddx::DevArray<int> inl, nl, rev, prow, degcnt;
+  ddx::DevArray<int> inl, nl, rev, degcnt;
   ddx::DevArray<int> ckey, bcnt, boff, bsph, cand;
   ddx::DevArray<int> inst;        // instance of each sphere (empty: one instance)
   double rmax = 0.0;              // largest radius
@@ -238,11 +242,14 @@ struct ddx_handle {
   // per point
   ddx::DevArray<double> fi, ui, zi;
   ddx::DevArray<unsigned long long> tmask;
-  ddx::DevArray<int> ptcnt, ptoff, cavflag, cavidx;
+  ddx::DevArray<int> ptoff, cavidx;
+  // per sphere and run of its points (setup): triples and exposed points, and
+  // their sums before it
+  ddx::DevArray<int> runcnt, runoff, cavcnt, cavrun;
   ddx::DevArray<double> ccav;
 
   // triples grouped by the sphere that contains the point
-  ddx::DevArray<int> paircnt, pairoff;
+  ddx::DevArray<int> paircnt, pairloc, tcnt;
   // sweep work: units of 64 triples per container, segments per container
   ddx::DevArray<int> ucnt, uoff, toff, segcnt, segoff;
   ddx::DevArray<int4> wstart;       // where each worker's range starts (k_worker_start)
@@ -272,6 +279,7 @@ struct ddx_handle {
   std::vector<int4> h_ctile, h_ftile, h_xtile;   // host copies of the tile tables
   std::vector<int> h_fgrp, h_xgrp;
   int maps_n = -1;                // sphere count the block maps were built for
+  int most = 0;                   // spheres of the largest instance
   bool mute_timers = false;       // launches outside the timed classes' meaning
   // sweep workers: by default enough for about kUnitsPerWorker units each (at
   // least kSweepWorkersPerCU per CU); ddx_autotune fixes workers_per_cu
@@ -292,6 +300,15 @@ struct ddx_handle {
   ddx::Lane lane[2];
   ddx::DevArray<double> x, y, rhs, r, part;
   int solve_serial = 0;
+  void *h_pinned = nullptr;   // the pinned block of everything below and the lanes' records
+  // counts of the setup, written by its kernels (pinned host memory)
+  int *h_counts = nullptr, *d_counts = nullptr;
+  // pinned host memory for a call's inputs and for the results (energies,
+  // then forces) that the pipeline leaves there; stage_busy: the device may
+  // still read the inputs; results_ok: the results are those on the device
+  double *h_stage = nullptr, *d_stage = nullptr, *h_out = nullptr, *d_out = nullptr;
+  bool stage_busy = false, results_ok = false;
+  bool setup_timed = false;       // events 0 and 6 bracket a setup not yet read
   hipEvent_t gev[2] = {};           // completion of a group's state copy
   int tag_solve = -1, tag_round = 0;  // attached to timed launches
 

@@ -5,7 +5,22 @@
 
 namespace ddx {
 
-// k_scan.hip — exclusive prefix sums (out has n+1 entries, out[n] = total)
+// k_scan.hip — exclusive prefix sums (out has n+1 entries, out[n] = total) of
+// min(in, cap); rec, if not null, also receives the total and max the largest
+// in (device or pinned host addresses; max for the first of the arrays only)
+struct Scan {
+  const int *in;
+  int *out;
+  size_t n;
+  int cap;
+  int *rec, *max;
+};
+constexpr int kMaxScans = 4;
+struct Scans {
+  Scan s[kMaxScans];
+};
+int scan_arrays(const Scan *scans, int count, DevArray<int> &tmp, hipStream_t s);
+// one array
 int scan_exclusive(const int *in, int *out, size_t n, DevArray<int> &tmp,
                    hipStream_t s);
 

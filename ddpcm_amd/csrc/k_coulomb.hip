@@ -353,6 +353,33 @@ __global__ void k_psi(int n, int nylm, double fac, const double *__restrict__ q,
   psi[k] = (k % nylm == 0) ? fac * q[k / nylm] : 0.0;
 }
 
+// The tile tables of one system (what coulomb_tiles builds for one instance):
+// potential tiles of kTW cavity points, and nfg groups of nfc field tiles, kFW
+// nuclei by `chunk` cavity points each.
+__global__ void k_single_tiles(int n, int ncav, int nct, int nfg, int nfc, int chunk,
+                               int4 *__restrict__ ctile, int4 *__restrict__ ftile,
+                               int *__restrict__ fgrp) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < nct) ctile[b] = make_int4(b * kTW, min(b * kTW + kTW, ncav), 0, n);
+  if (b < nfg * nfc) {
+    const int g = b / nfc, c = b - g * nfc;
+    const long long sb = (long long)c * chunk;
+    ftile[b] = make_int4(g * kFW, min(g * kFW + kFW, n), (int)sb,
+                         (int)min(sb + chunk, (long long)ncav));
+  }
+  if (b <= nfg) fgrp[b] = b * nfc;
+}
+
+// sources per field tile: about 32768 one-wave tiles (several rounds of the
+// resident waves, so that the uneven last chunks of each target tile do not
+// leave CUs idle), whole multiples of kFW and at least 4 kFW; work = target
+// tiles x sources
+long long field_chunk(long long work) {
+  long long chunk = (work + 32767) / 32768;
+  chunk = ((chunk + kFW - 1) / kFW) * kFW;
+  return std::max<long long>(chunk, 4 * kFW);
+}
+
 }  // namespace
 
 // Tiles of kTW targets, per instance q: targets toff[q] .. toff[q+1]-1,
@@ -370,13 +397,7 @@ void coulomb_tiles(const std::vector<int> &toff, const std::vector<int> &soff, b
   for (size_t q = 0; q < ninst; ++q)
     work += (long long)((toff[q + 1] - toff[q] + tw - 1) / tw) * (soff[q + 1] - soff[q]);
   long long chunk = 0x7fffffff;
-  if (split) {
-    // about 32768 one-wave tiles: several rounds of the resident waves, so
-    // that the uneven last chunks of each target tile do not leave CUs idle
-    chunk = (work + 32767) / 32768;
-    chunk = ((chunk + kFW - 1) / kFW) * kFW;
-    if (chunk < 4 * kFW) chunk = 4 * kFW;
-  }
+  if (split) chunk = field_chunk(work);
   tiles.clear();
   grp.clear();
   for (size_t q = 0; q < ninst; ++q) {
@@ -406,6 +427,23 @@ int upload_tiles(ddx_handle *h, DevArray<int4> &dt, const std::vector<int4> &t) 
 }  // namespace
 
 int build_coulomb_tiles(ddx_handle *h) {
+  if (h->ninst == 1) {
+    const int nfg = (h->n + kFW - 1) / kFW;
+    const long long chunk = field_chunk((long long)nfg * h->ncav);
+    const int nfc = std::max<int>(1, (int)((h->ncav + chunk - 1) / chunk));
+    h->nctile = (h->ncav + kTW - 1) / kTW;
+    h->nftile = nfg * nfc;
+    h->nfgrp = nfg;
+    DDX_TRY(h->ctile.reserve((size_t)h->nctile + 1));
+    DDX_TRY(h->ftile.reserve((size_t)h->nftile + 1));
+    DDX_TRY(h->fgrp.reserve((size_t)nfg + 1));
+    const int most = std::max(std::max(h->nctile, h->nftile), nfg + 1);
+    hipLaunchKernelGGL(k_single_tiles, dim3((most + 255) / 256), dim3(256), 0, h->stream, h->n,
+                       h->ncav, h->nctile, nfg, nfc, (int)chunk, h->ctile.p, h->ftile.p,
+                       h->fgrp.p);
+    DDX_HIP(hipGetLastError());
+    return DDX_OK;
+  }
   // the host tables live in the handle until the next setup, so the copies
   // need no wait here
   std::vector<int> g;

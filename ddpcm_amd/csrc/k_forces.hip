@@ -34,7 +34,7 @@ __host__ __device__ constexpr int lmi(int l, int m) { return l * l + l + m; }
 // l-outer, three rows in registers, with polleg's recurrence.
 template <int LMAX, int BT>
 __global__ __launch_bounds__(BT) void k_force_triple(
-    const int *__restrict__ inl, const int *__restrict__ pairoff,
+    const int *__restrict__ toff,
     const double4 *__restrict__ tgeo, const double2 *__restrict__ ttw,
     const double *__restrict__ sigma, const double *__restrict__ cf,
     double4 *__restrict__ fb) {
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(BT) void k_force_triple(
   const int c = blockIdx.x;
   for (int k = threadIdx.x; k < NY; k += BT) xs[k] = cf[k] * sigma[(size_t)c * NY + k];
   __syncthreads();
-  const int beg = pairoff[inl[c]], end = pairoff[inl[c + 1]];
+  const int beg = toff[c], end = toff[c + 1];
   for (int k = beg + threadIdx.x; k < end; k += BT) {
     const double4 g = tgeo[k];
     const double t = ttw[k].x;
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(BT) void k_force_owner(
 // threads over its triples.
 template <int BT>
 __global__ __launch_bounds__(BT) void k_force_container(
-    int ngrid, double eta, const int *__restrict__ inl, const int *__restrict__ pairoff,
+    int ngrid, double eta, const int *__restrict__ toff,
     const double4 *__restrict__ sph, const double4 *__restrict__ grid,
     const int *__restrict__ ptoff, const int *__restrict__ pttri,
     const double2 *__restrict__ ttw, const int *__restrict__ tp,
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(BT) void k_force_container(
     double *__restrict__ fc) {
   __shared__ double lds[4];
   const int c = blockIdx.x;
-  const int beg = pairoff[inl[c]], end = pairoff[inl[c + 1]];
+  const int beg = toff[c], end = toff[c + 1];
   const double4 sc = sph[c];
   const double tlow = 1.0 - eta;
   double f0 = 0.0, f1 = 0.0, f2 = 0.0;
@@ -338,11 +338,11 @@ int launch_triple(ddx_handle *h, const double *sigma, double4 *fb) {
   TimedLaunch tl(h, DDX_K_FORCES, h->stream);
   if (force_waves(h) == 1)
     hipExtLaunchKernelGGL((k_force_triple<LMAX, kWave>), dim3(h->n), dim3(kWave), 0, h->stream,
-                          tl.b, tl.e, 0, h->inl.p, h->pairoff.p, h->tgeo.p, h->ttw.p, sigma,
+                          tl.b, tl.e, 0, h->toff.p, h->tgeo.p, h->ttw.p, sigma,
                           h->cf.p, fb);
   else
     hipExtLaunchKernelGGL((k_force_triple<LMAX, 256>), dim3(h->n), dim3(256), 0, h->stream, tl.b,
-                          tl.e, 0, h->inl.p, h->pairoff.p, h->tgeo.p, h->ttw.p, sigma, h->cf.p,
+                          tl.e, 0, h->toff.p, h->tgeo.p, h->ttw.p, sigma, h->cf.p,
                           fb);
   DDX_HIP(hipGetLastError());
   return DDX_OK;
@@ -398,7 +398,7 @@ int forces_dd(ddx_handle *h, const double *d_phi, const double *d_sigma, const d
                        h->fi.p, h->ui.p, h->zi.p, h->xi.p, d_phi, h->cavidx.p, fo);
     DDX_HIP(hipGetLastError());
     hipLaunchKernelGGL(one ? k_force_container<kWave> : k_force_container<256>, dim3(n),
-                       dim3(one ? kWave : 256), 0, s, h->ngrid, h->eta, h->inl.p, h->pairoff.p,
+                       dim3(one ? kWave : 256), 0, s, h->ngrid, h->eta, h->toff.p,
                        h->sph.p, h->grid.p, h->ptoff.p, h->pttri.p, h->ttw.p, h->tp.p, fb,
                        h->fi.p, h->ui.p, h->xi.p, d_phi, h->cavidx.p, fc);
     DDX_HIP(hipGetLastError());

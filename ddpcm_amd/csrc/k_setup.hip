@@ -16,6 +16,14 @@
 //               pttri lists the triples of each point in neighbour order
 //               (the loop order of calcv, ddcosmo.f90:1701-1739); tslot is
 //               its inverse, the slot of each triple in its point's list.
+//
+// A small system's setup is bound by its launches and host round trips, not
+// by their work, so the counts that later kernels need are made where the data
+// is at hand: k_points also counts the triples of every (container, owner) and
+// leaves the offsets within a sphere's points, the sums over spheres are one
+// scan launch, and the host waits once, for the five totals that size the
+// triple arrays.  60 atoms: 290 us with 45 launches and copies and three waits,
+// now 77 us with 13 launches and one wait; 2000 atoms 490 -> 181 us.
 #include "ddx_device.hpp"
 #include "ddx_kernels.hpp"
 
@@ -71,6 +79,37 @@ __global__ void k_cell_fill(int n, const int *__restrict__ key, const int *__res
   bsph[boff[b] + atomicSub(&bcnt[b], 1) - 1] = i;
 }
 
+// The same search without the hash, for instances of at most kDirectSearch
+// spheres: one wave per sphere i tests every sphere of its instance, in
+// increasing j, 64 at a time.  cand and deg as k_nbr_find leaves them.
+// Up to there one launch of n / 64 tests a wave beats the hash's five
+// (2000 atoms: 35 -> 14 us; 512 molecules of up to 795: 371 us for the find
+// alone -> 67 us; 20 000 atoms: 72 us by the hash, n / 64 tests would take 250).
+constexpr int kDirectSearch = 4096;
+
+__global__ __launch_bounds__(kSetupThreads) void k_nbr_direct(
+    const double4 *__restrict__ sph, const int *__restrict__ inst, const int *__restrict__ soff,
+    int n, int *__restrict__ deg, int *__restrict__ cand) {
+  const int i = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave));
+  if (i >= n) return;
+  const int lane = lane_id();
+  const int sb = inst ? soff[inst[i]] : 0, se = inst ? soff[inst[i] + 1] : n;
+  const double4 si = sph[i];
+  int cnt = 0;
+#pragma unroll 4
+  for (int j0 = sb; j0 < se; j0 += kWave) {
+    const int j = j0 + lane;
+    const double4 sj = sph[min(j, se - 1)];
+    const bool hit = j < se && j != i && spheres_overlap(si, sj);
+    const unsigned long long bal = __ballot(hit);
+    const int pos = cnt + ballot_prefix(bal);
+    if (hit && pos < kMaxDegree) cand[(size_t)i * kMaxDegree + pos] = j;
+    cnt += __popcll(bal);
+  }
+  if (lane == 0) deg[i] = cnt;
+}
+
 // One wave per sphere i: the spheres j != i of its instance that overlap it,
 // from the buckets of the 27 cubes around it, in increasing j, into
 // cand(kMaxDegree, i); deg[i] = their number (also when above kMaxDegree,
@@ -119,7 +158,8 @@ __global__ __launch_bounds__(kSetupThreads) void k_nbr_find(
   __syncthreads();
   if (i < n) {
     if (lane == 0) deg[i] = cnt;
-    if (cnt <= kMaxDegree && lane < cnt) {
+    cnt = min(cnt, kMaxDegree);   // (more is an error, found after this kernel)
+    if (lane < cnt) {
       const int j = list[wv][lane];
       int rank = 0;
       for (int m = 0; m < cnt; ++m) rank += list[wv][m] < j ? 1 : 0;
@@ -128,119 +168,33 @@ __global__ __launch_bounds__(kSetupThreads) void k_nbr_find(
   }
 }
 
-// CSR from the sorted candidates
-__global__ void k_nbr_compact(int n, const int *__restrict__ inl, const int *__restrict__ cand,
-                              int *__restrict__ nl, int *__restrict__ prow) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = (int)(t / kMaxDegree), k = (int)(t % kMaxDegree);
+// One wave per sphere i: its CSR list from the sorted candidates, and
+// rev[q] = position of sphere i in the neighbour list of nl[q] (the number of
+// smaller candidates there).
+__global__ __launch_bounds__(kSetupThreads) void k_nbr_csr(int n, const int *__restrict__ deg,
+                                                           const int *__restrict__ cand,
+                                                           const int *__restrict__ inl,
+                                                           int *__restrict__ nl,
+                                                           int *__restrict__ rev) {
+  const int i = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave));
   if (i >= n) return;
-  const int b = inl[i];
-  if (k < inl[i + 1] - b) {
-    nl[b + k] = cand[t];
-    prow[b + k] = i;
+  const int lane = lane_id();
+  const int d = min(deg[i], kMaxDegree), b = inl[i];
+  const int j = lane < d ? cand[(size_t)i * kMaxDegree + lane] : 0;
+  const int dj = lane < d ? min(deg[j], kMaxDegree) : 0;
+  int r = 0;
+#pragma unroll 4
+  for (int k = 0; k < d; ++k) {
+    const int jk = __builtin_amdgcn_readlane(j, k), dk = __builtin_amdgcn_readlane(dj, k);
+    const int c = cand[(size_t)jk * kMaxDegree + min(lane, max(dk - 1, 0))];
+    const int rank = __popcll(__ballot(lane < dk && c < i));
+    r = lane == k ? rank : r;
   }
-}
-
-// rev[q] = position of sphere prow[q] in the neighbour list of nl[q]
-__global__ void k_nbr_rev(int nnl, const int *__restrict__ inl, const int *__restrict__ nl,
-                          const int *__restrict__ prow, int *__restrict__ rev) {
-  int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nnl) return;
-  int c = prow[q], o = nl[q];
-  int r = -1;
-  for (int k = inl[o]; k < inl[o + 1]; ++k)
-    if (nl[k] == c) { r = k - inl[o]; break; }
-  rev[q] = r;
-}
-
-// fi, ui, zi of every point (ddcosmo.f90:441-498), the mask of the
-// neighbours that contain it and the cavity flags.  One wave per sphere i:
-// its neighbours' centres and radii are staged in LDS (lane k loads
-// neighbour k; the degree is at most 64), then the lanes take the sphere's
-// points n = lane, lane + 64, ..., each adding its terms over the
-// neighbours in list order.  The exact terms (square root, divisions) are
-// evaluated only for the neighbours that may contain the point, |v|^2 at
-// most r^2 (1 + 1e-12): every t < 1 passes that test by far more than any
-// rounding.
-__global__ __launch_bounds__(kSetupThreads) void k_points(
-    const double4 *__restrict__ sph, const double4 *__restrict__ grid, int ngrid,
-    const int *__restrict__ inl, const int *__restrict__ nl, double eta, int igrad,
-    double *__restrict__ fi, double *__restrict__ ui, double *__restrict__ zi,
-    unsigned long long *__restrict__ tmask, int *__restrict__ ptcnt,
-    int *__restrict__ cavflag, int n) {
-  constexpr int kW = kSetupThreads / kWave;
-  __shared__ double4 nb[kW][kWave];
-  const int wave = threadIdx.x / kWave, lane = lane_id();
-  const int i = blockIdx.x * kW + wave;
-  if (i >= n) return;
-  const int beg = inl[i], deg = inl[i + 1] - beg;
-  if (lane < deg) nb[wave][lane] = sph[nl[beg + lane]];
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  const double4 si = sph[i];
-  for (int pn = lane; pn < ngrid; pn += kWave) {
-    const size_t p = (size_t)i * ngrid + pn;
-    const double4 g = grid[pn];
-    double f = 0.0, z0 = 0.0, z1 = 0.0, z2 = 0.0;
-    unsigned long long mask = 0, cand = 0;
-    // the neighbours that may contain the point (the cheap test), then the
-    // exact terms of those only, in neighbour order: the lanes of a wave
-    // would otherwise all wait through the square root and divisions of
-    // every neighbour that contains any one of them
-    for (int k = 0; k < deg; ++k) {
-      const double4 sj = nb[wave][k];
-      double v[3];
-      point_vec(si, g, sj, v);
-      const double d2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-      if (d2 <= sj.w * sj.w * (1.0 + 1e-12)) cand |= 1ull << k;
-    }
-    for (; cand; cand &= cand - 1) {
-      const int k = __ffsll((long long)cand) - 1;
-      const double4 sj = nb[wave][k];
-      double v[3];
-      point_vec(si, g, sj, v);
-      double vv = norm3(v);
-      double t = vv / sj.w;
-      if (t < 1.0) {
-        f += fsw(t, eta);
-        mask |= 1ull << k;
-        if (igrad && t > 1.0 - eta) {
-          double fac = dfsw(t, eta) / sj.w;
-          z0 += fac * v[0] / vv;
-          z1 += fac * v[1] / vv;
-          z2 += fac * v[2] / vv;
-        }
-      }
-    }
-    double u = (f <= 1.0) ? 1.0 - f : 0.0;
-    fi[p] = f;
-    ui[p] = u;
-    if (igrad) {
-      zi[3 * p + 0] = z0;
-      zi[3 * p + 1] = z1;
-      zi[3 * p + 2] = z2;
-    }
-    tmask[p] = mask;
-    ptcnt[p] = __popcll(mask);
-    cavflag[p] = u > 0.0 ? 1 : 0;
+  if (lane < d) {
+    nl[b + lane] = j;
+    rev[b + lane] = r;
   }
-}
-
-__global__ __launch_bounds__(kSetupThreads) void k_ccav(const double4 *__restrict__ sph,
-                                                        const double4 *__restrict__ grid,
-                                                        int ngrid, const int *__restrict__ cavflag,
-                                                        const int *__restrict__ cavidx,
-                                                        double *__restrict__ ccav, size_t np) {
-  const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  if (!cavflag[p]) return;
-  // 32-bit point indices (run_setup checks the count)
-  const unsigned i = (unsigned)p / (unsigned)ngrid, n = (unsigned)p - i * (unsigned)ngrid;
-  int ic = cavidx[p];
-  double4 si = sph[i], g = grid[n];
-  ccav[3 * (size_t)ic + 0] = si.x + si.w * g.x;
-  ccav[3 * (size_t)ic + 1] = si.y + si.w * g.y;
-  ccav[3 * (size_t)ic + 2] = si.z + si.w * g.z;
 }
 
 // OR of a 64-bit value over the wave (every lane receives it)
@@ -264,67 +218,224 @@ __device__ __forceinline__ int pair_of(const int *__restrict__ inl, const int *_
   return inl[nl[q]] + rev[q];
 }
 
-// One wave per owner sphere o: the number of its points inside each of its
-// neighbours (lane kr counts neighbour kr), in one pass over its masks.
-__global__ __launch_bounds__(kSetupThreads) void k_pair_count(
-    int n, int ngrid, const int *__restrict__ inl, const int *__restrict__ nl,
-    const int *__restrict__ rev, const unsigned long long *__restrict__ tmask,
-    int *__restrict__ paircnt) {
-  const int o = blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave;
-  if (o >= n) return;
-  const int lane = lane_id();
-  const int deg = inl[o + 1] - inl[o];
-  int cnt = 0;
-  for (int n0 = 0; n0 < ngrid; n0 += kWave) {
-    const int pn = n0 + lane;
-    const unsigned long long m = pn < ngrid ? tmask[(size_t)o * ngrid + pn] : 0ull;
-    unsigned long long u = wave_or64(m);
-    while (u) {
-      const int kr = __ffsll((long long)u) - 1;
-      u &= u - 1;
-      const int c = __popcll(__ballot((m >> kr) & 1ull));
-      if (lane == kr) cnt += c;
-    }
-  }
-  if (lane < deg) paircnt[pair_of(inl, nl, rev, o, lane)] = cnt;
+// A sphere's points are cut into `runs` (1 or kRuns) runs of whole 64-point
+// groups, one wave each: four where the spheres alone would leave most of the
+// chip's 1024 SIMDs idle.  Run r of sphere i is number i runs + r.
+constexpr int kRuns = 4;
+constexpr int kRunSpheres = 4096;   // fewer spheres than this: kRuns
+
+__device__ __forceinline__ int run_begin(int ngrid, int runs, int r) {
+  return min(ngrid, (ngrid + kWave - 1) / kWave * r / runs * kWave);
 }
 
-// One wave per owner sphere o, in one pass over its masks: for each point n
-// and each neighbour c containing it, the triple's place in c's run of
-// owner o (points ascending), its point index (tp) and its slot in the
+// fi, ui, zi of every point (ddcosmo.f90:441-498) and the mask of the
+// neighbours that contain it.  One wave per run of sphere i: the sphere's
+// neighbours' centres and radii are staged in LDS (lane k loads neighbour k;
+// the degree is at most 64), then the lanes take the run's points 64 at a
+// time, each adding its terms over the neighbours in list order.  The exact
+// terms (square root, divisions) are evaluated only for the neighbours that
+// may contain the point, |v|^2 at most r^2 (1 + 1e-12): every t < 1 passes
+// that test by far more than any rounding.  Beside them, while the masks are
+// in registers: the number of the run's triples and exposed points before
+// each point (ptoff, cavidx, within the run) and in all (runcnt, cavcnt), and
+// its triples with each neighbour (paircnt, by the pair's place in the
+// container's list and r).
+__global__ __launch_bounds__(kSetupThreads) void k_points(
+    const double4 *__restrict__ sph, const double4 *__restrict__ grid, int ngrid, int runs,
+    const int *__restrict__ inl, const int *__restrict__ nl, const int *__restrict__ rev,
+    double eta, int igrad, double *__restrict__ fi, double *__restrict__ ui,
+    double *__restrict__ zi, unsigned long long *__restrict__ tmask, int *__restrict__ ptoff,
+    int *__restrict__ cavidx, int *__restrict__ runcnt, int *__restrict__ cavcnt,
+    int *__restrict__ paircnt, int n) {
+  constexpr int kW = kSetupThreads / kWave;
+  __shared__ double4 nb[kW][kWave];
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  const int run = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kW + wave));
+  const int i = run / runs, r = run - i * runs;
+  if (i >= n) return;
+  const int beg = inl[i], deg = min(inl[i + 1] - beg, kMaxDegree);
+  const int jn = lane < deg ? nl[beg + lane] : 0;
+  if (lane < deg) nb[wave][lane] = sph[jn];
+  wave_lds_sync();
+  const double4 si = sph[i];
+  const int p0 = run_begin(ngrid, runs, r), p1 = run_begin(ngrid, runs, r + 1);
+  int pairs = 0, before = 0, cav = 0;
+  for (int n0 = p0; n0 < p1; n0 += kWave) {
+    const int pn = n0 + lane;
+    const bool in = pn < p1;
+    const size_t p = (size_t)i * ngrid + pn;
+    const double4 g = grid[in ? pn : p1 - 1];
+    double f = 0.0, z0 = 0.0, z1 = 0.0, z2 = 0.0;
+    unsigned long long mask = 0, cand = 0;
+    // the neighbours that may contain the point (the cheap test), then the
+    // exact terms of those only, in neighbour order: the lanes of a wave
+    // would otherwise all wait through the square root and divisions of
+    // every neighbour that contains any one of them
+    for (int k = 0; k < deg; ++k) {
+      const double4 sj = nb[wave][k];
+      double v[3];
+      point_vec(si, g, sj, v);
+      const double d2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+      if (d2 <= sj.w * sj.w * (1.0 + 1e-12)) cand |= 1ull << k;
+    }
+    if (!in) cand = 0;
+    for (; cand; cand &= cand - 1) {
+      const int k = __ffsll((long long)cand) - 1;
+      const double4 sj = nb[wave][k];
+      double v[3];
+      point_vec(si, g, sj, v);
+      double vv = norm3(v);
+      double t = vv / sj.w;
+      if (t < 1.0) {
+        f += fsw(t, eta);
+        mask |= 1ull << k;
+        if (igrad && t > 1.0 - eta) {
+          double fac = dfsw(t, eta) / sj.w;
+          z0 += fac * v[0] / vv;
+          z1 += fac * v[1] / vv;
+          z2 += fac * v[2] / vv;
+        }
+      }
+    }
+    const double u = (f <= 1.0) ? 1.0 - f : 0.0;
+    const unsigned long long open = __ballot(in && u > 0.0);
+    // triples before this lane's point, neighbour by neighbour, and the
+    // neighbours' counts in the lanes that keep them
+    int pre = before, all = 0;
+    unsigned long long w = wave_or64(mask);
+    while (w) {
+      const int kr = __ffsll((long long)w) - 1;
+      w &= w - 1;
+      const unsigned long long hit = __ballot((mask >> kr) & 1ull);
+      const int c = __popcll(hit);
+      pre += ballot_prefix(hit);
+      all += c;
+      if (lane == kr) pairs += c;
+    }
+    if (in) {
+      fi[p] = f;
+      ui[p] = u;
+      if (igrad) {
+        zi[3 * p + 0] = z0;
+        zi[3 * p + 1] = z1;
+        zi[3 * p + 2] = z2;
+      }
+      tmask[p] = mask;
+      ptoff[p] = pre;
+      cavidx[p] = cav + ballot_prefix(open);
+    }
+    before += all;
+    cav += __popcll(open);
+  }
+  if (lane == 0) {
+    runcnt[run] = before;
+    cavcnt[run] = cav;
+  }
+  if (lane < deg) paircnt[(size_t)(inl[jn] + rev[beg + lane]) * runs + r] = pairs;
+}
+
+// One wave per container c: the triples before each of its (owner, run)
+// (pairloc), their number (tcnt) and the sweep units they make (ucnt).
+__global__ __launch_bounds__(kSetupThreads) void k_pair_scan(int n, int runs,
+                                                             const int *__restrict__ inl,
+                                                             const int *__restrict__ paircnt,
+                                                             int *__restrict__ pairloc,
+                                                             int *__restrict__ tcnt,
+                                                             int *__restrict__ ucnt) {
+  const int c = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave));
+  if (c >= n) return;
+  const int lane = lane_id();
+  const int beg = inl[c], deg = inl[c + 1] - beg;
+  const size_t q = ((size_t)beg + lane) * runs;
+  int v[kRuns], sum = 0;
+#pragma unroll
+  for (int r = 0; r < kRuns; ++r) v[r] = (lane < deg && r < runs) ? paircnt[q + r] : 0;
+#pragma unroll
+  for (int r = 0; r < kRuns; ++r) sum += v[r];
+  int incl = sum;
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int t = __shfl_up(incl, off, kWave);
+    if (lane >= off) incl += t;
+  }
+  int at = incl - sum;
+#pragma unroll
+  for (int r = 0; r < kRuns; ++r) {
+    if (lane < deg && r < runs) pairloc[q + r] = at;
+    at += v[r];
+  }
+  if (lane == kWave - 1) {
+    tcnt[c] = incl;
+    ucnt[c] = (incl + kWave - 1) / kWave;
+  }
+}
+
+// One wave per run of owner sphere o, in one pass over its masks: the final
+// ptoff and cavidx of its points and the exposed points' coordinates, and for
+// each point and each neighbour c containing it the triple's place in c's run
+// of owner o (points ascending), its point index (tp) and its slot in the
 // point's list (pttri, tslot).  Lane kr keeps the next place of neighbour
 // kr's run.
-__global__ __launch_bounds__(kSetupThreads) void k_pair_fill(
-    int n, int ngrid, const int *__restrict__ inl, const int *__restrict__ nl,
+__global__ __launch_bounds__(kSetupThreads) void k_sphere_lists(
+    int n, int ngrid, int runs, const double4 *__restrict__ sph,
+    const double4 *__restrict__ grid, const int *__restrict__ inl, const int *__restrict__ nl,
     const int *__restrict__ rev, const unsigned long long *__restrict__ tmask,
-    const int *__restrict__ pairoff, const int *__restrict__ ptoff, int *__restrict__ tp,
+    const double *__restrict__ ui, const int *__restrict__ toff, const int *__restrict__ pairloc,
+    const int *__restrict__ runoff, const int *__restrict__ cavrun, int *__restrict__ ptoff,
+    int *__restrict__ cavidx, double *__restrict__ ccav, int *__restrict__ tp,
     int *__restrict__ pttri, int *__restrict__ tslot) {
-  const int o = blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave;
+  const int run = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave));
+  const int o = run / runs, r = run - o * runs;
   if (o >= n) return;
   const int lane = lane_id();
   const int deg = inl[o + 1] - inl[o];
-  int run = 0;
-  if (lane < deg) run = pairoff[pair_of(inl, nl, rev, o, lane)];
-  for (int n0 = 0; n0 < ngrid; n0 += kWave) {
+  const int tb = runoff[run], cb = cavrun[run];
+  int next = 0;
+  if (lane < deg) {
+    const int c = nl[inl[o] + lane];
+    next = toff[c] + pairloc[(size_t)pair_of(inl, nl, rev, o, lane) * runs + r];
+  }
+  const double4 so = sph[o];
+  const int p0 = run_begin(ngrid, runs, r), p1 = run_begin(ngrid, runs, r + 1);
+  for (int n0 = p0; n0 < p1; n0 += kWave) {
     const int pn = n0 + lane;
-    const size_t p = (size_t)o * ngrid + pn;
-    const unsigned long long m = pn < ngrid ? tmask[p] : 0ull;
-    unsigned long long u = wave_or64(m);
-    while (u) {
-      const int kr = __ffsll((long long)u) - 1;
-      u &= u - 1;
+    const bool in = pn < p1;
+    const size_t p = (size_t)o * ngrid + min(pn, p1 - 1);
+    const unsigned long long m = in ? tmask[p] : 0ull;
+    const double u = ui[p];
+    const int first = tb + ptoff[p], ic = cb + cavidx[p];
+    if (in) {
+      ptoff[p] = first;
+      cavidx[p] = ic;
+      if (u > 0.0) {
+        const double4 g = grid[pn];
+        ccav[3 * (size_t)ic + 0] = so.x + so.w * g.x;
+        ccav[3 * (size_t)ic + 1] = so.y + so.w * g.y;
+        ccav[3 * (size_t)ic + 2] = so.z + so.w * g.z;
+      }
+    }
+    unsigned long long w = wave_or64(m);
+    while (w) {
+      const int kr = __ffsll((long long)w) - 1;
+      w &= w - 1;
       const bool hit = (m >> kr) & 1ull;
       const unsigned long long b = __ballot(hit);
-      const int base = __shfl(run, kr, kWave);
+      const int base = __builtin_amdgcn_readlane(next, kr);
       if (hit) {
         const int idx = base + ballot_prefix(b);
-        const int slot = ptoff[p] + __popcll(m & ((1ull << kr) - 1ull));
+        const int slot = first + __popcll(m & ((1ull << kr) - 1ull));
         tp[idx] = (int)p;
         pttri[slot] = idx;
         tslot[idx] = slot;
       }
-      if (lane == kr) run += __popcll(b);
+      if (lane == kr) next += __popcll(b);
     }
+  }
+  if (run == n * runs - 1 && lane == 0) {
+    const size_t np = (size_t)n * ngrid;
+    ptoff[np] = runoff[run + 1];
+    cavidx[np] = cavrun[run + 1];
   }
 }
 
@@ -352,19 +463,20 @@ __device__ __forceinline__ void triple_record(const double4 &so, const double4 &
   tw = make_double2(t, w);
 }
 
-// One wave per container c: the records of its triples, all lanes busy, and
-// with g32 / w32 the FP32 sweeps' records of them (geo32_of, and W).
+// `wpc` waves (1 or 4) per container c: the records of its triples, all lanes
+// busy, and with g32 / w32 the FP32 sweeps' records of them (geo32_of, and W).
 __global__ __launch_bounds__(kSetupThreads) void k_triple_geo(
-    int n, int ngrid, double eta, const double4 *__restrict__ sph,
-    const double4 *__restrict__ grid, const int *__restrict__ inl,
-    const int *__restrict__ pairoff, const int *__restrict__ tp, const double *__restrict__ fi,
-    double4 *__restrict__ tgeo, double2 *__restrict__ ttw, float4 *__restrict__ g32,
-    float *__restrict__ w32) {
-  const int c = blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave;
+    int n, int ngrid, int wpc, double eta, const double4 *__restrict__ sph,
+    const double4 *__restrict__ grid, const int *__restrict__ toff, const int *__restrict__ tp,
+    const double *__restrict__ fi, double4 *__restrict__ tgeo, double2 *__restrict__ ttw,
+    float4 *__restrict__ g32, float *__restrict__ w32) {
+  const int w = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * (kSetupThreads / kWave) + threadIdx.x / kWave));
+  const int c = w / wpc;
   if (c >= n) return;
   const double4 sc = sph[c];
-  const int end = pairoff[inl[c + 1]];
-  for (int k = pairoff[inl[c]] + lane_id(); k < end; k += kWave) {
+  const int end = toff[c + 1];
+  for (int k = toff[c] + (w - c * wpc) * kWave + lane_id(); k < end; k += wpc * kWave) {
     const unsigned p = (unsigned)tp[k];
     const unsigned o = p / (unsigned)ngrid, pn = p - o * (unsigned)ngrid;
     double4 a;
@@ -383,17 +495,6 @@ __global__ __launch_bounds__(kSetupThreads) void k_triple_geo(
 // A launch of the sweep hands contiguous ranges of units to a fixed number
 // of workers; a segment is the part of one worker's range inside one
 // container, and each segment leaves one partial L* S vector.
-// toff: first triple of each container (n + 1 entries).
-__global__ void k_unit_count(int n, const int *__restrict__ inl, const int *__restrict__ pairoff,
-                             int *__restrict__ ucnt, int *__restrict__ toff) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-  const int b = pairoff[inl[c]], e = pairoff[inl[c + 1]];
-  ucnt[c] = (e - b + kWave - 1) / kWave;
-  toff[c] = b;
-  if (c == n - 1) toff[n] = e;
-}
-
 // Where each sweep worker starts: (container, unit, segment, triple) of its
 // first unit, worker w's being floor(w U / G), and the end of the last one's
 // range (G + 1 entries).  Made once per setup: found by every worker of every
@@ -437,26 +538,11 @@ __global__ void k_seg_count(int n, const int *__restrict__ uoff, long long U, lo
   segcnt[c] = cnt;
 }
 
-// the largest neighbour count into *out (zeroed before): a block maximum,
-// then one atomic maximum per workgroup
-__global__ __launch_bounds__(256) void k_max_degree(int n, const int *__restrict__ deg,
-                                                    int *__restrict__ out) {
-  __shared__ int wm[256 / kWave];
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  int m = wave_max_int(i < n ? deg[i] : 0);
-  if (lane_id() == 0) wm[threadIdx.x / kWave] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 256 / kWave; ++w) m = max(m, wm[w]);
-    atomicMax(out, max(m, wm[0]));
-  }
-}
-
-// cavity offset of each instance: the cavity index of its first point
-__global__ void k_cav_offsets(int ninst, int ngrid, const int *__restrict__ soff,
-                              const int *__restrict__ cavidx, int *__restrict__ out) {
+// cavity offset of each instance: the exposed points before its first sphere
+__global__ void k_cav_offsets(int ninst, int runs, const int *__restrict__ soff,
+                              const int *__restrict__ cavrun, int *__restrict__ out) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q <= ninst) out[q] = cavidx[(size_t)soff[q] * ngrid];
+  if (q <= ninst) out[q] = cavrun[(size_t)soff[q] * runs];
 }
 
 }  // namespace
@@ -473,121 +559,115 @@ int run_setup(ddx_handle *h) {
     return DDX_ERR_CAPACITY;
   }
 
-  // neighbour list on the spatial hash
-  unsigned T = 64;
-  while (T < 2u * (unsigned)n) T <<= 1;
-  const double inv_h = 1.0 / (2.0 * h->rmax * (1.0 + 1e-12));
   const int *inst = h->inst.p;
-  DDX_TRY(h->degcnt.reserve(n + 1));
-  DDX_TRY(h->inl.reserve(n + 1));
-  DDX_TRY(h->ckey.reserve(n));
-  DDX_TRY(h->bcnt.reserve(T + 1));
-  DDX_TRY(h->boff.reserve(T + 1));
-  DDX_TRY(h->bsph.reserve(n));
-  DDX_TRY(h->cand.reserve((size_t)n * kMaxDegree));
-  DDX_HIP(hipMemsetAsync(h->bcnt.p, 0, (T + 1) * sizeof(int), s));
-  hipLaunchKernelGGL(k_cell_count, dim3((n + 255) / 256), dim3(256), 0, s, h->sph.p, inst, n,
-                     inv_h, T - 1, h->ckey.p, h->bcnt.p);
-  DDX_HIP(hipGetLastError());
-  DDX_TRY(scan_exclusive(h->bcnt.p, h->boff.p, T, h->scan_tmp, s));
-  hipLaunchKernelGGL(k_cell_fill, dim3((n + 255) / 256), dim3(256), 0, s, n, h->ckey.p,
-                     h->boff.p, h->bcnt.p, h->bsph.p);
-  DDX_HIP(hipGetLastError());
-  {
-    const int W = kSetupThreads / kWave;
-    hipLaunchKernelGGL(k_nbr_find, dim3((n + W - 1) / W), dim3(kSetupThreads), 0, s, h->sph.p,
-                       inst, n, inv_h, T - 1, h->boff.p, h->bsph.p, h->degcnt.p, h->cand.p);
-    DDX_HIP(hipGetLastError());
-  }
-  DDX_TRY(scan_exclusive(h->degcnt.p, h->inl.p, n, h->scan_tmp, s));
-  // the largest degree into degcnt[n] (the scan reads the first n)
-  DDX_HIP(hipMemsetAsync(h->degcnt.p + n, 0, sizeof(int), s));
-  if (n > 0) {
-    hipLaunchKernelGGL(k_max_degree, dim3((n + 255) / 256), dim3(256), 0, s, n, h->degcnt.p,
-                       h->degcnt.p + n);
-    DDX_HIP(hipGetLastError());
-  }
-  int nnl = 0, maxdeg = 0;
-  DDX_HIP(hipMemcpyAsync(&maxdeg, h->degcnt.p + n, sizeof(int), hipMemcpyDeviceToHost, s));
-  DDX_HIP(hipMemcpyAsync(&nnl, h->inl.p + n, sizeof(int), hipMemcpyDeviceToHost, s));
-  DDX_HIP(hipStreamSynchronize(s));
-  h->nnl = nnl;
-  h->maxdeg = maxdeg;
-  if (maxdeg > kMaxDegree) {
-    set_error("a sphere overlaps %d others; at most %d are supported", maxdeg, kMaxDegree);
-    return DDX_ERR_CAPACITY;
-  }
-  DDX_TRY(h->nl.reserve(nnl + 1));
-  DDX_TRY(h->rev.reserve(nnl + 1));
-  DDX_TRY(h->paircnt.reserve(nnl + 1));
-  DDX_TRY(h->pairoff.reserve(nnl + 1));
-  DDX_TRY(h->prow.reserve(nnl + 1));
-  if (nnl > 0) {
-    const size_t nt = (size_t)n * kMaxDegree;
-    hipLaunchKernelGGL(k_nbr_compact, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, n,
-                       h->inl.p, h->cand.p, h->nl.p, h->prow.p);
-    DDX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_nbr_rev, dim3((nnl + 255) / 256), dim3(256), 0, s, nnl, h->inl.p,
-                       h->nl.p, h->prow.p, h->rev.p);
-    DDX_HIP(hipGetLastError());
+  const int W = kSetupThreads / kWave;
+  const dim3 per_sphere((n + W - 1) / W);
+  if (h->maps_n != n) {
+    DDX_TRY(h->soff.reserve(h->ninst + 1));
+    DDX_HIP(hipMemcpyAsync(h->soff.p, h->h_soff.data(), (h->ninst + 1) * sizeof(int),
+                           hipMemcpyHostToDevice, s));
+    h->most = 0;
+    for (int q = 0; q < h->ninst; ++q) h->most = std::max(h->most, h->h_soff[q + 1] - h->h_soff[q]);
   }
 
-  // per-point quantities
+  // neighbour lists; the arrays are sized by the degree cap, so that nothing
+  // here waits for a count
+  DDX_TRY(h->degcnt.reserve(n + 1));
+  DDX_TRY(h->inl.reserve(n + 1));
+  DDX_TRY(h->cand.reserve((size_t)n * kMaxDegree));
+  if (h->most <= kDirectSearch) {
+    hipLaunchKernelGGL(k_nbr_direct, per_sphere, dim3(kSetupThreads), 0, s, h->sph.p, inst,
+                       h->soff.p, n, h->degcnt.p, h->cand.p);
+    DDX_HIP(hipGetLastError());
+  } else {
+    unsigned T = 64;
+    while (T < 2u * (unsigned)n) T <<= 1;
+    const double inv_h = 1.0 / (2.0 * h->rmax * (1.0 + 1e-12));
+    DDX_TRY(h->ckey.reserve(n));
+    DDX_TRY(h->bcnt.reserve(T + 1));
+    DDX_TRY(h->boff.reserve(T + 1));
+    DDX_TRY(h->bsph.reserve(n));
+    DDX_HIP(hipMemsetAsync(h->bcnt.p, 0, (T + 1) * sizeof(int), s));
+    hipLaunchKernelGGL(k_cell_count, dim3((n + 255) / 256), dim3(256), 0, s, h->sph.p, inst, n,
+                       inv_h, T - 1, h->ckey.p, h->bcnt.p);
+    DDX_HIP(hipGetLastError());
+    DDX_TRY(scan_exclusive(h->bcnt.p, h->boff.p, T, h->scan_tmp, s));
+    hipLaunchKernelGGL(k_cell_fill, dim3((n + 255) / 256), dim3(256), 0, s, n, h->ckey.p,
+                       h->boff.p, h->bcnt.p, h->bsph.p);
+    DDX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_nbr_find, per_sphere, dim3(kSetupThreads), 0, s, h->sph.p, inst, n,
+                       inv_h, T - 1, h->boff.p, h->bsph.p, h->degcnt.p, h->cand.p);
+    DDX_HIP(hipGetLastError());
+  }
+  {
+    const Scan deg = {h->degcnt.p, h->inl.p, (size_t)n, kMaxDegree, h->d_counts + kCntPairs,
+                      h->d_counts + kCntDegree};
+    DDX_TRY(scan_arrays(&deg, 1, h->scan_tmp, s));
+  }
+  const size_t cap = (size_t)n * kMaxDegree + 1;
+  const int runs = n < kRunSpheres ? kRuns : 1;
+  DDX_TRY(h->nl.reserve(cap));
+  DDX_TRY(h->rev.reserve(cap));
+  DDX_TRY(h->paircnt.reserve(cap * runs));
+  DDX_TRY(h->pairloc.reserve(cap * runs));
+  hipLaunchKernelGGL(k_nbr_csr, per_sphere, dim3(kSetupThreads), 0, s, n, h->degcnt.p, h->cand.p,
+                     h->inl.p, h->nl.p, h->rev.p);
+  DDX_HIP(hipGetLastError());
+
+  // per-point quantities, and the counts of the triples
+  const size_t nrun = (size_t)n * runs;
   DDX_TRY(h->fi.reserve(np));
   DDX_TRY(h->ui.reserve(np));
   if (h->igrad) DDX_TRY(h->zi.reserve(3 * np));
   DDX_TRY(h->tmask.reserve(np));
-  DDX_TRY(h->ptcnt.reserve(np + 1));
   DDX_TRY(h->ptoff.reserve(np + 1));
-  DDX_TRY(h->cavflag.reserve(np + 1));
   DDX_TRY(h->cavidx.reserve(np + 1));
-  const dim3 pg((unsigned)((np + kSetupThreads - 1) / kSetupThreads));
-  hipLaunchKernelGGL(k_points, dim3((n + kSetupThreads / kWave - 1) / (kSetupThreads / kWave)),
-                     dim3(kSetupThreads), 0, s, h->sph.p, h->grid.p, ng, h->inl.p, h->nl.p, h->eta,
-                     h->igrad, h->fi.p, h->ui.p, h->igrad ? h->zi.p : nullptr, h->tmask.p,
-                     h->ptcnt.p, h->cavflag.p, n);
-  DDX_HIP(hipGetLastError());
-  DDX_TRY(scan_exclusive(h->ptcnt.p, h->ptoff.p, np, h->scan_tmp, s));
-  DDX_TRY(scan_exclusive(h->cavflag.p, h->cavidx.p, np, h->scan_tmp, s));
-  int ntri = 0, ncav = 0;
-  DDX_HIP(hipMemcpyAsync(&ntri, h->ptoff.p + np, sizeof(int), hipMemcpyDeviceToHost, s));
-  DDX_HIP(hipMemcpyAsync(&ncav, h->cavidx.p + np, sizeof(int), hipMemcpyDeviceToHost, s));
-
-  // triples per neighbour pair, grouped by container
-  if (nnl > 0) {
-    const int wpb = kSetupThreads / kWave;
-    hipLaunchKernelGGL(k_pair_count, dim3((n + wpb - 1) / wpb), dim3(kSetupThreads), 0, s, n, ng,
-                       h->inl.p, h->nl.p, h->rev.p, h->tmask.p, h->paircnt.p);
-    DDX_HIP(hipGetLastError());
-    DDX_TRY(scan_exclusive(h->paircnt.p, h->pairoff.p, nnl, h->scan_tmp, s));
-  } else {
-    DDX_HIP(hipMemsetAsync(h->pairoff.p, 0, sizeof(int), s));
-  }
-  DDX_TRY(h->ucnt.reserve(n + 1));
-  DDX_TRY(h->uoff.reserve(n + 1));
+  DDX_TRY(h->runcnt.reserve(nrun));
+  DDX_TRY(h->runoff.reserve(nrun + 1));
+  DDX_TRY(h->cavcnt.reserve(nrun));
+  DDX_TRY(h->cavrun.reserve(nrun + 1));
+  DDX_TRY(h->tcnt.reserve(n));
   DDX_TRY(h->toff.reserve(n + 1));
-  hipLaunchKernelGGL(k_unit_count, dim3((n + 255) / 256), dim3(256), 0, s, n, h->inl.p,
-                     h->pairoff.p, h->ucnt.p, h->toff.p);
+  DDX_TRY(h->ucnt.reserve(n));
+  DDX_TRY(h->uoff.reserve(n + 1));
+  const dim3 per_run((unsigned)((nrun + W - 1) / W));
+  hipLaunchKernelGGL(k_points, per_run, dim3(kSetupThreads), 0, s, h->sph.p, h->grid.p, ng, runs,
+                     h->inl.p, h->nl.p, h->rev.p, h->eta, h->igrad, h->fi.p, h->ui.p,
+                     h->igrad ? h->zi.p : nullptr, h->tmask.p, h->ptoff.p, h->cavidx.p,
+                     h->runcnt.p, h->cavcnt.p, h->paircnt.p, n);
   DDX_HIP(hipGetLastError());
-  DDX_TRY(scan_exclusive(h->ucnt.p, h->uoff.p, n, h->scan_tmp, s));
-  int nunit = 0;
-  DDX_HIP(hipMemcpyAsync(&nunit, h->uoff.p + n, sizeof(int), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_pair_scan, per_sphere, dim3(kSetupThreads), 0, s, n, runs, h->inl.p,
+                     h->paircnt.p, h->pairloc.p, h->tcnt.p, h->ucnt.p);
+  DDX_HIP(hipGetLastError());
+  {
+    constexpr int all = 0x7fffffff;
+    const Scan sums[4] = {
+        {h->runcnt.p, h->runoff.p, nrun, all, h->d_counts + kCntTriples, nullptr},
+        {h->cavcnt.p, h->cavrun.p, nrun, all, h->d_counts + kCntCav, nullptr},
+        {h->tcnt.p, h->toff.p, (size_t)n, all, nullptr, nullptr},
+        {h->ucnt.p, h->uoff.p, (size_t)n, all, h->d_counts + kCntUnits, nullptr}};
+    DDX_TRY(scan_arrays(sums, 4, h->scan_tmp, s));
+  }
   // the cavity offset of each instance, read back with the counts
   if (h->ninst > 1) {
-    if (h->maps_n != n) {
-      DDX_TRY(h->soff.reserve(h->ninst + 1));
-      DDX_HIP(hipMemcpyAsync(h->soff.p, h->h_soff.data(), (h->ninst + 1) * sizeof(int),
-                             hipMemcpyHostToDevice, s));
-    }
     DDX_TRY(h->cavoff.reserve((size_t)h->ninst + 1));
     hipLaunchKernelGGL(k_cav_offsets, dim3((h->ninst + 256) / 256), dim3(256), 0, s, h->ninst,
-                       ng, h->soff.p, h->cavidx.p, h->cavoff.p);
+                       runs, h->soff.p, h->cavrun.p, h->cavoff.p);
     DDX_HIP(hipGetLastError());
     h->h_cavoff.resize(h->ninst + 1);
     DDX_HIP(hipMemcpyAsync(h->h_cavoff.data(), h->cavoff.p, (h->ninst + 1) * sizeof(int),
                            hipMemcpyDeviceToHost, s));
   }
   DDX_HIP(hipStreamSynchronize(s));
+  const int nnl = h->h_counts[kCntPairs], maxdeg = h->h_counts[kCntDegree];
+  const int ntri = h->h_counts[kCntTriples], ncav = h->h_counts[kCntCav];
+  const int nunit = h->h_counts[kCntUnits];
+  h->nnl = nnl;
+  h->maxdeg = maxdeg;
+  if (maxdeg > kMaxDegree) {
+    set_error("a sphere overlaps %d others; at most %d are supported", maxdeg, kMaxDegree);
+    return DDX_ERR_CAPACITY;
+  }
   h->ntri = ntri;
   h->ncav = ncav;
   h->nunit = nunit;
@@ -627,13 +707,13 @@ int run_setup(ddx_handle *h) {
   DDX_TRY(h->tp.reserve(ntri + 1));
   DDX_TRY(h->pttri.reserve(ntri + 1));
   DDX_TRY(h->tslot.reserve(ntri + 1));
-  if (nnl > 0) {
-    const int wpb = kSetupThreads / kWave;
-    const dim3 grid_o((n + wpb - 1) / wpb);
-    hipLaunchKernelGGL(k_pair_fill, grid_o, dim3(kSetupThreads), 0, s, n, ng, h->inl.p, h->nl.p,
-                       h->rev.p, h->tmask.p, h->pairoff.p, h->ptoff.p, h->tp.p, h->pttri.p,
-                       h->tslot.p);
-    DDX_HIP(hipGetLastError());
+  DDX_TRY(h->ccav.reserve(3 * (size_t)ncav + 3));
+  hipLaunchKernelGGL(k_sphere_lists, per_run, dim3(kSetupThreads), 0, s, n, ng, runs, h->sph.p,
+                     h->grid.p, h->inl.p, h->nl.p, h->rev.p, h->tmask.p, h->ui.p, h->toff.p,
+                     h->pairloc.p, h->runoff.p, h->cavrun.p, h->ptoff.p, h->cavidx.p, h->ccav.p,
+                     h->tp.p, h->pttri.p, h->tslot.p);
+  DDX_HIP(hipGetLastError());
+  if (ntri > 0) {
     // the float copies come with the records when the handle runs the mixed
     // precision, else on the first FP32 sweep
     const bool f32 = h->prec == DDX_PREC_MIXED;
@@ -641,25 +721,16 @@ int run_setup(ddx_handle *h) {
       DDX_TRY(h->tgeo32.reserve(ntri + 1));
       DDX_TRY(h->ttw32.reserve(ntri + 1));
     }
-    hipLaunchKernelGGL(k_triple_geo, grid_o, dim3(kSetupThreads), 0, s, n, ng, h->eta, h->sph.p,
-                       h->grid.p, h->inl.p, h->pairoff.p, h->tp.p, h->fi.p, h->tgeo.p,
-                       h->ttw.p, f32 ? h->tgeo32.p : nullptr, f32 ? h->ttw32.p : nullptr);
+    hipLaunchKernelGGL(k_triple_geo, per_run, dim3(kSetupThreads), 0, s, n, ng, runs, h->eta,
+                       h->sph.p, h->grid.p, h->toff.p, h->tp.p, h->fi.p, h->tgeo.p, h->ttw.p,
+                       f32 ? h->tgeo32.p : nullptr, f32 ? h->ttw32.p : nullptr);
     DDX_HIP(hipGetLastError());
     h->have_geo32 = f32;
   }
-  DDX_TRY(h->ccav.reserve(3 * (size_t)ncav + 3));
-  hipLaunchKernelGGL(k_ccav, pg, dim3(kSetupThreads), 0, s, h->sph.p, h->grid.p, ng,
-                     h->cavflag.p, h->cavidx.p, h->ccav.p, np);
-  DDX_HIP(hipGetLastError());
   // the solver's block maps (once per handle: they depend on the sphere
-  // counts only; a batch's instance offsets went up with the counts above),
+  // counts only),
   // Coulomb tiles
   if (h->maps_n != n) {
-    if (h->ninst == 1) {
-      DDX_TRY(h->soff.reserve(h->ninst + 1));
-      DDX_HIP(hipMemcpyAsync(h->soff.p, h->h_soff.data(), (h->ninst + 1) * sizeof(int),
-                             hipMemcpyHostToDevice, s));
-    }
     DDX_TRY(build_solver_maps(h));
     h->maps_n = n;
   }

@@ -14,6 +14,12 @@
   solutions bit for bit, at one and several workgroups, with a workgroup's
   second element per thread absent, partial and full.  (At these sizes every
   sweep worker has one unit, so the operators' sums are split alike.)
+* test_setup_at_its_branches: the setup where its kernels change (direct or
+  hashed neighbour search, one or four waves a sphere, one or several tiles of
+  the prefix sums, fewer points than a wave): the neighbour lists and exposed
+  points against the definition evaluated here, and the triple lists, which
+  the two operators read in different orders, by <u, L v> = <L* u, v> (1e-12
+  of |u| |L v|: sums of up to 1e6 terms, rounding 1e-16 each).
 """
 import numpy as np
 import pytest
@@ -57,3 +63,38 @@ def test_single_system_equals_batch_of_two(n, lmax, ngrid, mixed):
         one, two = h.get(name), b.get(name)
         assert np.array_equal(one, two[:n]) and np.array_equal(one, two[n:]), name
     assert e == eb[0] == eb[1]
+
+
+@pytest.mark.parametrize("n,ngrid", [(1, 6), (5, 14), (65, 74), (300, 302), (2048, 26),
+                                     (2049, 26), (4095, 14), (4096, 14), (4097, 14)])
+def test_setup_at_its_branches(n, ngrid):
+    from ddpcm_amd.ddx import DDCosmo
+    from ddpcm_amd.inputs import synthetic_input
+    d = synthetic_input(n, 9 + n, 3, ngrid)
+    x, y, z, r = d.bohr()
+    h = DDCosmo(x, y, z, r, 3, ngrid)
+    c = np.stack([x, y, z], 1)
+    inl, nl = h.neighbours()
+    fi = h.get("fi")
+    grid = h.get("grid")
+    for i in range(n):
+        v = c[i] - c
+        near = (v * v).sum(1) <= (r[i] + r) ** 2
+        near[i] = False
+        j = np.flatnonzero(near)
+        assert np.array_equal(nl[inl[i] - 1:inl[i + 1] - 1] - 1, j)
+        p = c[i] + r[i] * grid
+        t = np.sqrt((((p[:, None] - c[None, j]) ** 2).sum(2))) / r[j]
+        chi = (1 - t) ** 3 * (6 * t * t + (15 * 0.1 - 12) * t + 0.1 - 1.5 + 6) / 0.1 ** 5
+        f = np.where(t >= 1, 0.0, np.where(t <= 0.9, 1.0, chi)).sum(1)
+        # (chi changes by up to 19 per unit t near the inner edge; t to 1e-14)
+        assert np.max(np.abs(fi[i] - f), initial=0.0) <= 1e-11
+    ui = h.get("ui")
+    assert np.array_equal(ui, np.where(fi <= 1.0, 1.0 - fi, 0.0))
+    own, pt = np.nonzero(ui > 0.0)
+    assert h.ncav == own.size
+    np.testing.assert_allclose(h.ccav, c[own] + r[own, None] * grid[pt], rtol=0, atol=1e-12)
+    rng = np.random.default_rng(1)
+    u, v = rng.standard_normal((2, n, 16))
+    lv, lu = h.lx(v), h.lstarx(u)
+    assert abs((u * lv).sum() - (lu * v).sum()) <= 1e-12 * np.linalg.norm(u) * np.linalg.norm(lv)
