@@ -459,10 +459,18 @@ __global__ __launch_bounds__(256) void k_project_g(int nylm, int ngrid, int ldm,
 // of S, contiguous in memory, are staged in LDS once; the four waves take
 // the point tiles of 16 (w, w + 4, ...), each an MFMA chain over lm with A
 // = the Y rows of the tile's points from YT (lm-major, zero-padded: each
-// quarter-wave reads 16 consecutive points, and the A operands of 8
-// k-steps are loaded before their MFMAs) and B from LDS.  Each finished
+// quarter-wave reads 16 consecutive points) and B from LDS.  Each finished
 // tile goes back through LDS so that 16 lanes store one sphere's 16 points
 // as one contiguous run.
+//   Where the spheres are few the kernel is bound by its chain of loads, so
+// the rows of S are loaded kStage values a thread at a time before any is
+// stored (one at a time, their latencies added up to most of the launch), the
+// first A operands load beside them, and the A operands of the next 8 k-steps
+// (or of the next tile's first) load while this step's MFMAs run.  Average
+// launch 12.4 -> 9.9 us at 200 atoms and lmax 10, 10.4 -> 8.9 us at 300 atoms
+// and lmax 8, 166 -> 150 us at 20 000 atoms and lmax 10; unchanged at 2000 atoms
+// and in the 512-molecule batch.
+constexpr int kStage = 16;
 template <typename T, int J>
 __global__ __launch_bounds__(256) void k_expand_t(int nylm, int ngrid, int ldnt, int nsph,
                                                   const T *__restrict__ YT,
@@ -479,26 +487,42 @@ __global__ __launch_bounds__(256) void k_expand_t(int nylm, int ngrid, int ldnt,
   const int nsp = min(16 * J, nsph - i0);
   // spheres whose molecules have all converged are not read again
   if (!spheres_active(gate, inst, ninst, i0, i0 + nsp)) return;
-  for (int k = threadIdx.x; k < 16 * J * nylm; k += 256)
-    sS[k] = k < nsp * nylm ? (T)S[(size_t)nylm * i0 + k] : T(0);
-  __syncthreads();
   const int lane = lane_id(), wave = threadIdx.x / kWave;
   const int row = lane & 15, kq = lane >> 4;
   T *trw = tr + wave * J * 16 * 17;
   const int ntile = (ngrid + 15) / 16;
-  for (int pt = wave + 4 * blockIdx.y; pt < ntile; pt += 4 * gridDim.y) {
+  const int nk = (nylm + 3) / 4;
+  // A operands of k-steps c0 .. c0 + 7 of point tile pt: YT(k, na) is zero
+  // past nylm rows (nylm4 of them) and ngrid points
+  T a[8], an[8];
+  auto load_a = [&](T (&v)[8], int pt, int c0) {
+    const T *Ak = YT + (size_t)kq * ldnt + 16 * pt + row;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = Ak[(size_t)4 * ldnt * min(c0 + u, nk - 1)];
+  };
+  const int first = wave + 4 * blockIdx.y;
+  load_a(a, min(first, ntile - 1), 0);
+  const int total = 16 * J * nylm, have = nsp * nylm;
+  const double *Sg = S + (size_t)nylm * i0;
+  for (int k0 = threadIdx.x; k0 < total; k0 += 256 * kStage) {
+    double v[kStage];
+#pragma unroll
+    for (int u = 0; u < kStage; ++u) v[u] = Sg[min(k0 + 256 * u, have - 1)];
+#pragma unroll
+    for (int u = 0; u < kStage; ++u) {
+      const int k = k0 + 256 * u;
+      if (k < total) sS[k] = k < have ? (T)v[u] : T(0);
+    }
+  }
+  __syncthreads();
+  for (int pt = first; pt < ntile; pt += 4 * gridDim.y) {
     const int n0 = pt * 16;
-    const int na = n0 + row;
     vt acc[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[j] = vt{T(0), T(0), T(0), T(0)};
-    // YT(k, na): zero past nylm rows (nylm4 of them) and ngrid points
-    const T *Ak = YT + (size_t)kq * ldnt + na;
-    const int nk = (nylm + 3) / 4;
     for (int c0 = 0; c0 < nk; c0 += 8) {
-      T a[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) a[u] = Ak[(size_t)4 * ldnt * min(c0 + u, nk - 1)];
+      const bool more = c0 + 8 < nk;
+      load_a(an, more ? pt : min(pt + 4 * (int)gridDim.y, ntile - 1), more ? c0 + 8 : 0);
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         if (c0 + u < nk) {
@@ -513,6 +537,8 @@ __global__ __launch_bounds__(256) void k_expand_t(int nylm, int ngrid, int ldnt,
           }
         }
       }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] = an[u];
     }
     // D(i = point, j = sphere) sits in lane j + 16 (i % 4), element i / 4
     // (f64) or lane j + 16 (i / 4), element i % 4 (f32)
