@@ -217,7 +217,7 @@ struct ddx_handle {
   // tables
   ddx::DevArray<double4> grid;    // (x, y, z, w) per Lebedev point
   ddx::DevArray<double> Y, Yw;    // basis (nylm, ngrid) and basis * w
-  ddx::DevArray<float> Y32, Yw32; // their float copies (mixed precision)
+  ddx::DevArray<float> Yw32;      // float copy of Yw (mixed precision)
   bool have_tables32 = false;
   // zero-padded layouts for the products' coalesced operand loads: Yw with
   // lm fastest in columns of ldm = 16 * row tiles over ldnp points (whole

@@ -38,8 +38,8 @@ constexpr int kProjSplit = 4;
 // xi(n, i) = [w_n] sum_lm Y(lm, n) S(lm, i)
 int expand(ddx_handle *h, hipStream_t s, const double *S, double *xi, bool wscale,
            const DiisState *gate);
-// the same two products in FP32 (v_mfma_f32_16x16x4f32, FP32 tables Yw32 /
-// Y32) for the mixed precision: P and xi in float, S and y in double
+// the same two products in FP32 (v_mfma_f32_16x16x4f32, FP32 copies of the
+// tables) for the mixed precision: P and xi in float, S and y in double
 int project32(ddx_handle *h, hipStream_t s, double alpha, const float *P, double *y,
               const DiisState *gate, int ysplit);
 int expand32(ddx_handle *h, hipStream_t s, const double *S, float *xi, bool wscale,

@@ -7,10 +7,10 @@
 //   expansion    xi(n, i) = [w_n] * sum_lm Y(lm, n) S(lm, i)
 //                (matvec.f90:196-204, forces_dd.f90:108-113).
 //
-// Projection: one workgroup per 16 spheres holds all nylm rows (up to 8
-// MFMA row tiles per pass); its four waves split the ngrid reduction and
-// are summed in LDS in a fixed order; each wave loads the operands of four
-// k-steps before issuing their MFMAs, to keep loads in flight.  Expansion:
+// Projection: one workgroup per 16 spheres holds up to 8 MFMA row tiles of the
+// nylm rows (one in small systems); its four waves split the ngrid reduction
+// and are summed in LDS in a fixed order; each wave loads the operands of
+// several k-steps before issuing their MFMAs, to keep loads in flight.  Expansion:
 // one workgroup per 16 J spheres with their S rows staged in LDS
 // (k_expand_t), its point tiles split over blockIdx.y when the sphere
 // tiles alone give too few workgroups.  The Y tables (<= 1.2 MB at lmax 10 / 1202 points) stay
@@ -28,156 +28,88 @@
 namespace ddx {
 namespace {
 
-constexpr int kMaxTiles = 8;   // row tiles of 16 per projection pass
-
-constexpr int kUnroll = 4;   // k-steps whose operands are loaded before their MFMAs
-constexpr int kUnroll32 = 2;   // k-steps in flight in the FP32 projection
-
-__global__ __launch_bounds__(256) void k_project(int nylm, int ngrid, int nsph, double alpha,
-                                                 const double *__restrict__ Yw,
-                                                 const double *__restrict__ P,
-                                                 double *__restrict__ y,
-                                                 const DiisState *__restrict__ gate) {
-  if (gate && gate->done) return;
-  __shared__ v4d red[3][kMaxTiles][kWave];
-  const int lane = lane_id(), wave = threadIdx.x / kWave;
-  // blockIdx.y splits the points into contiguous ranges of whole k-steps
-  // (so that each line of P is read by one workgroup); wave w of the split
-  // takes its k-steps w, w + 4, ... and the split's sum goes to
-  // y + blockIdx.y nylm nsph
-  const int nsteps = (ngrid + 3) / 4;
-  const int per = (nsteps + gridDim.y - 1) / gridDim.y;
-  const int kbeg = 4 * per * blockIdx.y, kend = min(ngrid, 4 * per * (int)(blockIdx.y + 1));
-  y += (size_t)blockIdx.y * nylm * nsph;
-  const int i0 = blockIdx.x * 16;
-  const int col = lane & 15, krow = lane >> 4;
-  const int sph = i0 + col;
-  const int ntile = (nylm + 15) / 16;
-  const double *Pc = P + (size_t)min(sph, nsph - 1) * ngrid;
-  for (int t0 = 0; t0 < ntile; t0 += kMaxTiles) {
-    const int nt = min(kMaxTiles, ntile - t0);
-    v4d acc[kMaxTiles];
-#pragma unroll
-    for (int t = 0; t < kMaxTiles; ++t) acc[t] = v4d{0.0, 0.0, 0.0, 0.0};
-    // k-steps of 4 points each
-    for (int kb = kbeg + 4 * wave; kb < kend; kb += 16 * kUnroll) {
-      double b[kUnroll];
-      double a[kUnroll][kMaxTiles];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int n = kb + 16 * u + krow;
-        const bool okn = n < kend;
-        b[u] = (okn && sph < nsph) ? Pc[n] : 0.0;
-#pragma unroll
-        for (int t = 0; t < kMaxTiles; ++t) {
-          const int m = 16 * (t0 + t) + col;
-          a[u][t] = (t < nt && okn && m < nylm) ? Yw[m + (size_t)nylm * n] : 0.0;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
-#pragma unroll
-        for (int t = 0; t < kMaxTiles; ++t)
-          if (t < nt) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][t], b[u], acc[t], 0, 0, 0);
-    }
-    if (wave > 0) {
-#pragma unroll
-      for (int t = 0; t < kMaxTiles; ++t)
-        if (t < nt) red[wave - 1][t][lane] = acc[t];
-    }
-    __syncthreads();
-    if (wave == 0 && sph < nsph) {
-#pragma unroll
-      for (int t = 0; t < kMaxTiles; ++t) {
-        if (t < nt) {
-          v4d sum = acc[t] + red[0][t][lane];
-          sum = sum + red[1][t][lane];
-          sum = sum + red[2][t][lane];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int m = 16 * (t0 + t) + krow + 4 * q;
-            if (m < nylm) y[m + (size_t)nylm * sph] = alpha * sum[q];
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-}
-
 // FP32 versions for the mixed precision, on v_mfma_f32_16x16x4f32:
 //   A(i, k) in lane i + 16 k, B(k, j) in lane j + 16 k,
 //   D(i, j) in lane j + 16 (i / 4), element i % 4.
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// projection with float tables and point values, FP32 accumulation; the
-// same workgroup shape and point split as k_project, y in double
-// (two k-steps in flight per wave: with four the compiler's schedule takes
-// 361 registers, or spills 832 bytes per lane under a two-workgroup bound)
-__global__ __launch_bounds__(256) void k_project32(int nylm, int ngrid, int nsph, double alpha,
-                                                   const float *__restrict__ Yw,
-                                                   const float *__restrict__ P,
-                                                   double *__restrict__ y,
-                                                   const DiisState *__restrict__ gate) {
+__device__ __forceinline__ v4d mfma4(double a, double b, v4d c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The projection of all but the largest systems, both precisions (T = float:
+// float tables and point values, FP32 accumulation, y in double): a workgroup
+// takes 16 spheres (blockIdx.x), a contiguous range of whole k-steps of the
+// points (blockIdx.y, so that each line of P is read by few workgroups) and NT
+// of the row tiles (blockIdx.z).  Wave w takes the range's k-steps w, w + 4,
+// ..., U of them loaded before their MFMAs; the four waves' sums meet in LDS
+// in a fixed order and go to y + blockIdx.y nylm nsph.  Every row tile's sum
+// is the same whatever NT and U are.
+template <typename T, int NT>
+__global__ __launch_bounds__(256) void k_project(int nylm, int ngrid, int nsph, double alpha,
+                                                 const T *__restrict__ Yw,
+                                                 const T *__restrict__ P,
+                                                 double *__restrict__ y,
+                                                 const DiisState *__restrict__ gate) {
+  typedef T vt __attribute__((ext_vector_type(4)));
+  // k-steps in flight (FP32 with eight tiles: two, four took 361 registers)
+  constexpr int U = NT == 1 ? 8 : sizeof(T) == 8 ? 4 : 2;
   if (gate && gate->done) return;
-  __shared__ v4f red[3][kMaxTiles][kWave];
+  __shared__ vt red[3][NT][kWave];
   const int lane = lane_id(), wave = threadIdx.x / kWave;
   const int nsteps = (ngrid + 3) / 4;
   const int per = (nsteps + gridDim.y - 1) / gridDim.y;
   const int kbeg = 4 * per * blockIdx.y, kend = min(ngrid, 4 * per * (int)(blockIdx.y + 1));
   y += (size_t)blockIdx.y * nylm * nsph;
-  const int i0 = blockIdx.x * 16;
   const int col = lane & 15, krow = lane >> 4;
-  const int sph = i0 + col;
-  const int ntile = (nylm + 15) / 16;
-  const float *Pc = P + (size_t)min(sph, nsph - 1) * ngrid;
-  for (int t0 = 0; t0 < ntile; t0 += kMaxTiles) {
-    const int nt = min(kMaxTiles, ntile - t0);
-    v4f acc[kMaxTiles];
+  const int sph = blockIdx.x * 16 + col;
+  const int t0 = blockIdx.z * NT, nt = min(NT, (nylm + 15) / 16 - t0);
+  const T *Pc = P + (size_t)min(sph, nsph - 1) * ngrid;
+  vt acc[NT];
 #pragma unroll
-    for (int t = 0; t < kMaxTiles; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int kb = kbeg + 4 * wave; kb < kend; kb += 16 * kUnroll32) {
-      float b[kUnroll32];
-      float a[kUnroll32][kMaxTiles];
+  for (int t = 0; t < NT; ++t) acc[t] = vt{T(0), T(0), T(0), T(0)};
+  for (int kb = kbeg + 4 * wave; kb < kend; kb += 16 * U) {
+    T b[U];
+    T a[U][NT];
 #pragma unroll
-      for (int u = 0; u < kUnroll32; ++u) {
-        const int n = kb + 16 * u + krow;
-        const bool okn = n < kend;
-        b[u] = (okn && sph < nsph) ? Pc[n] : 0.f;
+    for (int u = 0; u < U; ++u) {
+      const int n = kb + 16 * u + krow;
+      const bool okn = n < kend;
+      b[u] = (okn && sph < nsph) ? Pc[n] : T(0);
 #pragma unroll
-        for (int t = 0; t < kMaxTiles; ++t) {
-          const int m = 16 * (t0 + t) + col;
-          a[u][t] = (t < nt && okn && m < nylm) ? Yw[m + (size_t)nylm * n] : 0.f;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kUnroll32; ++u)
-#pragma unroll
-        for (int t = 0; t < kMaxTiles; ++t)
-          if (t < nt) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][t], b[u], acc[t], 0, 0, 0);
-    }
-    if (wave > 0) {
-#pragma unroll
-      for (int t = 0; t < kMaxTiles; ++t)
-        if (t < nt) red[wave - 1][t][lane] = acc[t];
-    }
-    __syncthreads();
-    if (wave == 0 && sph < nsph) {
-#pragma unroll
-      for (int t = 0; t < kMaxTiles; ++t) {
-        if (t < nt) {
-          v4f sum = acc[t] + red[0][t][lane];
-          sum = sum + red[1][t][lane];
-          sum = sum + red[2][t][lane];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int m = 16 * (t0 + t) + 4 * krow + q;
-            if (m < nylm) y[m + (size_t)nylm * sph] = alpha * (double)sum[q];
-          }
-        }
+      for (int t = 0; t < NT; ++t) {
+        const int m = 16 * (t0 + t) + col;
+        a[u][t] = (t < nt && okn && m < nylm) ? Yw[m + (size_t)nylm * n] : T(0);
       }
     }
-    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (t < nt) acc[t] = mfma4(a[u][t], b[u], acc[t]);
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      if (t < nt) red[wave - 1][t][lane] = acc[t];
+  }
+  __syncthreads();
+  if (wave > 0 || sph >= nsph) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (t < nt) {
+      vt sum = acc[t] + red[0][t][lane];
+      sum = sum + red[1][t][lane];
+      sum = sum + red[2][t][lane];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int m = 16 * (t0 + t) + (sizeof(T) == 8 ? krow + 4 * q : 4 * krow + q);
+        if (m < nylm) y[m + (size_t)nylm * sph] = alpha * (double)sum[q];
+      }
+    }
   }
 }
 
@@ -566,10 +498,15 @@ __global__ __launch_bounds__(256) void k_expand_t(int nylm, int ngrid, int ldnt,
   }
 }
 
-// sphere tiles per expansion workgroup: LDS for S and the transposes
+// sphere tiles per expansion workgroup: two where LDS holds the rows of S and
+// that still makes a workgroup per compute unit; below, one, whose MFMA chain
+// and staging are half as long (two -> one: 6.6 -> 5.6 us at 60 atoms, 9.9 ->
+// 8.5 us at 200 atoms and lmax 10, 10.0 -> 9.9 us at 1000; 13.5 -> 13.8 us at 2000)
 template <typename T>
-int expand_tiles(int nylm) {
-  return nylm * 16 * 2 * (int)sizeof(T) <= 48 * 1024 ? 2 : 1;
+int expand_tiles(const ddx_handle *h) {
+  const int split = ((h->ngrid + 15) / 16 + 3) / 4;   // at most (expand_split)
+  return h->nylm * 16 * 2 * (int)sizeof(T) <= 48 * 1024 && (h->n + 31) / 32 * split >= h->ncu
+             ? 2 : 1;
 }
 template <typename T>
 size_t expand_lds(int nylm, int J) {
@@ -632,10 +569,7 @@ int make_ptables(ddx_handle *h) {
 int make_tables32(ddx_handle *h) {
   if (h->have_tables32) return DDX_OK;
   const size_t n = (size_t)h->nylm * h->ngrid;
-  DDX_TRY(h->Y32.reserve(n));
   DDX_TRY(h->Yw32.reserve(n));
-  hipLaunchKernelGGL(k_to_f32, dim3((n + 255) / 256), dim3(256), 0, h->stream, n, h->Y.p,
-                     h->Y32.p);
   hipLaunchKernelGGL(k_to_f32, dim3((n + 255) / 256), dim3(256), 0, h->stream, n, h->Yw.p,
                      h->Yw32.p);
   DDX_HIP(hipGetLastError());
@@ -681,6 +615,35 @@ void launch_pg(ddx_handle *h, hipStream_t s, double alpha, const float *rw, doub
                         rw, y, gate, h->ninst > 1 ? h->inst.p : nullptr, h->ninst);
 }
 
+namespace {
+// k_project with all row tiles in a workgroup (up to eight a pass), or with one
+// where the workgroups that makes stay within four per compute unit.  A wave
+// issues an FP64 MFMA every 64 cycles, so that in a small system eight tiles of
+// 19 k-steps are a chain of 4 us in a few waves while most of the chip idles;
+// but every tile's workgroup reads P again, 16 lines an instruction, which
+// bounds larger systems.  Eight tiles -> one: 6.1 -> 3.6 us at 60 atoms (64
+// workgroups), 9.5 -> 5.9 us at 300 atoms and lmax 8 (456), 15.9 -> 8.2 us at
+// 200 atoms and lmax 10 (416); 9.4 -> 10.4 us at 1000 atoms and lmax 8 (1512).
+template <typename T, int NT>
+void launch_project_nt(ddx_handle *h, hipStream_t s, double alpha, const T *Yw, const T *P,
+                       double *y, const DiisState *gate, int ysplit, hipEvent_t b, hipEvent_t e) {
+  const int ntile = (h->nylm + 15) / 16;
+  hipExtLaunchKernelGGL((k_project<T, NT>),
+                        dim3((h->n + 15) / 16, ysplit, (ntile + NT - 1) / NT), dim3(256), 0, s, b,
+                        e, 0, h->nylm, h->ngrid, h->n, alpha, Yw, P, y, gate);
+}
+
+template <typename T>
+void launch_project(ddx_handle *h, hipStream_t s, double alpha, const T *Yw, const T *P,
+                    double *y, const DiisState *gate, int ysplit, hipEvent_t b, hipEvent_t e) {
+  const long long groups = (long long)((h->n + 15) / 16) * ysplit * ((h->nylm + 15) / 16);
+  if (groups <= 4 * h->ncu)
+    launch_project_nt<T, 1>(h, s, alpha, Yw, P, y, gate, ysplit, b, e);
+  else
+    launch_project_nt<T, 8>(h, s, alpha, Yw, P, y, gate, ysplit, b, e);
+}
+}  // namespace
+
 int project32_gathered(ddx_handle *h, hipStream_t s, double alpha, const float *rw, double *y,
                        const DiisState *gate, int ysplit, bool *done) {
   *done = false;
@@ -710,8 +673,7 @@ int project32(ddx_handle *h, hipStream_t s, double alpha, const float *P, double
     DDX_HIP(hipGetLastError());
     return DDX_OK;
   }
-  hipExtLaunchKernelGGL(k_project32, dim3((h->n + 15) / 16, ysplit), dim3(256), 0, s, tl.b, tl.e,
-                        0, h->nylm, h->ngrid, h->n, alpha, h->Yw32.p, P, y, gate);
+  launch_project<float>(h, s, alpha, h->Yw32.p, P, y, gate, ysplit, tl.b, tl.e);
   DDX_HIP(hipGetLastError());
   return DDX_OK;
 }
@@ -719,7 +681,7 @@ int project32(ddx_handle *h, hipStream_t s, double alpha, const float *P, double
 int expand32(ddx_handle *h, hipStream_t s, const double *S, float *xi, bool wscale,
              const DiisState *gate) {
   if (h->n <= 0) return DDX_OK;
-  const int J = expand_tiles<float>(h->nylm);
+  const int J = expand_tiles<float>(h);
   const size_t lds = expand_lds<float>(h->nylm, J);
   TimedLaunch tl(h, DDX_K_EXPAND, s);
   const int nx = (h->n + 16 * J - 1) / (16 * J);
@@ -739,8 +701,7 @@ int project(ddx_handle *h, hipStream_t s, double alpha, const double *P, double 
     DDX_HIP(hipGetLastError());
     return DDX_OK;
   }
-  hipExtLaunchKernelGGL(k_project, dim3((h->n + 15) / 16, ysplit), dim3(256), 0, s, tl.b, tl.e, 0,
-                        h->nylm, h->ngrid, h->n, alpha, h->Yw.p, P, y, gate);
+  launch_project<double>(h, s, alpha, h->Yw.p, P, y, gate, ysplit, tl.b, tl.e);
   DDX_HIP(hipGetLastError());
   return DDX_OK;
 }
@@ -748,7 +709,7 @@ int project(ddx_handle *h, hipStream_t s, double alpha, const double *P, double 
 int expand(ddx_handle *h, hipStream_t s, const double *S, double *xi, bool wscale,
            const DiisState *gate) {
   if (h->n <= 0) return DDX_OK;
-  const int J = expand_tiles<double>(h->nylm);
+  const int J = expand_tiles<double>(h);
   const size_t lds = expand_lds<double>(h->nylm, J);
   TimedLaunch tl(h, DDX_K_EXPAND, s);
   const int nx = (h->n + 16 * J - 1) / (16 * J);
