@@ -233,7 +233,7 @@ int pipeline(ddx_handle *h) {
   if (use_fmm(h))
     DDX_TRY(fmm_potential(h, h->charge.p, h->phi.p, h->igrad ? h->ef.p : nullptr));
   else
-    DDX_TRY(coulomb_potential(h, h->ctile.p, h->nctile, h->charge.p, h->sph.p, h->ccav.p,
+    DDX_TRY(coulomb_potential(h, h->ctile, h->charge.p, h->sph.p, h->ccav.p,
                               h->phi.p, h->igrad ? h->ef.p : nullptr));
   DDX_TRY(make_psi(h, h->charge.p, h->psi.p));
   DDX_TRY(build_rhs(h, h->phi.p, h->rhs.p));
@@ -627,7 +627,7 @@ int ddx_mkrhs(ddx_handle *h, const double *charge, double *phi, double *psi) {
   if (use_fmm(h))
     DDX_TRY(fmm_potential(h, h->charge.p, h->phi.p, nullptr));
   else
-    DDX_TRY(coulomb_potential(h, h->ctile.p, h->nctile, h->charge.p, h->sph.p, h->ccav.p,
+    DDX_TRY(coulomb_potential(h, h->ctile, h->charge.p, h->sph.p, h->ccav.p,
                               h->phi.p, nullptr));
   DDX_TRY(make_psi(h, h->charge.p, h->psi.p));
   DDX_TRY(download(phi, h->phi.p, h->ncav, h->stream));
@@ -649,17 +649,14 @@ int ddx_mkrhs_at(ddx_handle *h, int n, const double *charge, const double *x, co
   for (int i = 0; i < n; ++i) src[i] = make_double4(x[i], y[i], z[i], 0.0);
   DevArray<double4> dsrc;
   DevArray<double> dq, dtrg, dphi, dpsi;
-  DevArray<int4> dtile;
-  std::vector<int4> tiles;
-  std::vector<int> grp;
-  coulomb_tiles({0, ncav}, {0, n}, false, tiles, grp);
+  TileTable dtile;
+  DDX_TRY(potential_tiles(h, dtile, n, ncav));
   DDX_TRY(upload(dsrc, src.data(), n, s));
   DDX_TRY(upload(dq, charge, n, s));
   DDX_TRY(upload(dtrg, ccav, 3 * (size_t)ncav, s));
-  DDX_TRY(upload(dtile, tiles.data(), tiles.size(), s));
   DDX_TRY(dphi.reserve((size_t)ncav + 1));
   DDX_TRY(dpsi.reserve((size_t)nylm * n));
-  DDX_TRY(coulomb_potential(h, dtile.p, (int)tiles.size(), dq.p, dsrc.p, dtrg.p, dphi.p, nullptr));
+  DDX_TRY(coulomb_potential(h, dtile, dq.p, dsrc.p, dtrg.p, dphi.p, nullptr));
   DDX_TRY(make_psi_n(h, n, nylm, dq.p, dpsi.p));
   DDX_TRY(download(phi, dphi.p, ncav, s));
   DDX_TRY(download(psi, dpsi.p, (size_t)nylm * n, s));

@@ -141,6 +141,16 @@ struct FmmState {
   DevArray<int> perm;                   // the spheres in Morton order of their centres
 };
 
+// Tiles of the all-pairs Coulomb kernels (k_coulomb.hip): per workgroup a
+// range of targets and of sources of one instance; with the sources in chunks
+// also the first tile of each target tile (grp).
+struct TileTable {
+  DevArray<int4> tiles, info;
+  DevArray<int> grp;
+  std::vector<int4> rows;       // the instances' rows behind info
+  int ntile = 0, ngrp = 0;
+};
+
 // Event pairs around the launches of one kernel class (ddx_kernel_timer).
 // A launch made for a Jacobi/DIIS solve carries the solve's serial number
 // and round, so that rounds enqueued after convergence can be dropped.
@@ -267,17 +277,13 @@ struct ddx_handle {
   // block maps of the solver kernels: each workgroup of k_jacobi works on
   // a range of one instance's elements (jblk: instance, begin, end), each of
   // k_extrap on a range of its spheres (eblk); jboff / eboff: the blocks of
-  // each instance.  Coulomb tiles: per workgroup a range of <= 256 targets
-  // and of sources of one instance (ctile), and for the field at the
-  // nuclei the source chunks of each target tile (ftile, fgrp: tiles of
-  // each target group).
-  int nbj = 0, nbe = 0, nctile = 0, nftile = 0, nfgrp = 0;
-  ddx::DevArray<int4> jblk, eblk, ctile, ftile;
-  ddx::DevArray<int> jboff, eboff, fgrp, soff, cavoff;
-  ddx::DevArray<int4> xtile;      // tiles of a field between arbitrary point sets
-  ddx::DevArray<int> xgrp;
-  std::vector<int4> h_ctile, h_ftile, h_xtile;   // host copies of the tile tables
-  std::vector<int> h_fgrp, h_xgrp;
+  // each instance.  Coulomb tiles: the potential at the cavity points
+  // (ctile) and the field of the cavity charges at the nuclei (ftile).
+  int nbj = 0, nbe = 0;
+  ddx::DevArray<int4> jblk, eblk;
+  ddx::DevArray<int> jboff, eboff, soff, cavoff;
+  ddx::TileTable ctile, ftile;
+  ddx::TileTable xtile;           // of a field between arbitrary point sets
   int maps_n = -1;                // sphere count the block maps were built for
   int most = 0;                   // spheres of the largest instance
   bool mute_timers = false;       // launches outside the timed classes' meaning

@@ -109,18 +109,18 @@ int energy_dot(ddx_handle *h, const double *a, const double *b, double scale,
                double *d_out);
 
 // k_coulomb.hip — all-pairs potential and field (mkrhs.f90, efld.f90) on
-// tile tables (targets tb..te-1, sources sb..se-1 per workgroup)
-void coulomb_tiles(const std::vector<int> &toff, const std::vector<int> &soff, bool split,
-                   std::vector<int4> &tiles, std::vector<int> &grp);
-// h->ctile (cavity points from the spheres) and h->ftile / h->fgrp (the
-// nuclei from the cavity points), per instance
+// tile tables (targets tb..te-1, sources sb..se-1 per workgroup), which are
+// made on the device
+int potential_tiles(ddx_handle *h, TileTable &t, int nsrc, int ntrg);
+// h->ctile (cavity points from the spheres) and h->ftile (the nuclei from the
+// cavity points), per instance
 int build_coulomb_tiles(ddx_handle *h);
 // phi; with ef != NULL also the field ef(3, .) of the same sources
-int coulomb_potential(ddx_handle *h, const int4 *tiles, int ntile, const double *q,
-                      const double4 *src, const double *trg3, double *phi, double *ef);
+int coulomb_potential(ddx_handle *h, const TileTable &t, const double *q, const double4 *src,
+                      const double *trg3, double *phi, double *ef);
 // ef(3, .) from per-chunk partials summed per target group
-int coulomb_field(ddx_handle *h, const int4 *tiles, int ntile, const int *grp, int ngrp,
-                  const double *q, const double *src3, const double *trg3, double *ef);
+int coulomb_field(ddx_handle *h, const TileTable &t, const double *q, const double *src3,
+                  const double *trg3, double *ef);
 int coulomb_field_points(ddx_handle *h, int nsrc, const double *q, const double *src3, int ntrg,
                          const double *trg3, double *ef);
 int make_psi(ddx_handle *h, const double *charge, double *psi);

@@ -1,11 +1,10 @@
 // All-pairs Coulomb sums for point-charge solutes.
 //   potential  phi(j) = sum_i q_i / |r_j - r_i|            (mkrhs.f90:102-114)
 //   field      E(j)   = sum_i q_i (r_j - r_i) / |r_j - r_i|^3  (efld.f90:98-114)
-// Each thread owns one or two targets; sources stream through LDS.  Work
-// comes as a table of tiles (targets tb..te-1, at most 512 for the potential
-// and 64 for the tiled field, and sources sb..se-1): for a batch of molecules
-// every tile stays inside one molecule, so each sums only its own molecule's
-// charges.
+// Each lane owns one target; sources stream through LDS.  Work comes as a
+// table of tiles (targets tb..te-1, at most 64, and sources sb..se-1): for a
+// batch of molecules every tile stays inside one molecule, so each sums only
+// its own molecule's charges.
 // The potential kernel can return the field of the same sources as well
 // (the solute field at the cavity points that the forces contract with
 // zeta), which costs one all-pairs pass less than a separate field kernel.
@@ -26,8 +25,8 @@ namespace ddx {
 namespace {
 
 constexpr int kCT = 256;          // threads per workgroup, sources per LDS tile
-constexpr int kTW = 2 * kCT;      // targets per tile: two per thread
-constexpr int kFW = kWave;        // targets per tile of the tiled field: one per lane
+constexpr int kTW = 2 * kCT;      // targets per tile of the uniform tiling: two per thread
+constexpr int kFW = kWave;        // targets per tile of the table-driven kernels: one per lane
 
 // 1/sqrt(x) for x > 0: v_rsq_f64 (relative error below 2^-24 on gfx950)
 // and one third-order correction: with e = 1 - x y^2, y (1 + e/2 + 3e^2/8)
@@ -39,82 +38,67 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
 }
 
 // phi(j) and, with FIELD, the field ef(:, j) of the same sources, from one
-// evaluation of 1/r per pair; tile (tb, te, sb, se) per workgroup, targets
-// tb + t and tb + t + kCT in thread t (each source read from LDS serves two)
+// evaluation of 1/r per pair; one wave per tile (tb, te, sb, se) of at most
+// kFW targets, one per lane, the sources through LDS kFW at a time and added
+// in order.
+//   Bound by FP64 issue: 18 operations and one v_rsq_f64 a pair, four pairs in
+// flight (a bound of 6 or 8 waves per SIMD costs the unrolled loop its
+// registers: 610 and 698 us against 601 at 2000 atoms).  One-wave workgroups of
+// 64 targets spread over the chip whatever their number; with 512 targets to a
+// workgroup of four waves (two per thread) 642 atoms made 61 workgroups.  That
+// form -> this one, in us (lmax, grid): 60 atoms (6, 302) 9.5 -> 5.9; 259 (6,
+// 110) 30 -> 17; 642 (6, 110) 71 -> 39; 200 (10, 1202) 27.5 -> 24.0; 1000 (8,
+// 590) 202 -> 195; 2000 (8, 590) 614 -> 601.  Two targets per lane in one wave:
+// 70 us at 642 atoms, 755 at 2000.
 template <bool FIELD>
-__global__ __launch_bounds__(kCT) void k_potential(const int4 *__restrict__ tiles,
+__global__ __launch_bounds__(kFW) void k_potential(const int4 *__restrict__ tiles,
                                                    const double *__restrict__ q,
                                                    const double4 *__restrict__ src,
                                                    const double *__restrict__ trg,
                                                    double *__restrict__ phi,
                                                    double *__restrict__ ef) {
-  __shared__ double4 tile[kCT];
+  __shared__ double4 tile[kFW];
   const int4 tl = tiles[blockIdx.x];
-  const int j0 = tl.x + threadIdx.x, j1 = j0 + kCT;
-  double ax = 0.0, ay = 0.0, az = 0.0, bx = 0.0, by = 0.0, bz = 0.0;
-  if (j0 < tl.y) {
-    ax = trg[3 * (size_t)j0];
-    ay = trg[3 * (size_t)j0 + 1];
-    az = trg[3 * (size_t)j0 + 2];
+  const int j = tl.x + (int)threadIdx.x, jc = min(j, tl.y - 1);
+  const double ax = trg[3 * (size_t)jc], ay = trg[3 * (size_t)jc + 1],
+               az = trg[3 * (size_t)jc + 2];
+  double va = 0.0, e0 = 0.0, e1 = 0.0, e2 = 0.0;
+  int i = min(tl.z + (int)threadIdx.x, tl.w - 1);
+  double4 s = make_double4(0.0, 0.0, 0.0, 0.0);
+  double qi = 0.0;
+  if (tl.z < tl.w) {
+    s = src[i];
+    qi = q[i];
   }
-  if (j1 < tl.y) {
-    bx = trg[3 * (size_t)j1];
-    by = trg[3 * (size_t)j1 + 1];
-    bz = trg[3 * (size_t)j1 + 2];
-  }
-  double va = 0.0, ea0 = 0.0, ea1 = 0.0, ea2 = 0.0;
-  double vb = 0.0, eb0 = 0.0, eb1 = 0.0, eb2 = 0.0;
-  for (int i0 = tl.z; i0 < tl.w; i0 += kCT) {
-    int i = i0 + threadIdx.x;
-    if (i < tl.w) {
-      double4 s = src[i];
-      tile[threadIdx.x] = make_double4(s.x, s.y, s.z, q[i]);
-    }
-    __syncthreads();
-    int cnt = min(kCT, tl.w - i0);
+  for (int i0 = tl.z; i0 < tl.w; i0 += kFW) {
+    wave_lds_sync();   // the previous sources are read
+    tile[threadIdx.x] = make_double4(s.x, s.y, s.z, qi);
+    wave_lds_sync();
+    i = min(i + kFW, tl.w - 1);   // the next sources, loaded under this block's sums
+    s = src[i];
+    qi = q[i];
+    const int cnt = min(kFW, tl.w - i0);
+#pragma unroll 4
     for (int k = 0; k < cnt; ++k) {
-      const double4 s = tile[k];
-      {
-        const double dx = ax - s.x, dy = ay - s.y, dz = az - s.z;
-        const double y = rsqrt_nr(dx * dx + dy * dy + dz * dz);
-        const double qy = s.w * y;
-        va = va + qy;
-        if (FIELD) {
-          const double f = qy * (y * y);
-          ea0 = ea0 + f * dx;
-          ea1 = ea1 + f * dy;
-          ea2 = ea2 + f * dz;
-        }
-      }
-      {
-        const double dx = bx - s.x, dy = by - s.y, dz = bz - s.z;
-        const double y = rsqrt_nr(dx * dx + dy * dy + dz * dz);
-        const double qy = s.w * y;
-        vb = vb + qy;
-        if (FIELD) {
-          const double f = qy * (y * y);
-          eb0 = eb0 + f * dx;
-          eb1 = eb1 + f * dy;
-          eb2 = eb2 + f * dz;
-        }
+      const double4 sk = tile[k];
+      const double dx = ax - sk.x, dy = ay - sk.y, dz = az - sk.z;
+      const double y = rsqrt_nr(dx * dx + dy * dy + dz * dz);
+      const double qy = sk.w * y;
+      va = va + qy;
+      if (FIELD) {
+        const double f = qy * (y * y);
+        e0 = e0 + f * dx;
+        e1 = e1 + f * dy;
+        e2 = e2 + f * dz;
       }
     }
-    __syncthreads();
   }
-  if (j0 < tl.y) {
-    phi[j0] = va;
+  if (j < tl.y) {
+    phi[j] = va;
     if (FIELD) {
-      ef[3 * (size_t)j0] = ea0;
-      ef[3 * (size_t)j0 + 1] = ea1;
-      ef[3 * (size_t)j0 + 2] = ea2;
-    }
-  }
-  if (j1 < tl.y) {
-    phi[j1] = vb;
-    if (FIELD) {
-      ef[3 * (size_t)j1] = eb0;
-      ef[3 * (size_t)j1 + 1] = eb1;
-      ef[3 * (size_t)j1 + 2] = eb2;
+      ef[3 * (size_t)j] = e0;
+      ef[3 * (size_t)j + 1] = e1;
+      ef[3 * (size_t)j + 2] = e2;
     }
   }
 }
@@ -257,40 +241,50 @@ __global__ __launch_bounds__(kFW) void k_field_w(const int4 *__restrict__ tiles,
 }
 
 // ef of the targets of group g = the partials of its tiles grp[g] ..
-// grp[g+1]-1 (the source chunks of one target tile) in a fixed order: each
-// target's chunks are split over kRw threads (chunk c to thread c mod kRw),
-// whose sums meet in LDS in thread order.
+// grp[g+1]-1 (the source chunks of one target tile) in a fixed order: the
+// chunks are split over kRw waves (chunk c to wave c mod kRw), lane t of each
+// adding target t's, eight tiles loaded before they are added, and the waves'
+// sums meet in LDS in wave order.  A tile's partials are one contiguous run of
+// a wave's loads (with the lanes across the chunks they were 64 lines): 128 -> 44
+// us at 2000 atoms (lmax 8, 590 points), 65 -> 27 at 1000.
 constexpr int kRw = 4;
 __global__ __launch_bounds__(kFW * kRw) void k_field_reduce_w(const int *__restrict__ grp,
                                                               const int4 *__restrict__ tiles,
                                                               const double *__restrict__ part,
                                                               double *__restrict__ ef) {
-  __shared__ double red[kFW * kRw][3];
+  __shared__ double red[kRw][3][kFW];
   const int b0 = grp[blockIdx.x], b1 = grp[blockIdx.x + 1];
   const int4 tl = tiles[b0];
-  const int r = threadIdx.x % kRw, t = threadIdx.x / kRw;
+  const int t = threadIdx.x % kFW, r = threadIdx.x / kFW;
   double e0 = 0.0, e1 = 0.0, e2 = 0.0;
-  for (int b = b0 + r; b < b1; b += kRw) {
-    const size_t o = ((size_t)b * kFW + t) * 3;
-    e0 += part[o];
-    e1 += part[o + 1];
-    e2 += part[o + 2];
+  for (int b = b0 + r; b < b1; b += 8 * kRw) {
+    double v[8][3];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const size_t o = ((size_t)min(b + u * kRw, b1 - 1) * kFW + t) * 3;
+      v[u][0] = part[o];
+      v[u][1] = part[o + 1];
+      v[u][2] = part[o + 2];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (b + u * kRw < b1) {
+        e0 += v[u][0];
+        e1 += v[u][1];
+        e2 += v[u][2];
+      }
+    }
   }
-  red[threadIdx.x][0] = e0;
-  red[threadIdx.x][1] = e1;
-  red[threadIdx.x][2] = e2;
+  red[r][0][t] = e0;
+  red[r][1][t] = e1;
+  red[r][2][t] = e2;
   __syncthreads();
   const int j = tl.x + t;
-  if (r == 0 && j < tl.y) {
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int k = 0; k < kRw; ++k) {
-      s0 += red[threadIdx.x + k][0];
-      s1 += red[threadIdx.x + k][1];
-      s2 += red[threadIdx.x + k][2];
-    }
-    ef[3 * (size_t)j] = s0;
-    ef[3 * (size_t)j + 1] = s1;
-    ef[3 * (size_t)j + 2] = s2;
+  if (r < 3 && j < tl.y) {   // wave r: component r
+    double sum = 0.0;
+#pragma unroll
+    for (int k = 0; k < kRw; ++k) sum += red[k][r][t];
+    ef[3 * (size_t)j + r] = sum;
   }
 }
 
@@ -353,131 +347,127 @@ __global__ void k_psi(int n, int nylm, double fac, const double *__restrict__ q,
   psi[k] = (k % nylm == 0) ? fac * q[k / nylm] : 0.0;
 }
 
-// The tile tables of one system (what coulomb_tiles builds for one instance):
-// potential tiles of kTW cavity points, and nfg groups of nfc field tiles, kFW
-// nuclei by `chunk` cavity points each.
-__global__ void k_single_tiles(int n, int ncav, int nct, int nfg, int nfc, int chunk,
-                               int4 *__restrict__ ctile, int4 *__restrict__ ftile,
-                               int *__restrict__ fgrp) {
+// A tile table: tiles of kFW targets, per instance; `info` holds each
+// instance's first target, first source, first tile and first target tile
+// (and the ends after the last instance; for one instance the two rows come
+// with the launch).  With a chunk length the sources of each target tile are
+// cut into chunks, one tile each, and grp receives the first tile of each
+// target tile.
+struct TileRows {
+  int4 a, b;
+};
+__global__ void k_make_tiles(int ninst, int ntile, long long chunk, TileRows one,
+                             const int4 *__restrict__ info, int4 *__restrict__ tiles,
+                             int *__restrict__ grp) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < nct) ctile[b] = make_int4(b * kTW, min(b * kTW + kTW, ncav), 0, n);
-  if (b < nfg * nfc) {
-    const int g = b / nfc, c = b - g * nfc;
-    const long long sb = (long long)c * chunk;
-    ftile[b] = make_int4(g * kFW, min(g * kFW + kFW, n), (int)sb,
-                         (int)min(sb + chunk, (long long)ncav));
+  if (b > ntile) return;
+  if (b == ntile) {
+    if (grp) grp[ninst > 1 ? info[ninst].w : one.b.w] = ntile;
+    return;
   }
-  if (b <= nfg) fgrp[b] = b * nfc;
+  int4 lo = one.a, hi = one.b;
+  if (ninst > 1) {
+    int l = 0, h = ninst;   // info[l].z <= b < info[h].z
+    while (h - l > 1) {
+      const int m = (l + h) >> 1;
+      if (info[m].z <= b) l = m;
+      else h = m;
+    }
+    lo = info[l];
+    hi = info[l + 1];
+  }
+  const int ntt = hi.w - lo.w, nch = (hi.z - lo.z) / ntt;
+  const int tt = (b - lo.z) / nch, c = (b - lo.z) - tt * nch;
+  const int tb = lo.x + tt * kFW;
+  const long long sb = lo.y + c * chunk;
+  tiles[b] = make_int4(tb, min(tb + kFW, hi.x), (int)sb, (int)min(sb + chunk, (long long)hi.y));
+  if (grp && c == 0) grp[lo.w + tt] = b;
 }
 
 // sources per field tile: about 32768 one-wave tiles (several rounds of the
 // resident waves, so that the uneven last chunks of each target tile do not
 // leave CUs idle), whole multiples of kFW and at least 4 kFW; work = target
 // tiles x sources
+constexpr long long kFieldTiles = 32768;
 long long field_chunk(long long work) {
-  long long chunk = (work + 32767) / 32768;
+  long long chunk = (work + kFieldTiles - 1) / kFieldTiles;
   chunk = ((chunk + kFW - 1) / kFW) * kFW;
   return std::max<long long>(chunk, 4 * kFW);
 }
 
-}  // namespace
-
-// Tiles of kTW targets, per instance q: targets toff[q] .. toff[q+1]-1,
-// sources soff[q] .. soff[q+1]-1.  With `split`, the sources of each target
-// tile are cut into chunks (multiples of kCT, at least 4 kCT) so that there
-// are about 1024 tiles in all; grp then holds the first tile of each target
-// tile's chunks.
-void coulomb_tiles(const std::vector<int> &toff, const std::vector<int> &soff, bool split,
-                   std::vector<int4> &tiles, std::vector<int> &grp) {
-  // split: the tiled field, kFW targets per tile (one wave) and the sources
-  // cut into chunks; otherwise kTW targets and all of the molecule's sources
-  const int tw = split ? kFW : kTW;
-  const size_t ninst = toff.size() - 1;
+// targets toff[q] .. toff[q+1]-1 and sources soff[q] .. soff[q+1]-1 of ninst
+// instances; split: the sources in chunks, with the groups.  The rows of
+// several instances stay in t's host vector until its next use.
+int make_tiles(ddx_handle *h, TileTable &t, int ninst, const int *toff, const int *soff,
+               bool split) {
   long long work = 0;   // target tiles x sources
-  for (size_t q = 0; q < ninst; ++q)
-    work += (long long)((toff[q + 1] - toff[q] + tw - 1) / tw) * (soff[q + 1] - soff[q]);
-  long long chunk = 0x7fffffff;
-  if (split) chunk = field_chunk(work);
-  tiles.clear();
-  grp.clear();
-  for (size_t q = 0; q < ninst; ++q) {
-    const int sb = soff[q], se = soff[q + 1];
-    for (int tb = toff[q]; tb < toff[q + 1]; tb += tw) {
-      const int te = std::min(tb + tw, toff[q + 1]);
-      grp.push_back((int)tiles.size());
-      if (se <= sb) {
-        tiles.push_back(make_int4(tb, te, sb, sb));
-        continue;
-      }
-      for (long long c = sb; c < se; c += chunk)
-        tiles.push_back(make_int4(tb, te, (int)c, (int)std::min<long long>(c + chunk, se)));
-    }
+  for (int q = 0; q < ninst; ++q)
+    work += (long long)((toff[q + 1] - toff[q] + kFW - 1) / kFW) * (soff[q + 1] - soff[q]);
+  const long long chunk = split ? field_chunk(work) : 0x7fffffff;
+  t.rows.resize(ninst + 1);
+  long long nt = 0, ng = 0;
+  for (int q = 0; q <= ninst; ++q) {
+    t.rows[q] = make_int4(toff[q], soff[q], (int)nt, (int)ng);
+    if (q == ninst) break;
+    const long long ntt = (toff[q + 1] - toff[q] + kFW - 1) / kFW;
+    const long long nch = std::max<long long>(1, (soff[q + 1] - soff[q] + chunk - 1) / chunk);
+    nt += ntt * nch;
+    ng += ntt;
   }
-  grp.push_back((int)tiles.size());
-}
-
-namespace {
-int upload_tiles(ddx_handle *h, DevArray<int4> &dt, const std::vector<int4> &t) {
-  DDX_TRY(dt.reserve(t.size() + 1));
-  if (!t.empty())
-    DDX_HIP(hipMemcpyAsync(dt.p, t.data(), t.size() * sizeof(int4), hipMemcpyHostToDevice,
-                           h->stream));
-  return DDX_OK;
-}
-}  // namespace
-
-int build_coulomb_tiles(ddx_handle *h) {
-  if (h->ninst == 1) {
-    const int nfg = (h->n + kFW - 1) / kFW;
-    const long long chunk = field_chunk((long long)nfg * h->ncav);
-    const int nfc = std::max<int>(1, (int)((h->ncav + chunk - 1) / chunk));
-    h->nctile = (h->ncav + kTW - 1) / kTW;
-    h->nftile = nfg * nfc;
-    h->nfgrp = nfg;
-    DDX_TRY(h->ctile.reserve((size_t)h->nctile + 1));
-    DDX_TRY(h->ftile.reserve((size_t)h->nftile + 1));
-    DDX_TRY(h->fgrp.reserve((size_t)nfg + 1));
-    const int most = std::max(std::max(h->nctile, h->nftile), nfg + 1);
-    hipLaunchKernelGGL(k_single_tiles, dim3((most + 255) / 256), dim3(256), 0, h->stream, h->n,
-                       h->ncav, h->nctile, nfg, nfc, (int)chunk, h->ctile.p, h->ftile.p,
-                       h->fgrp.p);
-    DDX_HIP(hipGetLastError());
-    return DDX_OK;
+  if (nt > 0x7ffffffell) {
+    set_error("%lld Coulomb tiles exceed the 32-bit index", nt);
+    return DDX_ERR_CAPACITY;
   }
-  // the host tables live in the handle until the next setup, so the copies
-  // need no wait here
-  std::vector<int> g;
-  // potential (and solute field) at the cavity points from the spheres
-  coulomb_tiles(h->h_cavoff, h->h_soff, false, h->h_ctile, g);
-  h->nctile = (int)h->h_ctile.size();
-  DDX_TRY(upload_tiles(h, h->ctile, h->h_ctile));
-  // field of the cavity charges at the nuclei
-  coulomb_tiles(h->h_soff, h->h_cavoff, true, h->h_ftile, h->h_fgrp);
-  h->nftile = (int)h->h_ftile.size();
-  h->nfgrp = (int)h->h_fgrp.size() - 1;
-  DDX_TRY(upload_tiles(h, h->ftile, h->h_ftile));
-  DDX_TRY(h->fgrp.reserve(h->h_fgrp.size()));
-  DDX_HIP(hipMemcpyAsync(h->fgrp.p, h->h_fgrp.data(), h->h_fgrp.size() * sizeof(int),
-                         hipMemcpyHostToDevice, h->stream));
-  return DDX_OK;
-}
-
-int coulomb_potential(ddx_handle *h, const int4 *tiles, int ntile, const double *q,
-                      const double4 *src, const double *trg3, double *phi, double *ef) {
-  if (ntile <= 0) return DDX_OK;
-  TimedLaunch tl(h, DDX_K_POTENTIAL, h->stream);
-  if (ef)
-    hipExtLaunchKernelGGL(k_potential<true>, dim3(ntile), dim3(kCT), 0, h->stream, tl.b, tl.e, 0,
-                          tiles, q, src, trg3, phi, ef);
-  else
-    hipExtLaunchKernelGGL(k_potential<false>, dim3(ntile), dim3(kCT), 0, h->stream, tl.b, tl.e,
-                          0, tiles, q, src, trg3, phi, nullptr);
+  t.ntile = (int)nt;
+  t.ngrp = (int)ng;
+  DDX_TRY(t.tiles.reserve((size_t)nt + 1));
+  if (split) DDX_TRY(t.grp.reserve((size_t)ng + 1));
+  if (ninst > 1) {
+    DDX_TRY(t.info.reserve(ninst + 1));
+    DDX_HIP(hipMemcpyAsync(t.info.p, t.rows.data(), (ninst + 1) * sizeof(int4),
+                           hipMemcpyHostToDevice, h->stream));
+  }
+  hipLaunchKernelGGL(k_make_tiles, dim3((unsigned)(nt / 256 + 1)), dim3(256), 0, h->stream, ninst,
+                     (int)nt, chunk, TileRows{t.rows[0], t.rows[ninst > 1 ? 1 : ninst]}, t.info.p,
+                     t.tiles.p, split ? t.grp.p : nullptr);
   DDX_HIP(hipGetLastError());
   return DDX_OK;
 }
 
-int coulomb_field(ddx_handle *h, const int4 *tiles, int ntile, const int *grp, int ngrp,
-                  const double *q, const double *src3, const double *trg3, double *ef) {
+}  // namespace
+
+int potential_tiles(ddx_handle *h, TileTable &t, int nsrc, int ntrg) {
+  const int toff[2] = {0, ntrg}, soff[2] = {0, nsrc};
+  return make_tiles(h, t, 1, toff, soff, false);
+}
+
+int build_coulomb_tiles(ddx_handle *h) {
+  // potential (and solute field) at the cavity points from the spheres, and
+  // the field of the cavity charges at the nuclei
+  DDX_TRY(make_tiles(h, h->ctile, h->ninst, h->h_cavoff.data(), h->h_soff.data(), false));
+  return make_tiles(h, h->ftile, h->ninst, h->h_soff.data(), h->h_cavoff.data(), true);
+}
+
+int coulomb_potential(ddx_handle *h, const TileTable &t, const double *q, const double4 *src,
+                      const double *trg3, double *phi, double *ef) {
+  const int ntile = t.ntile;
+  if (ntile <= 0) return DDX_OK;
+  TimedLaunch tl(h, DDX_K_POTENTIAL, h->stream);
+  if (ef)
+    hipExtLaunchKernelGGL(k_potential<true>, dim3(ntile), dim3(kFW), 0, h->stream, tl.b, tl.e, 0,
+                          t.tiles.p, q, src, trg3, phi, ef);
+  else
+    hipExtLaunchKernelGGL(k_potential<false>, dim3(ntile), dim3(kFW), 0, h->stream, tl.b, tl.e,
+                          0, t.tiles.p, q, src, trg3, phi, nullptr);
+  DDX_HIP(hipGetLastError());
+  return DDX_OK;
+}
+
+int coulomb_field(ddx_handle *h, const TileTable &t, const double *q, const double *src3,
+                  const double *trg3, double *ef) {
+  const int ntile = t.ntile, ngrp = t.ngrp;
+  const int4 *tiles = t.tiles.p;
+  const int *grp = t.grp.p;
   if (ntile <= 0 || ngrp <= 0) return DDX_OK;
   DDX_TRY(h->fpart.reserve((size_t)ntile * kFW * 3));
   {
@@ -496,16 +486,9 @@ int coulomb_field(ddx_handle *h, const int4 *tiles, int ntile, const int *grp, i
 int coulomb_field_points(ddx_handle *h, int nsrc, const double *q, const double *src3, int ntrg,
                          const double *trg3, double *ef) {
   if (ntrg <= 0) return DDX_OK;
-  std::vector<int4> &t = h->h_xtile;
-  std::vector<int> &g = h->h_xgrp;
-  DDX_HIP(hipStreamSynchronize(h->stream));   // the previous tables' copies are done
-  coulomb_tiles({0, ntrg}, {0, nsrc}, true, t, g);
-  DDX_TRY(upload_tiles(h, h->xtile, t));
-  DDX_TRY(h->xgrp.reserve(g.size()));
-  DDX_HIP(hipMemcpyAsync(h->xgrp.p, g.data(), g.size() * sizeof(int), hipMemcpyHostToDevice,
-                         h->stream));
-  return coulomb_field(h, h->xtile.p, (int)t.size(), h->xgrp.p, (int)g.size() - 1, q, src3, trg3,
-                       ef);
+  const int toff[2] = {0, ntrg}, soff[2] = {0, nsrc};
+  DDX_TRY(make_tiles(h, h->xtile, 1, toff, soff, true));
+  return coulomb_field(h, h->xtile, q, src3, trg3, ef);
 }
 
 int make_psi_n(ddx_handle *h, int n, int nylm, const double *charge, double *psi) {

@@ -444,14 +444,12 @@ int field_forces_fields(ddx_handle *h, const double *d_charge, const double *d_z
     if (fmm)
       DDX_TRY(fmm_potential(h, d_charge, phi_scratch, ef));
     else
-      DDX_TRY(coulomb_potential(h, h->ctile.p, h->nctile, d_charge, h->sph.p, h->ccav.p,
-                                phi_scratch, ef));
+      DDX_TRY(coulomb_potential(h, h->ctile, d_charge, h->sph.p, h->ccav.p, phi_scratch, ef));
   }
   if (fmm)
     DDX_TRY(fmm_zeta_field(h, d_zeta, ez));
   else
-    DDX_TRY(coulomb_field(h, h->ftile.p, h->nftile, h->fgrp.p, h->nfgrp, d_zeta, h->ccav.p, c3,
-                          ez));
+    DDX_TRY(coulomb_field(h, h->ftile, d_zeta, h->ccav.p, c3, ez));
   return DDX_OK;
 }
 

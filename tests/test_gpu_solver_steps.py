@@ -20,6 +20,10 @@
   points against the definition evaluated here, and the triple lists, which
   the two operators read in different orders, by <u, L v> = <L* u, v> (1e-12
   of |u| |L v|: sums of up to 1e6 terms, rounding 1e-16 each).
+* test_field_at_tile_edges, test_potential_at_tile_edges: the Coulomb sums
+  where a tile of 64 targets, a block of 64 sources or a chunk of sources ends,
+  against the sums written out here (1e-12 of the sum of the terms' sizes: a
+  few thousand terms of a few ulp each).
 """
 import numpy as np
 import pytest
@@ -98,3 +102,34 @@ def test_setup_at_its_branches(n, ngrid):
     u, v = rng.standard_normal((2, n, 16))
     lv, lu = h.lx(v), h.lstarx(u)
     assert abs((u * lv).sum() - (lu * v).sum()) <= 1e-12 * np.linalg.norm(u) * np.linalg.norm(lv)
+
+
+def _coulomb(q, s, t):
+    """Potential and field sums, with the sums of their terms' sizes."""
+    d = t[:, None] - s[None]
+    r = np.sqrt((d * d).sum(2))
+    v, f = q / r, (q / r ** 3)[:, :, None] * d
+    return v.sum(1), np.abs(v).sum(1), f.sum(1), np.abs(f).sum(1)
+
+
+@pytest.mark.parametrize("nsrc,ntrg", [(0, 3), (1, 1), (63, 64), (64, 65), (65, 63), (255, 129),
+                                       (256, 128), (257, 1), (1100, 200), (4000, 64)])
+def test_field_at_tile_edges(nsrc, ntrg):
+    from ddpcm_amd.ddx import DDCosmo
+    rng = np.random.default_rng(nsrc + ntrg)
+    h = DDCosmo([0.0], [0.0], [0.0], [2.0], 2, 26)
+    q, s = rng.uniform(-1, 1, nsrc), rng.uniform(-9, 9, (nsrc, 3))
+    t = rng.uniform(10, 30, (ntrg, 3))
+    _, _, f, size = _coulomb(q, s, t)
+    assert np.all(np.abs(h.efld(q, s, t) - f) <= 1e-12 * size)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 129])
+def test_potential_at_tile_edges(n):
+    from ddpcm_amd.ddx import DDCosmo
+    from ddpcm_amd.inputs import synthetic_input
+    x, y, z, r = synthetic_input(n, 31 + n, 2, 50).bohr()
+    h = DDCosmo(x, y, z, r, 2, 50)
+    q = np.linspace(-1.0, 1.5, n)
+    v, size, _, _ = _coulomb(q, np.stack([x, y, z], 1), h.ccav)
+    assert np.all(np.abs(h.mkrhs(q)[0] - v) <= 1e-12 * size)
