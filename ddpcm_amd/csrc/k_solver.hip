@@ -880,8 +880,10 @@ __global__ __launch_bounds__(kExtrapThreads) void k_extrap_one(
     slot[q] = (unsigned)st->slot[q];
     coef[q] = st->coef[q];
   }
+  // (the slots past ncoef need not exist: a shorter history has fewer of them)
 #pragma unroll
-  for (int q = 0; q < kDiisMax; ++q) slot[q] = __builtin_amdgcn_readfirstlane((int)slot[q]);
+  for (int q = 0; q < kDiisMax; ++q)
+    slot[q] = __builtin_amdgcn_readfirstlane((int)(q < ncoef ? slot[q] : slot[0]));
   if (done) return;
   const unsigned c0 = n * blockIdx.x / nbe, c1 = n * (blockIdx.x + 1) / nbe;
   const unsigned ne = (c1 - c0) * nylm, e0 = c0 * nylm;

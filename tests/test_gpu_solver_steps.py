@@ -14,6 +14,8 @@
   solutions bit for bit, at one and several workgroups, with a workgroup's
   second element per thread absent, partial and full.  (At these sizes every
   sweep worker has one unit, so the operators' sums are split alike.)
+* test_short_histories: histories shorter than the largest give the same
+  solution (1e-10 in the h^-1/2 norm for increments below 1e-12).
 * test_setup_at_its_branches: the setup where its kernels change (direct or
   hashed neighbour search, one or four waves a sphere, one or several tiles of
   the prefix sums, fewer points than a wave): the neighbour lists and exposed
@@ -67,6 +69,22 @@ def test_single_system_equals_batch_of_two(n, lmax, ngrid, mixed):
         one, two = h.get(name), b.get(name)
         assert np.array_equal(one, two[:n]) and np.array_equal(one, two[n:]), name
     assert e == eb[0] == eb[1]
+
+
+@pytest.mark.parametrize("star", [False, True])
+@pytest.mark.parametrize("n", [3, 70])
+def test_short_histories(n, star):
+    from ddpcm_amd.ddx import DDCosmo
+    from ddpcm_amd.inputs import synthetic_input
+    x, y, z, r = synthetic_input(n, 5 + n, 6, 110).bohr()
+    h = DDCosmo(x, y, z, r, 6, 110)
+    rhs = np.random.default_rng(n).standard_normal((n, h.nylm))
+    x0 = h.get("facl")[None, :] * rhs
+    ref, _, ok = h.jacobi_diis(star, rhs, x0, tol=1e-12)
+    assert ok
+    for m in (11, 12, 18, 24):
+        got, _, ok = h.jacobi_diis(star, rhs, x0, diis_max=m, tol=1e-12)
+        assert ok and h.hnorm(got - ref) <= 1e-10, m
 
 
 @pytest.mark.parametrize("n,ngrid", [(1, 6), (5, 14), (65, 74), (300, 302), (2048, 26),
