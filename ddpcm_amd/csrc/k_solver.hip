@@ -24,6 +24,7 @@
 #include "ddx_kernels.hpp"
 
 #include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <iterator>
 
@@ -270,6 +271,21 @@ __device__ __forceinline__ void jacobi_two_elements(
   }
 }
 
+// The state as the round found it, for k_diis_extrap: into the next state by
+// one workgroup, all loads ahead of the stores.
+__device__ __forceinline__ void copy_state(DiisState *st) {
+  constexpr int kWords = (int)(offsetof(DiisState, hist) / sizeof(double));
+  constexpr int kEach = (kWords + kJThreads - 1) / kJThreads;
+  const double *from = reinterpret_cast<const double *>(st);
+  double *to = reinterpret_cast<double *>(st + 1);
+  double v[kEach];
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) v[i] = from[min((int)threadIdx.x + i * kJThreads, kWords - 1)];
+#pragma unroll
+  for (int i = 0; i < kEach; ++i)
+    if ((int)threadIdx.x + i * kJThreads < kWords) to[threadIdx.x + i * kJThreads] = v[i];
+}
+
 // k_jacobi for one system of at most 512 elements per workgroup, two per
 // thread: the same sums, arranged for latency.  Such a launch (under 700
 // workgroups at 2000 atoms) is a chain of memory round trips of 0.7 us and
@@ -291,6 +307,10 @@ __global__ __launch_bounds__(kJThreads) void k_jacobi_two(unsigned nn, unsigned 
                                                           const double *__restrict__ facl,
                                                           Systems sys) {
   const SysArgs a = sys.s[blockIdx.y];
+  if (blockIdx.x == nbj) {   // (launched where k_diis_extrap follows)
+    copy_state(a.st);
+    return;
+  }
   asm volatile("" ::"s"(a.rhs), "s"(a.y), "s"(a.yp), "s"(a.segoff), "s"(a.x), "s"(a.ed),
                "s"(a.st), "s"(a.yacc), "s"(a.part), "s"(facl));
   const DiisState *__restrict__ st = a.st;
@@ -352,9 +372,9 @@ __global__ __launch_bounds__(kJThreads) void k_jacobi_two(unsigned nn, unsigned 
         (wpart[0][q] + wpart[1][q]) + (wpart[2][q] + wpart[3][q]);
 }
 
-// The DIIS bookkeeping of one iteration on one wave, all in registers: lane r
-// holds row r of the bordered Gram matrix B (0-based here; the reference's
-// b(r+1, c+1)), n1 = nmat + 1 <= 25 rows.
+// The DIIS bookkeeping of one iteration on one wave, on the bordered Gram matrix
+// B (0-based here; the reference's b(r+1, c+1)) of n1 = nmat + 1 <= 25 rows,
+// staged in LDS.
 //
 //   drop-10 rule   when nmat reached diis_max the 10 oldest vectors go: rows
 //                  and columns 11.. move to 1.. (jacobi_diis.f90:216-227)
@@ -449,11 +469,82 @@ __device__ __forceinline__ double max_abs(double a, double b) {
   return m;
 }
 
+constexpr int kGramSums = kPartStride + 2;
+// the staged B: kB rows of kBs doubles (an odd stride: a column's rows fall into
+// different banks), and room for the new row after the oldest have gone
+constexpr int kBs = kB + 2, kStage = (kB + 1) * kBs;
+
+// The Gram-row dot products and the increment norms of the previous iteration
+// into red: value q < 26 is the sum of nblk workgroup partials part[q nbj ..],
+// values 26 and 27 those of nblk_e partials part_e0 and part_e1.  Eight
+// consecutive lanes share a value, each sums every eighth partial, so that all
+// loads are in flight together, and the eight partial sums meet in three
+// lane-pair stages within the group.
+__device__ __forceinline__ void gram_sums(int tid, int nblk, int nblk_e,
+                                          const double *__restrict__ part, int nbj,
+                                          const double *__restrict__ part_e0,
+                                          const double *__restrict__ part_e1, double *red) {
+#pragma clang fp contract(off)
+  const int q = tid / kTPQ, r = tid % kTPQ;
+  const bool norm_row = q >= kPartStride;
+  const double *src = q > kPartStride ? part_e1 : norm_row ? part_e0 : part + (size_t)q * nbj;
+  const int nb = norm_row ? nblk_e : nblk;
+  // (a wave's eight values need as many loads as the longest of them)
+  const bool last = __builtin_amdgcn_readfirstlane(tid / kWave) == kPartStride * kTPQ / kWave;
+  const int most = last ? max(nblk, nblk_e) : nblk;
+  double s;
+  if (most <= kTPQ * 8)
+    s = sum_partials<8>(src, nb, r);
+  else if (most <= kTPQ * 16)
+    s = sum_partials<16>(src, nb, r);
+  else
+    s = sum_partials<24>(src, nb, r);
+  s += partner<3>(s);
+  s += partner<4>(s);
+  s += partner<5>(s);
+  if (r == 0 && q < kGramSums) red[q] = s;
+}
+
+// `per` >= 192 threads take the words of the state's B through registers
+// (load_b) to LDS (stage_b).
+constexpr int kBWords = (kB * kB + 191) / 192;
+__device__ __forceinline__ void load_b(const DiisState *st, int t, int per,
+                                       double (&v)[kBWords]) {
+#pragma unroll
+  for (int i = 0; i < kBWords; ++i) v[i] = st->b[min(t + i * per, kB * kB - 1)];
+}
+__device__ __forceinline__ void stage_b(double *bs, int t, int per, const double (&v)[kBWords]) {
+#pragma unroll
+  for (int i = 0; i < kBWords; ++i) {
+    const int q = t + i * per;
+    if (q < kB * kB) bs[q / kB * kBs + q % kB] = v[i];
+  }
+}
+
+// Row and column nmat + off of the staged B for the new vector, by one wave:
+// the border's 1, the dots, the self dot.
+__device__ __forceinline__ void add_row(double *bs, const double *red, int off, int nmat) {
+  const int c = min(lane_id(), nmat);
+  const double dot = red[c == nmat ? kDiisMax : max(c - 1, 0)], v = c == 0 ? 1.0 : dot;
+  bs[(nmat + off) * kBs + c + off] = v;
+  bs[(c + off) * kBs + nmat + off] = v;
+  wave_lds_sync();
+}
+
+// Entry (r, c) of the bordered matrix: row and column 0 are (0, 1, 1, ..), the
+// others are the staged B's, `off` rows and columns further on (0, or 10 when
+// the oldest vectors go).
+__device__ __forceinline__ double border(const double *bs, int off, int r, int c) {
+  const double v = bs[(r + off) * kBs + c + off];
+  const double edge = r == c ? 0.0 : 1.0;
+  return r == 0 || c == 0 ? edge : v;
+}
+
 // Gauss-Jordan with full pivoting on the bordered system of k_diis_small,
-// n1 <= 2 J rows, by one wave without barriers.  Lane L works on row
-// r = L & 31 and on the columns 2 j + (L >> 5), j < J; lane r < kB holds row r
-// in a on entry.  A row exchange of the reference is an exchange of two `pos`
-// values (a lane's current row index); the right-hand side e_1 is bv.
+// n1 = nmat + 1 <= 2 J rows, by one wave without barriers.  Lane L works on row
+// r = L & 31 and on the columns 2 j + (L >> 5), j < J.  A row exchange of the
+// reference is an exchange of two `pos` values (a lane's current row index);
+// the right-hand side e_1 is bv.
 //   Pivot: the largest |a(j, k)| over the rows and columns not yet pivoted,
 // first in row-major order of the current indices on ties, as the reference's
 // nested loops pick it.  Each lane takes the maximum of its own columns and
@@ -473,23 +564,27 @@ __device__ __forceinline__ double max_abs(double a, double b) {
 // six-stage reductions of 64-bit values.  Average launch of k_diis_small, four
 // waves -> one wave and its loads unchained: 15.5 -> 9.8 us at 60 atoms (up
 // to 22 rows), 20.9 -> 13.7 us at 2000 atoms (up to 25), 19.2 -> 12.6 us on a
-// batch of 64 molecules.
+// batch of 64 molecules.  B staged in LDS by the whole workgroup instead of row
+// by row in registers, the candidates' inverses ahead of the search's end and
+// the dots of few partials not padded to the norm's number: 13.7 -> 12.9 us at
+// 2000 atoms.
 template <int J>
-__device__ __forceinline__ bool eliminate(const double (&a)[kB], int n1, double *rowbuf,
+__device__ __forceinline__ bool eliminate(const double *bs, int off, int nmat, double *rowbuf,
                                           double &bv, int &pos) {
 #pragma clang fp contract(off)
   constexpr int JP = J <= 4 ? 4 : J <= 8 ? 8 : 16;
   typedef double Row __attribute__((ext_vector_type(JP)));
   const int lane = lane_id(), r = lane & 31, half = lane >> 5;
+  const int n1 = nmat + 1;
   Row g;
 #pragma unroll
   for (int j = 0; j < JP; ++j) g[j] = 0.0;
 #pragma unroll
   for (int j = 0; j < J; ++j) {
-    const double lo = a[2 * j];
-    const double hi = partner<0>(2 * j + 1 < kB ? a[2 * j + 1 < kB ? 2 * j + 1 : 0] : 0.0);
-    const double v = half ? hi : lo;
-    g[j] = (r < n1 && 2 * j + half < n1) ? v : 0.0;
+    const int c = 2 * j + half;
+    double v = border(bs, off, min(r, nmat), min(c, nmat));
+    asm volatile("" : "+v"(v));   // (unconditional: all loads in flight together)
+    g[j] = (r < n1 && c < n1) ? v : 0.0;
   }
   bv = (r == 0) ? 1.0 : 0.0;
   pos = r;
@@ -509,10 +604,11 @@ __device__ __forceinline__ bool eliminate(const double (&a)[kB], int n1, double 
     for (int j = J - 1; j >= 0; --j) jc = (fabs(g[j]) == big) ? j : jc;
     const int code = pos * 32 + 2 * jc + half;
     // every lane inverts its own candidate while the search goes on
-    const double rec = 1.0 / big;
+    double rec = 1.0 / big;
     const unsigned long long bits = (unsigned long long)__double_as_longlong(big);
     const unsigned hi = (unsigned)(bits >> 32), lo = (unsigned)bits;
     const unsigned mhi = wave_max_u32(hi);
+    asm volatile("" : "+v"(rec));   // (not after the search: it fills the search's waits)
     unsigned long long cand = __ballot(hi == mhi);
     if (__popcll(cand) > 1) {
       const unsigned mlo = wave_max_u32(hi == mhi ? lo : 0u);
@@ -567,6 +663,42 @@ __device__ __forceinline__ bool eliminate(const double (&a)[kB], int n1, double 
   return true;
 }
 
+// eliminate with the register count of a lane that the system's size needs
+__device__ __forceinline__ bool eliminate_any(const double *bs, int off, int nmat,
+                                              double *rowbuf, double &bv, int &pos) {
+  bool ok;
+  if (nmat < 8) ok = eliminate<4>(bs, off, nmat, rowbuf, bv, pos);
+  else if (nmat < 14) ok = eliminate<7>(bs, off, nmat, rowbuf, bv, pos);
+  else if (nmat < 20) ok = eliminate<10>(bs, off, nmat, rowbuf, bv, pos);
+  else ok = eliminate<13>(bs, off, nmat, rowbuf, bv, pos);
+  return ok;
+}
+
+// The new B into the state, by one wave: the new row and column, or all of it
+// where the oldest vectors went.
+__device__ __forceinline__ void store_b(const double *bs, int off, int nmat, DiisState *st) {
+  const int lane = lane_id();
+  if (off) {
+    for (int q = lane; q < kB * kB; q += kWave) {
+      const int r = q / kB, c = q % kB;
+      if (r <= nmat && c <= nmat) st->b[q] = border(bs, off, r, c);
+    }
+  } else if (lane <= nmat) {
+    const double v = border(bs, 0, nmat, lane);
+    st->b[nmat * kB + lane] = v;
+    st->b[lane * kB + nmat] = v;
+  }
+}
+
+// logical slots once the oldest have been recycled: j <- j + 10 for j < nmat,
+// the recycled ones after
+__device__ __forceinline__ int recycle(int myslot, int off, int nmat, int diis_max) {
+  const int lane = lane_id();
+  const int src = lane < nmat ? lane + 10 : lane - nmat;
+  const int moved = __shfl(myslot, src < diis_max ? src : 0, kWave);
+  return off ? moved : myslot;
+}
+
 __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
     int diis_max, int nbj, int nbe, int nsph_all, const int *__restrict__ jboff,
     const int *__restrict__ eboff, const int *__restrict__ soff, int ninst, int maxit,
@@ -595,35 +727,16 @@ __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
     nsph = soff[inst + 1] - soff[inst];
   }
   DiisState *sum = ninst > 1 ? q0.st + ninst : nullptr;
-  // lane r: row r of B and logical slot r
-  double a[kB];
-#pragma unroll
-  for (int c = 0; c < kB; ++c) a[c] = st->b[min(lane, kB - 1) * kB + c];
   int myslot = st->slot[min(lane, kDiisMax - 1)];
-  __shared__ double red[kPartStride + 1];
-  // Gram-row dot products and the increment norm of the previous iteration
-  // (value 26): eight consecutive lanes share a value, each sums every eighth
-  // workgroup partial, so that all loads are in flight together, and the
-  // eight partial sums meet in three lane-pair stages within the group
-  {
-    const int q = tid / kTPQ, r = tid % kTPQ;
-    const bool norm_row = q >= kPartStride;
-    const double *src = norm_row ? q0.part_e + eb : q0.part + jb + (size_t)q * nbj;
-    const int nb = norm_row ? nblk_e : nblk;
-    double s;
-    if (max(nblk, nblk_e) <= kTPQ * 8)
-      s = sum_partials<8>(src, nb, r);
-    else
-      s = sum_partials<32>(src, nb, r);
-    s += partner<3>(s);
-    s += partner<4>(s);
-    s += partner<5>(s);
-    if (r == 0 && q <= kPartStride) red[q] = s;
-  }
+  __shared__ double bs[kStage];
+  __shared__ double red[kGramSums];
+  double old[kBWords];
+  load_b(st, tid, kSmallThreads, old);
+  gram_sums(tid, nblk, nblk_e, q0.part + jb, nbj, q0.part_e + eb, q0.part_e + eb, red);
+  stage_b(bs, tid, kSmallThreads, old);
   __syncthreads();
   if (done) return;
   const int off = (nmat >= diis_max) ? 10 : 0;
-  const int ndot = nmat - off - 1;
   const int lastslot = __builtin_amdgcn_readlane(myslot, __builtin_amdgcn_readfirstlane(nmat - 1));
   if (pending) {
     // rms of the per-sphere norms and the convergence test of the previous
@@ -644,78 +757,23 @@ __global__ __launch_bounds__(kSmallThreads) void k_diis_small(
   }
   // the bordered system is one wave's work from here on
   if (wave != 0) return;
-  // B update
-  {
-  // lane i + 1 keeps dot i; every lane keeps the self dot
-  const int qi = (lane >= 1 && lane <= kDiisMax) ? lane - 1 : 0;
-  double mydot = red[qi];
-  const double self = red[kDiisMax];
-  if (!(lane >= 1 && lane - 1 < ndot)) mydot = 0.0;
-  if (nmat >= diis_max) {
-    const int m = nmat - 10;
-    // rows 1..m-1 <- rows 11..m+9, then columns likewise
-    double moved[kB];
-#pragma unroll
-    for (int c = 0; c < kB; ++c) moved[c] = __shfl(a[c], min(lane + 10, kWave - 1), kWave);
-    if (lane >= 1 && lane <= m - 1) {
-#pragma unroll
-      for (int c = 0; c < kB; ++c) a[c] = moved[c];
-#pragma unroll
-      for (int c = 1; c + 10 < kB; ++c) a[c] = (c <= m - 1) ? a[c + 10] : a[c];
-    }
-    // slots: logical j (0-based) <- j + 10 for j < m, recycled ones after
-    int src = (lane < m) ? lane + 10 : lane - m;
-    myslot = __shfl(myslot, src < diis_max ? src : 0, kWave);
-    nmat = m;
-  }
-  // makeb: row / column nmat (0-based) of the new vector
-  if (nmat == 1) {
-    if (lane == 0) { a[0] = 0.0; a[1] = 1.0; }
-    if (lane == 1) { a[0] = 1.0; a[1] = self; }
-  } else {
-    double rowv[kB];   // rowv[c] = dot c-1, from the block's LDS copy
-    rowv[0] = 0.0;
-#pragma unroll
-    for (int c = 1; c < kB; ++c) rowv[c] = red[c - 1];
-#pragma unroll
-    for (int c = 0; c < kB; ++c) {
-      if (c == nmat) {
-        if (lane == 0) a[c] = 1.0;
-        else if (lane < nmat) a[c] = mydot;
-        else if (lane == nmat) a[c] = self;
-      }
-    }
-    if (lane == nmat) {
-      a[0] = 1.0;
-#pragma unroll
-      for (int c = 1; c < kB; ++c)
-        if (c < nmat) a[c] = rowv[c];
-    }
-  }
-  }
+  nmat -= off;
+  myslot = recycle(myslot, off, nmat, diis_max);
+  add_row(bs, red, off, nmat);
   // persist B and the slot map; k_extrap leaves this iteration's norm
-  if (lane < kB) {
-#pragma unroll
-    for (int c = 0; c < kB; ++c) st->b[lane * kB + c] = a[c];
-  }
+  store_b(bs, off, nmat, st);
   if (lane < diis_max) st->slot[lane] = myslot;
   if (lane == 0) {
     st->pending_norm = 1;
     q0.newslot[inst] = lastslot;
   }
 
-  // the register count of a lane follows the system's size
   __shared__ __align__(16) double rowbuf[32];
-  const int n1 = nmat + 1;
   double bv;
   int pos;
-  bool ok;
-  if (n1 <= 8) ok = eliminate<4>(a, n1, rowbuf, bv, pos);
-  else if (n1 <= 14) ok = eliminate<7>(a, n1, rowbuf, bv, pos);
-  else if (n1 <= 20) ok = eliminate<10>(a, n1, rowbuf, bv, pos);
-  else ok = eliminate<13>(a, n1, rowbuf, bv, pos);
+  const bool ok = eliminate_any(bs, off, nmat, rowbuf, bv, pos);
   if (ok) {
-    if (lane < n1 && pos >= 1) st->coef[pos - 1] = bv;
+    if (lane <= nmat && pos >= 1) st->coef[pos - 1] = bv;
   }
   const int cur = __builtin_amdgcn_readlane(myslot, ok ? __builtin_amdgcn_readfirstlane(nmat) : 0);
   if (lane == 0) {
@@ -831,6 +889,56 @@ __global__ __launch_bounds__(kJThreads) void k_extrap(int nylm, size_t nn, int d
   if (threadIdx.x == 0) part[blockIdx.x] = tot;
 }
 
+// Sum of the squared norms of `count` <= 64 spheres by one wave, a sphere to a
+// lane: its nylm terms from LDS in order, eight loaded ahead of the additions.
+__device__ __forceinline__ double sphere_norms(const double *terms, unsigned count,
+                                               unsigned nylm) {
+  double usq = 0.0;
+  const unsigned lane = (unsigned)lane_id();
+  if (lane < count) {
+    const double *t = terms + lane * nylm;
+    const int last = (int)nylm - 1;
+    double sq = 0.0, ahead[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ahead[i] = t[min(i, last)];
+    for (int l = 0; l <= last; l += 8) {
+      double v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i] = ahead[i];
+        ahead[i] = t[min(l + 8 + i, last)];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (l + i <= last) sq += v[i];
+    }
+    const double u = sqrt(sq);
+    usq += u * u;
+  }
+  return wave_sum(usq);
+}
+
+// one element of the C newest history vectors, all loads in flight together
+template <int C>
+__device__ __forceinline__ void load_history_c(const double *__restrict__ xd, unsigned nn,
+                                               unsigned k, const unsigned (&slot)[kB - 1],
+                                               double (&v)[kB - 1]) {
+#pragma unroll
+  for (int q = 0; q < C; ++q)
+    v[q] = load_at<double>(xd, (slot[q] * nn + k) * (unsigned)sizeof(double));
+#pragma unroll
+  for (int q = C; q < kB - 1; ++q) v[q] = 0.0;
+}
+
+// ... at least `depth` of them
+__device__ __forceinline__ void load_history(const double *__restrict__ xd, unsigned nn,
+                                             unsigned k, const unsigned (&slot)[kB - 1], int depth,
+                                             double (&v)[kB - 1]) {
+  if (depth <= 8) load_history_c<8>(xd, nn, k, slot, v);
+  else if (depth <= 16) load_history_c<16>(xd, nn, k, slot, v);
+  else load_history_c<kB - 1>(xd, nn, k, slot, v);
+}
+
 // x_new = sum_i c_i x_i of one element: the history values of the C >= ncoef
 // newest slots are loaded together (those past ncoef re-read slot 0 and are
 // not added).
@@ -908,29 +1016,152 @@ __global__ __launch_bounds__(kExtrapThreads) void k_extrap_one(
   }
   __syncthreads();
   if (threadIdx.x >= kWave) return;
-  double usq = 0.0;
-  if (threadIdx.x < c1 - c0) {
-    const double *t = terms + threadIdx.x * nylm;
-    const int last = (int)nylm - 1;
-    double sq = 0.0, ahead[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ahead[i] = t[min(i, last)];
-    for (int l = 0; l <= last; l += 8) {
-      double v[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        v[i] = ahead[i];
-        ahead[i] = t[min(l + 8 + i, last)];
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (l + i <= last) sq += v[i];
-    }
-    const double u = sqrt(sq);
-    usq += u * u;
-  }
-  usq = wave_sum(usq);
+  const double usq = sphere_norms(terms, c1 - c0, nylm);
   if (threadIdx.x == 0) a.part_e[blockIdx.x] = usq;
+}
+
+// k_diis_small and k_extrap_one in one launch, for one system whose workgroups
+// have a compute unit each: every workgroup solves the bordered system for itself (its
+// wave 0; the same operations, so the same weights in all of them), while its
+// other waves, one element to a thread, have the iterate and the history in
+// flight; then they extrapolate as k_extrap_one does.
+//   They read the copy of the state that k_jacobi_two left behind it, and the
+// first of them writes the state.  A workgroup may leave its norm partial
+// while another still sums the previous iteration's, so the two iterations'
+// partials alternate between two arrays, by the iteration's parity.
+//   Bound by the elimination (one wave's serial chain, 0.6 us a row).  Launches
+// of 7.2 to 21 us and 4.6 us become one of 8.3 to 21.4 us at 60 atoms; a whole
+// step, two launches -> one: 60 atoms 1203 -> 1165 us, 259 atoms 1510 -> 1469,
+// 400 atoms 1538 -> 1484 (lmax 6).
+__global__ __launch_bounds__(kExtrapThreads, 4) void k_diis_extrap(
+    unsigned n, unsigned nylm, unsigned nn, unsigned nbe, int nbj, int diis_max, int maxit,
+    const double *__restrict__ invl1, const double *__restrict__ cf, Systems sys) {
+  const SysArgs s = sys.s[blockIdx.y];
+  asm volatile("" ::"s"(s.x), "s"(s.xs), "s"(s.xd), "s"(s.st), "s"(s.inc), "s"(s.part),
+               "s"(s.part_e), "s"(invl1), "s"(cf));
+  const DiisState *__restrict__ old = s.st + 1;
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const unsigned nelem = blockDim.x - kWave;   // one element to a thread
+  __shared__ double terms[kExtrapTerms];
+  __shared__ double bs[kStage];
+  __shared__ double red[kGramSums];
+  __shared__ double weight[kB];
+  __shared__ __align__(16) double rowbuf[32];
+  __shared__ int solved;
+  const bool done = old->done != 0, pending = old->pending_norm != 0;
+  const double tol = old->tol;
+  const int nmat0 = old->nmat, it0 = old->it;
+  const int off = nmat0 >= diis_max ? 10 : 0, nmat = nmat0 - off;   // nmat: the weights' number
+  const unsigned c0 = n * blockIdx.x / nbe, c1 = n * (blockIdx.x + 1) / nbe;
+  const unsigned ne = (c1 - c0) * nylm, e0 = c0 * nylm;
+  // the previous iteration's norm and convergence test, as in k_diis_small
+  const auto test = [&](double &norm) {
+    norm = sqrt(red[kPartStride + (it0 & 1)] / (double)(int)n);
+    return pending && (norm < tol || it0 + 1 >= maxit);
+  };
+  double norm;
+  // (two paths with the same barriers, so that no register of one is kept in
+  // the other)
+  if (wave == 0) {
+    const int slots = old->slot[min(lane, kDiisMax - 1)];
+    gram_sums(tid, nbj, (int)nbe, s.part, nbj, s.part_e, s.part_e + nbe, red);
+    __syncthreads();
+    if (done) return;
+    const bool stop = test(norm);
+    double bv;
+    int pos;
+    bool ok = false;
+    if (!stop) {
+      add_row(bs, red, off, nmat);
+      ok = eliminate_any(bs, off, nmat, rowbuf, bv, pos);
+      if (ok && lane <= nmat && pos >= 1) weight[pos - 1] = bv;
+      if (lane == 0) solved = ok;
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) {
+      DiisState *st = s.st;
+      if (pending && lane == 0) {
+        if (it0 <= kMaxIter) st->hist[it0] = norm;
+        st->it = it0 + 1;
+        st->norm = norm;
+        st->ok = norm < tol;
+      }
+      if (stop) {
+        instance_done(nullptr, st, s.rec, it0, norm, norm < tol);
+        if (lane == 0) st->done = 1;
+      } else {
+        store_b(bs, off, nmat, st);
+        const int myslot = recycle(slots, off, nmat, diis_max);
+        if (lane < diis_max) st->slot[lane] = myslot;
+        const int cur = __builtin_amdgcn_readlane(
+            myslot, __builtin_amdgcn_readfirstlane(ok ? nmat : 0));
+        if (lane == 0) {
+          st->cur = cur;
+          st->nmat = ok ? nmat + 1 : 1;
+          st->pending_norm = 1;
+          if (!ok) st->singular += 1;
+        }
+      }
+    }
+    if (!stop) __syncthreads();
+    return;
+  }
+  // the old B into LDS, and beside it what the elements need
+  double b[kBWords];
+  load_b(old, tid - kWave, nelem, b);
+  unsigned slot[kB - 1];
+  {
+    int all[kDiisMax];
+#pragma unroll
+    for (int q = 0; q < kDiisMax; ++q) all[q] = old->slot[q];
+#pragma unroll
+    for (int q = 0; q < kB - 1; ++q) {   // (past nmat: slot 0, read and not added)
+      const int s = off ? all[q + 10 < kDiisMax ? q + 10 : 0] : all[q];
+      slot[q] = (unsigned)__builtin_amdgcn_readfirstlane(q < nmat ? s : all[0]);
+    }
+  }
+  unsigned k = e0 + min((unsigned)tid - kWave, ne - 1);
+  double x = s.x[k], il = invl1[k % nylm], cl = cf[k % nylm], v[kB - 1];
+  if (tid < kGramSums * kTPQ)
+    gram_sums(tid, nbj, (int)nbe, s.part, nbj, s.part_e, s.part_e + nbe, red);
+  stage_b(bs, tid - kWave, nelem, b);
+  load_history(s.xd, nn, k, slot, nmat, v);
+  __syncthreads();
+  if (done) return;
+  const bool stop = test(norm);
+  __syncthreads();
+  if (stop) return;
+  const bool ok = solved != 0;
+  for (unsigned j = (unsigned)tid - kWave; j < ne; j += nelem) {
+    if (j >= nelem) {
+      k = e0 + j;
+      x = s.x[k];
+      il = invl1[k % nylm];
+      cl = cf[k % nylm];
+      load_history(s.xd, nn, k, slot, nmat, v);
+    }
+    double xn = 0.0;
+    if (ok) {
+#pragma unroll
+      for (int q = 0; q < kB - 1; ++q)
+        if (q < nmat) xn = xn + weight[q] * v[q];
+    } else {   // the plain Jacobi step: the newest vector
+#pragma unroll
+      for (int q = 0; q < kB - 1; ++q)
+        if (q == nmat - 1) xn = v[q];
+    }
+    const double inc = xn - x;
+    s.x[k] = xn;
+    if (s.xs) s.xs[k] = cl * (s.xs_inc ? inc : xn);
+    if (s.inc) s.inc[k] = inc;
+    terms[j] = il * inc * inc;
+  }
+  __syncthreads();
+  if (wave != 1) return;
+  const double usq = sphere_norms(terms, c1 - c0, nylm);
+  const int it = pending ? it0 + 1 : it0;   // this iteration
+  if (lane == 0) s.part_e[(it & 1) * nbe + blockIdx.x] = usq;
 }
 
 // rms of the per-sphere norms and the convergence test (rmsvec,
@@ -1226,11 +1457,11 @@ int solve_begin(ddx_handle *h, Lane &ln, int star, int diis_max, double tol, con
     DDX_TRY(ln.xd.reserve(nn * diis_max));
     DDX_TRY(ln.ed.reserve(nn * diis_max));
   }
-  DDX_TRY(ln.part.reserve((size_t)h->nbj * kPartStride + h->nbe + 1));
+  DDX_TRY(ln.part.reserve((size_t)h->nbj * kPartStride + 2 * (size_t)h->nbe + 1));
   // the L* sweep leaves per-segment sums that k_jacobi reads: its buffer must
   // not move once the solve has started
   if (star) DDX_TRY(ln.yp.reserve((size_t)h->nseg_cap * h->nylm + 1));
-  DDX_TRY(ln.diis.reserve(h->ninst + 1));
+  DDX_TRY(ln.diis.reserve(h->ninst + 1));   // and the summary, or k_diis_extrap's copy
   DDX_TRY(ln.misc.reserve(h->ninst + 1));
   DDX_TRY(ln.res.reserve(2 * (size_t)h->ninst + 2));
   ln.star = star;
@@ -1274,6 +1505,15 @@ bool extrap_one_fits(const ddx_handle *h, size_t nn, int diis_max) {
   return jacobi_two_fits(h, nn, diis_max) && most <= kWave && most * h->nylm <= kExtrapTerms;
 }
 
+// Whether k_diis_extrap takes a system: as k_extrap_one, and a compute unit for
+// every workgroup of both solves.  With two workgroups to a unit, each loading
+// the state and the dots for itself, there is nothing left to gain: a step of
+// 642 atoms takes 1583 us with it and 1588 without, 1000 atoms (lmax 8) 3363
+// and 3331.
+bool diis_extrap_fits(const ddx_handle *h, size_t nn, int diis_max) {
+  return extrap_one_fits(h, nn, diis_max) && 2 * h->nbe <= h->ncu;
+}
+
 // `nr` rounds of one solve, or of a direct and an adjoint solve in lockstep
 int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
   Lane &l0 = *lanes[0];
@@ -1283,6 +1523,7 @@ int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
   const int nbj = h->nbj, nbe = h->nbe, ninst = h->ninst;
   const double *invl1 = h->cf.p + h->nylm;   // 1/(l+1) table stored after cf
   const int diis_max = l0.diis_max;
+  const bool fused = diis_extrap_fits(h, nn, diis_max);
   Systems sys{};
   for (int k = 0; k < count; ++k) sys.s[k] = sys_args(h, *lanes[k]);
   for (int g = 0; g < nr; ++g, ++l0.enqueued) {
@@ -1315,7 +1556,7 @@ int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
       // mixed precision keeps the residual history in FP32
       const auto launch = [&](auto two, auto one) {
         if (jacobi_two_fits(h, nn, diis_max))
-          hipExtLaunchKernelGGL(two, dim3(nbj, count), dim3(kJThreads), 0, s, tl.b, tl.e, 0,
+          hipExtLaunchKernelGGL(two, dim3(nbj + (fused ? 1 : 0), count), dim3(kJThreads), 0, s, tl.b, tl.e, 0,
                                 (unsigned)nn, (unsigned)h->nylm, diis_max, (unsigned)nbj,
                                 h->facl.p, sys);
         else
@@ -1326,6 +1567,16 @@ int enqueue_rounds(ddx_handle *h, Lane *const *lanes, int count, int nr) {
       else launch(k_jacobi_two<double>, k_jacobi<double>);
     }
     DDX_HIP(hipGetLastError());
+    if (fused) {
+      TimedLaunch tl(h, DDX_K_DIIS, s);
+      const int most = (h->n + nbe - 1) / nbe * h->nylm;   // elements of a workgroup
+      const int nt = std::max(kSmallThreads,
+                              std::min(kExtrapThreads, kWave + (most + kWave - 1) / kWave * kWave));
+      hipExtLaunchKernelGGL(k_diis_extrap, dim3(nbe, count), dim3(nt), 0, s, tl.b, tl.e, 0, (unsigned)h->n, (unsigned)h->nylm, (unsigned)nn,
+                            (unsigned)nbe, nbj, diis_max, l0.max_iter, invl1, h->cf.p, sys);
+      DDX_HIP(hipGetLastError());
+      continue;
+    }
     if (diis_max > 0) {
       TimedLaunch tl(h, DDX_K_DIIS, s);
       hipExtLaunchKernelGGL(k_diis_small, dim3(ninst, count), dim3(kSmallThreads), 0, s, tl.b,
