@@ -13,7 +13,7 @@
 // One sweep kernel serves both operators, and both at once: the triples are
 // grouped by container c, one wave per container.  The per-(l, m) constant
 // cf = facs * 4pi/(2l+1) is applied outside the triple loop: L X contracts
-// with X' = cf X (uniform across the wave, read through the scalar cache),
+// with X' = cf X (16 values to a vector register, read by row broadcast),
 // L* S accumulates sum_t coef_t p~ trig in registers per lane and multiplies
 // by cf after one LDS transpose reduction per container.  When the direct
 // and the adjoint solve run in lockstep a single pass over the triples
@@ -26,6 +26,8 @@
 // (ddcosmo.f90:1103-1125).
 #include "ddx_device.hpp"
 #include "ddx_kernels.hpp"
+
+#include <type_traits>
 
 namespace ddx {
 namespace {
@@ -75,74 +77,204 @@ __host__ __device__ constexpr int aidx(int lmax, int m0, int m1, int l, int m, b
   return mspan(lmax, m0, m) + (m == 0 ? l : 2 * (l - m) + (neg ? 1 : 0));
 }
 
-// X' of the container in the wave's LDS row
-template <typename R>
-using LdsPtr = __attribute__((address_space(3))) const R *;
+// X' of the container, 16 values to a register: lane i holds the values 16 j + i
+// mod 16 in r[j], so that every row of 16 lanes holds them all and an FMA reads
+// value e of its row by row_newbcast.
+//   What it replaces: every lane read the values from the wave's LDS row, a
+// broadcast of 16 bytes in 8 cycles to each pair of values, so that at lmax 8
+// the eight waves of a compute unit took the LDS 2600 cycles a triple against
+// 3400 of FP64 issue, and waited for each read a few instructions later.  With
+// the values as scalars (8 or 16 to a load through the scalar cache, one load
+// ahead) the paired FP64 sweep of 2000 atoms took as long, 56 and 51 us, waiting
+// for those; without either 32.  Paired FP64 sweep, LDS -> registers, us: 60
+// atoms (lmax 6) 5.6 -> 4.7; 642 (6) 9.0 -> 6.9; 1000 (8) 34.9 -> 26.4; 2000 (8)
+// 57 -> 44.5; 1500 (10) 132 -> 108; 500 (12) 66 -> 59; 300 (16) 80 -> 70.  FP32:
+// 642 (6) 6.8 -> 5.7; 2000 (8) 36.3 -> 36.2.  What bounds the FP64 sweep now is
+// its issue (43 us at 2000 atoms with every load and store left out) and the
+// scattered stores of the terms (13 us in part under it).
+template <typename R, int NY>
+struct XRow {
+  static constexpr int NR = (NY + 15) / 16;
+  R r[NR];
+};
+__device__ __forceinline__ double fma_r(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
+__device__ __forceinline__ float fma_r(float a, float b, float c) { return fmaf(a, b, c); }
+
+// The sums of one basis value p: ap += p qc and an += p qs (the adjoint's),
+// a += x_NA p and b += x_NB p (L X), x_N the value that lane N of the row holds.
+//   A DPP read of a register must follow its last write by a vector instruction
+// by two more instructions, which the compiler does not see to inside an asm
+// block: the adjoint's FMAs come first, or waits stand in their place.
+template <int NA, int NB>
+__device__ __forceinline__ void fma4(double &ap, double &an, double &a, double &b, double p, double qc, double qs,
+                                     double xa, double xb) {
+  asm("v_fmac_f64_e32 %0, %4, %5\n\t"
+      "v_fmac_f64_e32 %1, %4, %6\n\t"
+      "v_fmac_f64_dpp %2, %7, %4 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %3, %8, %4 row_newbcast:%10 row_mask:0xf bank_mask:0xf"
+      : "+&v"(ap), "+&v"(an), "+&v"(a), "+&v"(b)
+      : "v"(p), "v"(qc), "v"(qs), "v"(xa), "v"(xb), "n"(NA), "n"(NB));
+}
+template <int NA, int NB>
+__device__ __forceinline__ void fma4(float &ap, float &an, float &a, float &b, float p, float qc, float qs,
+                                     float xa, float xb) {
+  asm("v_fmac_f32_e32 %0, %4, %5\n\t"
+      "v_fmac_f32_e32 %1, %4, %6\n\t"
+      "v_fmac_f32_dpp %2, %7, %4 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %3, %8, %4 row_newbcast:%10 row_mask:0xf bank_mask:0xf"
+      : "+&v"(ap), "+&v"(an), "+&v"(a), "+&v"(b)
+      : "v"(p), "v"(qc), "v"(qs), "v"(xa), "v"(xb), "n"(NA), "n"(NB));
+}
+template <int NA>
+__device__ __forceinline__ void fma2(double &ap, double &a, double p, double qc, double xa) {
+  asm("v_fmac_f64_e32 %0, %2, %3\n\t"
+      "s_nop 0\n\t"
+      "v_fmac_f64_dpp %1, %4, %2 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+      : "+&v"(ap), "+&v"(a)
+      : "v"(p), "v"(qc), "v"(xa), "n"(NA));
+}
+template <int NA>
+__device__ __forceinline__ void fma2(float &ap, float &a, float p, float qc, float xa) {
+  asm("v_fmac_f32_e32 %0, %2, %3\n\t"
+      "s_nop 0\n\t"
+      "v_fmac_f32_dpp %1, %4, %2 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+      : "+&v"(ap), "+&v"(a)
+      : "v"(p), "v"(qc), "v"(xa), "n"(NA));
+}
+template <int NA, int NB>
+__device__ __forceinline__ void dot2(double &a, double &b, double p, double xa, double xb) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %3, %2 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %4, %2 row_newbcast:%6 row_mask:0xf bank_mask:0xf"
+      : "+&v"(a), "+&v"(b)
+      : "v"(p), "v"(xa), "v"(xb), "n"(NA), "n"(NB));
+}
+template <int NA, int NB>
+__device__ __forceinline__ void dot2(float &a, float &b, float p, float xa, float xb) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f32_dpp %0, %3, %2 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %1, %4, %2 row_newbcast:%6 row_mask:0xf bank_mask:0xf"
+      : "+&v"(a), "+&v"(b)
+      : "v"(p), "v"(xa), "v"(xb), "n"(NA), "n"(NB));
+}
+template <int NA>
+__device__ __forceinline__ void dot1(double &a, double p, double xa) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %2, %1 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+      : "+&v"(a)
+      : "v"(p), "v"(xa), "n"(NA));
+}
+template <int NA>
+__device__ __forceinline__ void dot1(float &a, float p, float xa) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f32_dpp %0, %2, %1 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+      : "+&v"(a)
+      : "v"(p), "v"(xa), "n"(NA));
+}
+
+// f(B), f(B + 1), .., f(E - 1) with the index as a constant expression
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
+#define DDX_INLINE __attribute__((always_inline))
+
+// the sums of p = p~_lm for the two entries (l, +-m)
+template <int LMAX, bool DIR, bool ACC, int AM0, int AM1, int L, int M, typename R, int NY>
+__device__ __forceinline__ void visit(const XRow<R, NY> &X, R p, R qc, R qs, R &a, R &b, R *acc) {
+  constexpr int ea = lmi(L, M), eb = lmi(L, -M);
+  if constexpr (ACC) {
+    R &ap = acc[aidx(LMAX, AM0, AM1, L, M, false)];
+    if constexpr (M == 0) {
+      if constexpr (DIR) fma2<ea % 16>(ap, a, p, qc, X.r[ea / 16]);
+      else ap = fma_r(p, qc, ap);
+    } else {
+      R &an = acc[aidx(LMAX, AM0, AM1, L, M, true)];
+      if constexpr (DIR) {
+        fma4<ea % 16, eb % 16>(ap, an, a, b, p, qc, qs, X.r[ea / 16], X.r[eb / 16]);
+      } else {
+        ap = fma_r(p, qc, ap);
+        an = fma_r(p, qs, an);
+      }
+    }
+  } else if constexpr (DIR) {
+    if constexpr (M == 0) dot1<ea % 16>(a, p, X.r[ea / 16]);
+    else dot2<ea % 16, eb % 16>(a, b, p, X.r[ea / 16], X.r[eb / 16]);
+  }
+}
 
 // One triple: returns sum_lm p~_lm trig_m Xc'_lm when DIR and adds
 // coef p~_lm trig_m to the accumulators of AM0 <= |m| < AM1 (trig_m =
 // cos(m phi) for m >= 0, sin(|m| phi) for m < 0).  Without DIR the
 // recurrences in m only step up to AM0 before the l recurrence starts.
-template <typename R, int LMAX, bool DIR, int AM0, int AM1>
-__device__ __forceinline__ R sweep_triple(R cthe, R sthe, R cphi, R sphi, R t, LdsPtr<R> Xc, R coef,
-                                          R *acc) {
+// ct = t cos theta, st = t sin theta, t2 = t^2; coef is x0 w0 rounded, and the
+// entry (0, 0) adds the product itself.  All roundings are written out: the DIIS
+// extrapolation makes 1e-9 of a sum contracted differently.
+template <int LMAX, bool DIR, int AM0, int AM1>
+__device__ __forceinline__ double sweep_triple(double ct, double st, double t2, double cphi,
+                                               double sphi,
+                                               const XRow<double, (LMAX + 1) * (LMAX + 1)> &X,
+                                               double x0, double w0, double coef,
+                                               double *acc) {
+#pragma clang fp contract(off)
+  typedef double R;
   constexpr bool ADJ = AM0 < AM1;
   constexpr int MB = DIR ? 0 : AM0;          // first m with the l recurrence
   constexpr int ME = DIR ? LMAX + 1 : AM1;   // one past the last m needed
-  const R ct = cthe * t, st = sthe * t, t2 = t * t;
   R s = 0.0;
   R pmm = 1.0;   // t^m P_m^m
   R cm = 1.0, sm = 0.0, cprev = 0.0, sprev = 0.0;
-#pragma unroll
-  for (int m = 0; m < ME; ++m) {
-    if (m >= MB) {
-      const bool acc_m = ADJ && m >= AM0 && m < AM1;
+  static_for<0, ME>([&](auto mc) DDX_INLINE {
+    constexpr int m = decltype(mc)::value;
+    if constexpr (m >= MB) {
+      constexpr bool acc_m = ADJ && m >= AM0 && m < AM1;
       R qc = 0.0, qs = 0.0;
       if (acc_m) {
         qc = (m == 0) ? coef : coef * cm;
         qs = (m == 0) ? R(0) : coef * sm;
       }
       R a = 0.0, b = 0.0;
-      // X' of this m is read from LDS only after the previous m's sum: the
-      // compiler would otherwise keep all nylm values in registers
-      LdsPtr<R> Xm = Xc;
-      if (DIR) asm volatile("" : "+v"(Xm) : "v"(s));
-      auto visit = [&](int l, R p) {
-        if (DIR) {
-          a += p * Xm[lmi(l, m)];
-          if (m > 0) b += p * Xm[lmi(l, -m)];
-        }
-        if (acc_m) {
-          acc[aidx(LMAX, AM0, AM1, l, m, false)] += p * qc;
-          if (m > 0) acc[aidx(LMAX, AM0, AM1, l, m, true)] += p * qs;
-        }
-      };
-      R p0 = pmm;
-      visit(m, p0);
-      if (m < LMAX) {
-        R p1 = ((R)(2 * m + 1) * ct) * p0;
-        visit(m + 1, p1);
-#pragma unroll
-        for (int l = m + 2; l <= LMAX; ++l) {
+      // one m after the other: what is live stays within the registers
+      if (DIR && m > 0) asm volatile("" : "+v"(pmm) : "v"(s));
+      R p0 = 0.0, p1 = pmm;   // p~(l - 1, m), p~(l, m)
+      static_for<m, LMAX + 1>([&](auto lc) DDX_INLINE {
+        constexpr int l = decltype(lc)::value;
+        if constexpr (l == m + 1) {
+          p0 = p1;
+          p1 = ((R)(2 * m + 1) * ct) * p0;
+        } else if constexpr (l > m + 1) {
           constexpr R one = 1;
-          const R ca = (R)(2 * l - 1) * (one / (R)(l - m));
-          const R cb = (R)(l + m - 1) * (one / (R)(l - m));
-          const R p2 = ca * (ct * p1) - cb * (t2 * p0);
-          visit(l, p2);
+          constexpr R ca = (R)(2 * l - 1) * (one / (R)(l - m));
+          constexpr R cb = (R)(l + m - 1) * (one / (R)(l - m));
+          const R p2 = __builtin_fma(ca, ct * p1, -(cb * (t2 * p0)));
           p0 = p1;
           p1 = p2;
         }
-      }
-      if (DIR) s += (m == 0) ? a : (cm * a + sm * b);
+        if constexpr (l == 0) {
+          if constexpr (acc_m) acc[0] = __builtin_fma(x0, w0, acc[0]);
+          visit<LMAX, DIR, false, AM0, AM1, l, m>(X, p1, qc, qs, a, b, acc);
+        } else {
+          visit<LMAX, DIR, acc_m, AM0, AM1, l, m>(X, p1, qc, qs, a, b, acc);
+        }
+      });
+      if (DIR) s = (m == 0) ? a : s + __builtin_fma(cm, a, sm * b);
     }
-    if (m + 1 < ME) {
+    if constexpr (m + 1 < ME) {
       pmm = (-(R)(2 * m + 1) * st) * pmm;
       R cn, sn;
       if (m == 0) { cn = cphi; sn = sphi; }
-      else { cn = R(2) * cphi * cm - cprev; sn = R(2) * cphi * sm - sprev; }
+      else {
+        cn = __builtin_fma(R(2) * cphi, cm, -cprev);
+        sn = __builtin_fma(R(2) * cphi, sm, -sprev);
+      }
       cprev = cm; sprev = sm; cm = cn; sm = sn;
     }
-  }
+  });
   return s;
 }
 
@@ -165,7 +297,8 @@ __host__ __device__ constexpr double basis_beta(int l, int m) {
 // Xc holds K X' and the caller multiplies the adjoint sums by K.
 template <int LMAX, bool DIR, int AM0, int AM1>
 __device__ __forceinline__ float sweep_triple32(float ct, float st, float cphi, float sphi,
-                                                LdsPtr<float> Xc, float coef, float *acc) {
+                                                const XRow<float, (LMAX + 1) * (LMAX + 1)> &X,
+                                                float coef, float *acc) {
   constexpr bool ADJ = AM0 < AM1;
   constexpr int MB = DIR ? 0 : AM0;          // first m with the l recurrence
   constexpr int ME = DIR ? LMAX + 1 : AM1;   // one past the last m needed
@@ -173,50 +306,30 @@ __device__ __forceinline__ float sweep_triple32(float ct, float st, float cphi, 
   float s = 0.0f;
   float qmm = 1.0f;
   float cm = 1.0f, sm = 0.0f, cprev = 0.0f, sprev = 0.0f;
-#pragma unroll
-  for (int m = 0; m < ME; ++m) {
-    if (m >= MB) {
-      const bool acc_m = ADJ && m >= AM0 && m < AM1;
+  static_for<0, ME>([&](auto mc) DDX_INLINE {
+    constexpr int m = decltype(mc)::value;
+    if constexpr (m >= MB) {
+      constexpr bool acc_m = ADJ && m >= AM0 && m < AM1;
       float qc = 0.0f, qs = 0.0f;
       if (acc_m) {
         qc = (m == 0) ? coef : coef * cm;
         qs = (m == 0) ? 0.0f : coef * sm;
       }
       float a = 0.0f, b = 0.0f;
-      LdsPtr<float> Xm = Xc;
-      if (DIR) asm volatile("" : "+v"(Xm) : "v"(s));
-      auto visit = [&](int l, float q) {
-        if (DIR) {
-          if (l == m) {
-            a = q * Xm[lmi(l, m)];
-            if (m > 0) b = q * Xm[lmi(l, -m)];
-          } else {
-            a = fmaf(q, Xm[lmi(l, m)], a);
-            if (m > 0) b = fmaf(q, Xm[lmi(l, -m)], b);
-          }
-        }
-        if (acc_m) {
-          float &ap = acc[aidx(LMAX, AM0, AM1, l, m, false)];
-          ap = fmaf(q, qc, ap);
-          if (m > 0) {
-            float &an = acc[aidx(LMAX, AM0, AM1, l, m, true)];
-            an = fmaf(q, qs, an);
-          }
-        }
-      };
-      float q0 = qmm;
-      visit(m, q0);
-      if (m < LMAX) {
-        float q1 = ct * q0;
-        visit(m + 1, q1);
-#pragma unroll
-        for (int l = m + 2; l <= LMAX; ++l) {
+      if (DIR && m > 0) asm volatile("" : "+v"(qmm) : "v"(s));
+      float q0 = 0.0f, q1 = qmm;   // q(l - 1, m), q(l, m)
+      static_for<m, LMAX + 1>([&](auto lc) DDX_INLINE {
+        constexpr int l = decltype(lc)::value;
+        if constexpr (l == m + 1) {
+          q0 = q1;
+          q1 = ct * q0;
+        } else if constexpr (l > m + 1) {
           const float q2 = fmaf(-(float)basis_beta(l, m), t2 * q0, ct * q1);
-          visit(l, q2);
           q0 = q1;
           q1 = q2;
         }
-      }
+        visit<LMAX, DIR, acc_m, AM0, AM1, l, m>(X, q1, qc, qs, a, b, acc);
+      });
       if (DIR) {
         if (m == 0) {
           s = a;
@@ -226,7 +339,7 @@ __device__ __forceinline__ float sweep_triple32(float ct, float st, float cphi, 
         }
       }
     }
-    if (m + 1 < ME) {
+    if constexpr (m + 1 < ME) {
       qmm = st * qmm;
       float cn, sn;
       if (m == 0) {
@@ -238,7 +351,7 @@ __device__ __forceinline__ float sweep_triple32(float ct, float st, float cphi, 
       }
       cprev = cm; sprev = sm; cm = cn; sm = sn;
     }
-  }
+  });
   return s;
 }
 
@@ -258,18 +371,18 @@ struct Geo<float> {
 };
 
 // One pass over triples beg..end-1 (end > beg) of a container: rw[tslot] =
-// W (R . X_c) when DIR (X' in xsh), and when AM0 < AM1 the (l, +-m),
+// W (R . X_c) when DIR, and when AM0 < AM1 the (l, +-m),
 // AM0 <= m < AM1, entries of the chunk's share of (L*S)_c, -cf * sum_t w_n
 // xi(n, o) W p~ trig, into the segment row yp.  The FP32 pass works on the
-// scaled basis of sweep_triple32: xsh holds K X' and the sums are scaled by
+// scaled basis of sweep_triple32: X holds K X' and the sums are scaled by
 // cf K (the table after cf, 1/(l+1), 1/facl and K in cf).
 template <typename R, int LMAX, bool DIR, int AM0, int AM1>
 __device__ __forceinline__ void sweep_pass(
     int beg, int end, const typename Geo<R>::G4 *__restrict__ tgeo,
     const typename Geo<R>::G2 *__restrict__ ttw,
-    const int *__restrict__ tslot, const int *__restrict__ tp, LdsPtr<R> xsh,
-    R *__restrict__ rw, int spare, const R *__restrict__ xiw, const double *__restrict__ cf,
-    double *__restrict__ yp) {
+    const int *__restrict__ tslot, const int *__restrict__ tp, const XRow<R, (LMAX + 1) * (LMAX + 1)> &X,
+    R *__restrict__ rw, int spare, const R *__restrict__ xiw,
+    const double *__restrict__ cf, double *__restrict__ yp) {
   constexpr bool F = sizeof(R) == 4;
   constexpr bool ADJ = AM0 < AM1;
   constexpr int NA = ADJ ? mspan(LMAX, AM0, AM1) : 1;
@@ -313,7 +426,7 @@ __device__ __forceinline__ void sweep_pass(
       if constexpr (ADJ) nxt.x = xiw[nxt.p];
       const bool live = k < end;
       const R coef = ADJ ? (live ? cur.x * cur.w : R(0)) : R(0);
-      const R v = sweep_triple32<LMAX, DIR, AM0, AM1>(cur.g.x, cur.g.y, cur.g.z, cur.g.w, xsh,
+      const R v = sweep_triple32<LMAX, DIR, AM0, AM1>(cur.g.x, cur.g.y, cur.g.z, cur.g.w, X,
                                                       coef, acc);
       if constexpr (DIR) rw[live ? cur.s : spare] = cur.w * v;
       k += kWave;
@@ -330,49 +443,46 @@ __device__ __forceinline__ void sweep_pass(
       if (it + 1 < nit) step(B, C, A);
     }
   } else {
-    // FP64: loads under their bounds tests, stages copied down after each
-    // triple (the passes of lmax >= 8 need the registers a third stage takes)
-    G4 z4;
-    z4.x = z4.y = z4.z = z4.w = R(0);
-    G2 z2;
-    z2.x = z2.y = R(0);
-    G4 g0 = z4, g1 = z4;
-    G2 w0 = z2, w1 = z2;
-    int s0 = 0, s1 = 0, p1 = 0;
-    R x0 = R(0);
-    if (k < end) {
-      g0 = tgeo[k];
-      w0 = ttw[k];
-      if (DIR) s0 = tslot[k];
-      if (ADJ) x0 = xiw[tp[k]];
+    // Indices past the chunk as in FP32.  One stage of registers: the triple's
+    // values leave the loaded registers first, then the loads of the next
+    // triple go into these and are waited for a whole evaluation later.  (A loop
+    // that copied stages down, with its loads under bounds tests, waited for
+    // them in the iteration that issued them.)
+    const int last = end - 1;
+    const int k0 = min(k, last);
+    G4 g = tgeo[k0];
+    G2 w = ttw[k0];
+    int slot = 0, pn = 0;
+    R x = R(0);
+    if constexpr (DIR) slot = tslot[k0];
+    if constexpr (ADJ) {
+      x = xiw[tp[k0]];
+      pn = tp[min(k + kWave, last)];
     }
-    if (k + kWave < end) {
-      g1 = tgeo[k + kWave];
-      w1 = ttw[k + kWave];
-      if (DIR) s1 = tslot[k + kWave];
-      if (ADJ) p1 = tp[k + kWave];
-    }
-    for (; k < end; k += kWave) {
-      const int k2 = k + 2 * kWave;
-      G4 g2 = z4;
-      G2 w2 = z2;
-      int s2 = 0, p2 = 0;
-      if (k2 < end) {
-        g2 = tgeo[k2];
-        w2 = ttw[k2];
-        if (DIR) s2 = tslot[k2];
-        if (ADJ) p2 = tp[k2];
+    for (int it = (end - beg + kWave - 1) / kWave; it > 0; --it) {
+      const bool live = k < end;
+      R ct = g.x * w.x, st = g.y * w.x, t2 = w.x * w.x;
+      R cphi, sphi, wt, x0 = R(0);
+      int at = 0;
+      asm volatile("v_mov_b64_e32 %0, %1" : "=&v"(cphi) : "v"(g.z));
+      asm volatile("v_mov_b64_e32 %0, %1" : "=&v"(sphi) : "v"(g.w));
+      asm volatile("v_mov_b64_e32 %0, %1" : "=&v"(wt) : "v"(w.y));
+      if constexpr (DIR) at = live ? slot : spare;
+      if constexpr (ADJ) x0 = live ? x : R(0);
+      R coef = x0 * wt;
+      asm volatile("" : "+v"(ct), "+v"(st), "+v"(t2), "+v"(x0), "+v"(coef), "+v"(at));
+      const int j = min(k + kWave, last);
+      g = tgeo[j];
+      w = ttw[j];
+      if constexpr (DIR) slot = tslot[j];
+      if constexpr (ADJ) {
+        x = xiw[pn];
+        pn = tp[min(k + 2 * kWave, last)];
       }
-      R x1 = R(0);
-      if (ADJ && k + kWave < end) x1 = xiw[p1];
-      const R coef = ADJ ? x0 * (R)w0.y : R(0);
-      const R v = sweep_triple<R, LMAX, DIR, AM0, AM1>((R)g0.x, (R)g0.y, (R)g0.z, (R)g0.w,
-                                                       (R)w0.x, xsh, coef, acc);
-      if (DIR) rw[s0] = (R)w0.y * v;
-      g0 = g1; g1 = g2;
-      w0 = w1; w1 = w2;
-      s0 = s1; s1 = s2;
-      x0 = x1; p1 = p2;
+      __builtin_amdgcn_sched_barrier(0);
+      const R v = sweep_triple<LMAX, DIR, AM0, AM1>(ct, st, t2, cphi, sphi, X, x0, wt, coef, acc);
+      if constexpr (DIR) rw[at] = wt * v;
+      k += kWave;
     }
   }
   if constexpr (ADJ) {
@@ -408,15 +518,15 @@ template <typename R, int LMAX, bool DIR, int B>
 __device__ __forceinline__ void sweep_blocks(
     int beg, int end, const typename Geo<R>::G4 *__restrict__ tgeo,
     const typename Geo<R>::G2 *__restrict__ ttw,
-    const int *__restrict__ tslot, const int *__restrict__ tp, LdsPtr<R> xsh,
-    R *__restrict__ rw, int spare, const R *__restrict__ xiw, const double *__restrict__ cf,
-    double *__restrict__ yp) {
+    const int *__restrict__ tslot, const int *__restrict__ tp, const XRow<R, (LMAX + 1) * (LMAX + 1)> &X,
+    R *__restrict__ rw, int spare, const R *__restrict__ xiw,
+    const double *__restrict__ cf, double *__restrict__ yp) {
   constexpr bool F = sizeof(R) == 4;
   constexpr int M0 = mblock_begin(LMAX, DIR, B, F), M1 = mblock_begin(LMAX, DIR, B + 1, F);
-  sweep_pass<R, LMAX, DIR && B == 0, M0, M1>(beg, end, tgeo, ttw, tslot, tp, xsh, rw, spare, xiw,
-                                             cf, yp);
+  sweep_pass<R, LMAX, DIR && B == 0, M0, M1>(beg, end, tgeo, ttw, tslot, tp, X, rw, spare,
+                                             xiw, cf, yp);
   if constexpr (M1 <= LMAX) sweep_blocks<R, LMAX, DIR, B + 1>(beg, end, tgeo, ttw, tslot, tp,
-                                                             xsh, rw, spare, xiw, cf, yp);
+                                                             X, rw, spare, xiw, cf, yp);
 }
 
 // Triples beg..end-1 of container c: rw[tslot] = W (R . X_c) when DIR
@@ -430,23 +540,20 @@ __device__ __forceinline__ void sweep_chunk(
     R *__restrict__ rw, int spare, const R *__restrict__ xiw, const double *__restrict__ cf,
     double *__restrict__ yp) {
   constexpr int NY = (LMAX + 1) * (LMAX + 1);
-  // X'_c in the wave's LDS row (rounded to R; K X' in FP32, for the scaled
-  // basis of sweep_triple32): every lane reads the same word (broadcast)
-  __shared__ R xsh_all[kSweepWaves][DIR ? NY : 1];
-  R *xsh = xsh_all[__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave))];
-  if (DIR) {
-    wave_lds_sync();   // reads of the previous segment's X' are done
-    for (int k = lane_id(); k < NY; k += kWave) {
+  // (rounded to R; K X' in FP32, for the scaled basis of sweep_triple32)
+  XRow<R, NY> X;
+  if constexpr (DIR) {
+#pragma unroll
+    for (int j = 0; j < XRow<R, NY>::NR; ++j) {
+      const int k = min(16 * j + (lane_id() & 15), NY - 1);
       const double x = Xs[(size_t)c * NY + k];
-      xsh[k] = sizeof(R) == 4 ? (R)(x * cf[3 * NY + k]) : (R)x;
+      X.r[j] = sizeof(R) == 4 ? (R)(x * cf[3 * NY + k]) : (R)x;
     }
-    wave_lds_sync();
   }
-  const LdsPtr<R> xl = (LdsPtr<R>)xsh;
   if constexpr (ADJ)
-    sweep_blocks<R, LMAX, DIR, 0>(beg, end, tgeo, ttw, tslot, tp, xl, rw, spare, xiw, cf, yp);
+    sweep_blocks<R, LMAX, DIR, 0>(beg, end, tgeo, ttw, tslot, tp, X, rw, spare, xiw, cf, yp);
   else
-    sweep_pass<R, LMAX, true, 0, 0>(beg, end, tgeo, ttw, tslot, tp, xl, rw, spare, xiw, cf, yp);
+    sweep_pass<R, LMAX, true, 0, 0>(beg, end, tgeo, ttw, tslot, tp, X, rw, spare, xiw, cf, yp);
 }
 
 // One wave per worker w (kSweepWaves to a workgroup, w < G): units
@@ -586,6 +693,7 @@ __device__ __forceinline__ void p2l_pass(int i, double4 si, double rc2, int sb, 
                                          const double *__restrict__ cf, double *__restrict__ A) {
   constexpr int NA = mspan(P, AM0, AM1);
   constexpr int NY = (P + 1) * (P + 1);
+  const XRow<double, NY> none{};
   double acc[NA];
 #pragma unroll
   for (int k = 0; k < NA; ++k) acc[k] = 0.0;
@@ -611,7 +719,7 @@ __device__ __forceinline__ void p2l_pass(int i, double4 si, double rc2, int sb, 
         sphi = vy / rxy;
       }
     }
-    sweep_triple<double, P, false, AM0, AM1>(cthe, sthe, cphi, sphi, t, nullptr, coef, acc);
+    sweep_triple<P, false, AM0, AM1>(cthe * t, sthe * t, t * t, cphi, sphi, none, coef, 1.0, coef, acc);
   }
   int base = 0, len = NA;
   wave_reduce_split<0, NA, double>(acc, base, len);

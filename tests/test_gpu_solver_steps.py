@@ -22,6 +22,10 @@
   points against the definition evaluated here, and the triple lists, which
   the two operators read in different orders, by <u, L v> = <L* u, v> (1e-12
   of |u| |L v|: sums of up to 1e6 terms, rounding 1e-16 each).
+* test_operators_at_every_lmax: the sweeps hold X' in rows of 16 values and their
+  sums in blocks that depend on lmax, so L and L* are checked against the oracle
+  at each one, 1e-12 in FP64; in FP32 the basis recurrences of lmax steps over
+  (lmax + 1)^2 values lose up to their product in ulps.
 * test_field_at_tile_edges, test_potential_at_tile_edges: the Coulomb sums
   where a tile of 64 targets, a block of 64 sources or a chunk of sources ends,
   against the sums written out here (1e-12 of the sum of the terms' sizes: a
@@ -120,6 +124,21 @@ def test_setup_at_its_branches(n, ngrid):
     u, v = rng.standard_normal((2, n, 16))
     lv, lu = h.lx(v), h.lstarx(u)
     assert abs((u * lv).sum() - (lu * v).sum()) <= 1e-12 * np.linalg.norm(u) * np.linalg.norm(lv)
+
+
+@pytest.mark.parametrize("lmax", range(17))
+def test_operators_at_every_lmax(oracle_mod, lmax):
+    from ddpcm_amd.ddx import DDCosmo
+    from ddpcm_amd.inputs import synthetic_input
+    x, y, z, r = synthetic_input(7, 3, lmax, 302).bohr()
+    h = DDCosmo(x, y, z, r, lmax, 302)
+    o = oracle_mod.Oracle(x, y, z, r, lmax, 302)
+    v = np.random.default_rng(lmax).standard_normal((7, h.nylm))
+    ref = o.lx(v), o.lstarx(v)
+    for mixed, tol in ((0, 1e-12), (1, 6e-8 * (lmax + 1) ** 3 + 1e-6)):
+        h.set_precision(mixed)
+        for got, want in zip((h.lx(v), h.lstarx(v)), ref):
+            assert np.linalg.norm(got - want) <= tol * np.linalg.norm(want)
 
 
 def _coulomb(q, s, t):
