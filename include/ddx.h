@@ -314,7 +314,8 @@ int ddx_set_graphs(ddx_handle *h, int enable);
 #define DDX_K_PROJECT 2      /* MFMA projection onto harmonics           */
 #define DDX_K_EXPAND 3       /* MFMA expansion on the grid (xi)          */
 #define DDX_K_JACOBI 4       /* Jacobi update + DIIS Gram row            */
-#define DDX_K_DIIS 5         /* DIIS bordered solve                      */
+#define DDX_K_DIIS 5         /* DIIS bordered solve (small systems: and  */
+                             /* the extrapolation, in one launch)        */
 #define DDX_K_EXTRAP 6       /* DIIS extrapolation + increment norm      */
 #define DDX_K_FIELD 7        /* all-pairs field                          */
 #define DDX_K_POTENTIAL 8    /* all-pairs potential                      */
