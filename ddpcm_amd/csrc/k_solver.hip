@@ -554,6 +554,10 @@ __device__ __forceinline__ double border(const double *bs, int off, int r, int c
 // pivoted column holds the in-place inverse, which neither later pivots nor
 // the solution read: it becomes zero, which is never a pivot, and stays zero,
 // the pivot rows' entries being zero there too.
+//   NaN is never a pivot (it compares with nothing in the reference's search; the
+// largest of a lane's values leaves it out, and a lane that has nothing else
+// takes no part), and once nothing else is left the system is singular: the
+// iteration keeps the Jacobi step and DIIS starts again.
 //   The pivot row reaches the other lanes through LDS (in issue order within
 // the wave, no barrier).  The update a - pc * dum keeps the reference's two
 // roundings: `keep` is 1, and 0 with dum = -1 on the pivot row, whose result
@@ -598,7 +602,7 @@ __device__ __forceinline__ bool eliminate(const double *bs, int off, int nmat, d
     for (int w = 2; w < J; w *= 2)
 #pragma unroll
       for (int j = 0; j + w < J; j += 2 * w) m[j] = max_abs(m[j], m[j + w]);
-    const double big = rowlive ? m[0] : 0.0;
+    const double big = rowlive && m[0] > 0.0 ? m[0] : 0.0;   // (NaN: no candidate)
     int jc = 0;
 #pragma unroll
     for (int j = J - 1; j >= 0; --j) jc = (fabs(g[j]) == big) ? j : jc;
