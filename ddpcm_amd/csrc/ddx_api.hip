@@ -318,6 +318,7 @@ int pipeline(ddx_handle *h) {
 
 // (its time is read once the events have passed: here nothing waits)
 int timed_setup(ddx_handle *h) {
+  h->setup_timed = false;
   DDX_HIP(hipEventRecord(h->ev[0], h->stream));
   DDX_TRY(run_setup(h));
   DDX_HIP(hipEventRecord(h->ev[6], h->stream));
@@ -579,6 +580,8 @@ int ddx_get_array(const ddx_handle *hc, const char *name, double *dst) {
   }
   const double *src = nullptr;
   size_t cnt = 0;
+  if (!strcmp(name, "fi") || !strcmp(name, "ui") || !strcmp(name, "zi") || !strcmp(name, "ccav"))
+    DDX_TRY(lists_ready(h, "ddx_get_array"));
   if (!strcmp(name, "fi")) { src = h->fi.p; cnt = np; }
   else if (!strcmp(name, "ui")) { src = h->ui.p; cnt = np; }
   else if (!strcmp(name, "zi")) {
@@ -610,6 +613,7 @@ int ddx_get_array(const ddx_handle *hc, const char *name, double *dst) {
 int ddx_get_neighbours(const ddx_handle *hc, int *inl, int *nl) {
   ddx_handle *h = const_cast<ddx_handle *>(hc);
   if (!h || !inl || !nl) return DDX_ERR_ARG;
+  DDX_TRY(lists_ready(h, "ddx_get_neighbours"));
   DDX_HIP(hipMemcpyAsync(inl, h->inl.p, (h->n + 1) * sizeof(int), hipMemcpyDeviceToHost, h->stream));
   if (h->nnl)
     DDX_HIP(hipMemcpyAsync(nl, h->nl.p, h->nnl * sizeof(int), hipMemcpyDeviceToHost, h->stream));
@@ -621,6 +625,7 @@ int ddx_get_neighbours(const ddx_handle *hc, int *inl, int *nl) {
 
 int ddx_mkrhs(ddx_handle *h, const double *charge, double *phi, double *psi) {
   if (!h || !charge || !phi || !psi) return DDX_ERR_ARG;
+  DDX_TRY(lists_ready(h, "ddx_mkrhs"));
   DDX_TRY(reserve_vectors(h));
   DDX_TRY(stage_inputs(h, nullptr, nullptr, nullptr, nullptr, charge));
   DDX_TRY(h->phi.reserve((size_t)h->ncav + 1));
@@ -667,6 +672,7 @@ int ddx_cosmo(ddx_handle *h, int star, int cart, const double *phi, const double
               const double *psi, double *sigma, double *esolv) {
   if (!h || !psi || !sigma) return DDX_ERR_ARG;
   DDX_TRY(single(h, "ddx_cosmo"));
+  DDX_TRY(lists_ready(h, "ddx_cosmo"));
   h->results_ok = false;
   hipStream_t s = h->stream;
   size_t nn = (size_t)h->nylm * h->n;
@@ -698,6 +704,7 @@ int ddx_cosmo(ddx_handle *h, int star, int cart, const double *phi, const double
 int ddx_forces_dd(ddx_handle *h, const double *phi, const double *sigma, const double *s_adj,
                   double *fx) {
   if (!h || !phi || !sigma || !s_adj || !fx) return DDX_ERR_ARG;
+  DDX_TRY(lists_ready(h, "ddx_forces_dd"));
   h->results_ok = false;
   hipStream_t s = h->stream;
   size_t nn = (size_t)h->nylm * h->n;
@@ -712,6 +719,7 @@ int ddx_forces_dd(ddx_handle *h, const double *phi, const double *sigma, const d
 
 int ddx_mkzeta(ddx_handle *h, const double *s_adj, double *zeta) {
   if (!h || !s_adj || !zeta) return DDX_ERR_ARG;
+  DDX_TRY(lists_ready(h, "ddx_mkzeta"));
   hipStream_t s = h->stream;
   DDX_TRY(reserve_vectors(h));
   DDX_TRY(upload(h->s, s_adj, (size_t)h->nylm * h->n, s));
@@ -738,6 +746,7 @@ int ddx_efld(ddx_handle *h, int nsrc, const double *src, const double *csrc, int
 
 static int op_apply(ddx_handle *h, int which, const double *x, double *y) {
   if (!h || !x || !y) return DDX_ERR_ARG;
+  if (which < 2) DDX_TRY(lists_ready(h, which ? "ddx_lstarx" : "ddx_lx"));
   hipStream_t s = h->stream;
   size_t nn = (size_t)h->nylm * h->n;
   DDX_TRY(reserve_vectors(h));
@@ -775,6 +784,7 @@ int ddx_jacobi_diis(ddx_handle *h, int star, int diis_max, double tol, const dou
                     double *x, int *n_iter, int *ok) {
   if (!h || !rhs || !x || !n_iter || !ok) return DDX_ERR_ARG;
   DDX_TRY(single(h, "ddx_jacobi_diis"));
+  DDX_TRY(lists_ready(h, "ddx_jacobi_diis"));
   hipStream_t s = h->stream;
   size_t nn = (size_t)h->nylm * h->n;
   DDX_TRY(reserve_vectors(h));

@@ -215,6 +215,7 @@ struct ddx_handle {
   int ncav = 0, nnl = 0, ntri = 0, maxdeg = 0;
   bool have_setup = false, have_sigma = false, have_s = false, have_charge = false;
   bool conv_sigma = false, conv_s = false;   // the last solutions converged
+  bool have_lists = false;   // the setup's lists are whole: one that fails leaves them half made
 
   hipStream_t stream = nullptr;
   hipEvent_t ev[10] = {};

@@ -26,6 +26,9 @@ int scan_exclusive(const int *in, int *out, size_t n, DevArray<int> &tmp,
 
 // k_setup.hip — ddinit on the device (ddcosmo.f90:308-468)
 int run_setup(ddx_handle *h);
+// DDX_ERR_STATE where the handle's last setup failed, for every call that
+// walks its lists; `what` names the call
+int lists_ready(const ddx_handle *h, const char *what);
 
 // k_gemm.hip — FP64 MFMA products with the harmonic tables
 // y(lm, i) = alpha sum_n Yw(lm, n) P(n, i), as ysplit partial sums over

@@ -740,6 +740,7 @@ int ddx_guess_train(ddx_handle *h, int steps, double lr, double *loss) {
     set_error("ddx_guess_train needs a converged solve on the handle");
     return DDX_ERR_STATE;
   }
+  DDX_TRY(lists_ready(h, "ddx_guess_train"));
   double l[2] = {0.0, 0.0};
   DDX_TRY(train_guess(h, 0, h->rhs.p, h->sigma.p, steps, lr, &l[0]));
   if (h->have_s && h->conv_s) DDX_TRY(train_guess(h, 1, h->psi.p, h->s.p, steps, lr, &l[1]));

@@ -547,8 +547,15 @@ __global__ void k_cav_offsets(int ninst, int runs, const int *__restrict__ soff,
 
 }  // namespace
 
+int lists_ready(const ddx_handle *h, const char *what) {
+  if (h->have_lists) return DDX_OK;
+  set_error("%s: the setup of the handle's geometry failed; upload another one and run it", what);
+  return DDX_ERR_STATE;
+}
+
 int run_setup(ddx_handle *h) {
   hipStream_t s = h->stream;
+  h->have_setup = h->have_lists = false;
   int n = h->n, ng = h->ngrid;
   size_t np = (size_t)n * ng;
   h->np = np;
@@ -649,13 +656,14 @@ int run_setup(ddx_handle *h) {
     DDX_TRY(scan_arrays(sums, 4, h->scan_tmp, s));
   }
   // the cavity offset of each instance, read back with the counts
+  std::vector<int> cavoff;
   if (h->ninst > 1) {
     DDX_TRY(h->cavoff.reserve((size_t)h->ninst + 1));
     hipLaunchKernelGGL(k_cav_offsets, dim3((h->ninst + 256) / 256), dim3(256), 0, s, h->ninst,
                        runs, h->soff.p, h->cavrun.p, h->cavoff.p);
     DDX_HIP(hipGetLastError());
-    h->h_cavoff.resize(h->ninst + 1);
-    DDX_HIP(hipMemcpyAsync(h->h_cavoff.data(), h->cavoff.p, (h->ninst + 1) * sizeof(int),
+    cavoff.resize(h->ninst + 1);
+    DDX_HIP(hipMemcpyAsync(cavoff.data(), h->cavoff.p, (h->ninst + 1) * sizeof(int),
                            hipMemcpyDeviceToHost, s));
   }
   DDX_HIP(hipStreamSynchronize(s));
@@ -671,6 +679,7 @@ int run_setup(ddx_handle *h) {
   h->ntri = ntri;
   h->ncav = ncav;
   h->nunit = nunit;
+  if (h->ninst > 1) h->h_cavoff.swap(cavoff);
   // workers: whole multiples of the R = 8 per CU one-wave workgroups that
   // the FP64 sweeps keep resident (two waves per SIMD; the lmax 6 FP32 sweep
   // holds four), as many as give about
@@ -736,7 +745,7 @@ int run_setup(ddx_handle *h) {
   }
   if (h->ninst == 1) h->h_cavoff.assign({0, ncav});
   DDX_TRY(build_coulomb_tiles(h));
-  h->have_setup = true;
+  h->have_setup = h->have_lists = true;
   h->stats.ntriples = ntri;
   h->stats.nnl = nnl;
   h->stats.ncav = ncav;

@@ -179,7 +179,10 @@ int ddx_energy_forces(ddx_handle *h, const double *charge, double *esolv,
  * ddx_energy_forces so that a caller can keep inputs in HBM).
  * ddx_upload copies coordinates (bohr), radii and charges to the device;
  * ddx_run repeats setup (neighbours, fi/ui/zi, cavity), RHS, both solves
- * and the forces from them; ddx_result copies E and F back. */
+ * and the forces from them; ddx_result copies E and F back.  After a setup
+ * that fails (DDX_ERR_CAPACITY) the calls that need the setup's arrays return
+ * DDX_ERR_STATE until another geometry has been uploaded and run; the last
+ * results stay. */
 int ddx_upload(ddx_handle *h, const double *x, const double *y,
                const double *z, const double *rvdw, const double *charge);
 int ddx_run(ddx_handle *h);

@@ -7,7 +7,13 @@
   therefore follow the plain Jacobi iteration, done here with the oracle's
   operators; 1e-11 of the iterate's size for nine steps of operators that agree
   to 1e-12.
+* test_failed_setup_is_refused: after a geometry whose setup failed (a sphere
+  with more than 64 neighbours) every call that walks the setup's lists, which
+  are half made then, is refused; the sizes and the last results stay; the next
+  good geometry gives a fresh handle's results, bit for bit.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -37,3 +43,64 @@ def test_nan_residuals_reset_diis(oracle_mod, n, lmax, ngrid, star):
         v = facl * (far - op(v))
     far = slice(n // 2, n)
     assert np.max(np.abs(got[far] - v[far])) <= 1e-11 * np.max(np.abs(v))
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_failed_setup_is_refused(batch):
+    from ddpcm_amd.ddx import DDCosmo, DDCosmoBatch, DDXError
+    from ddpcm_amd.inputs import synthetic_input
+    n = 80
+    d = synthetic_input(n, 3, 4, 50)
+    x, y, z, r = d.bohr()
+    q = d.charge
+    copies = 2 if batch else 1
+
+    def new():
+        if batch:
+            return DDCosmoBatch([x] * 2, [y] * 2, [z] * 2, [r] * 2, 4, 50)
+        return DDCosmo(x, y, z, r, 4, 50)
+
+    def upload(v, scale):
+        v.upload(*[np.tile(a, copies) for a in (scale * x, scale * y, scale * z, r, q)])
+
+    h = new()
+    upload(h, 1.0)
+    h.run()
+    before = h.result()
+    sigma = h.get("sigma")
+    v = np.ones((copies * n, h.nylm))
+    cav = np.zeros(h.ncav)
+    upload(h, 0.01)   # all spheres within one another: 79 neighbours each
+    with pytest.raises(DDXError) as e:
+        h.run()
+    assert e.value.code == 4
+    calls = [lambda: h.lx(v), lambda: h.lstarx(v), lambda: h.mkrhs(np.tile(q, copies)),
+             lambda: h.forces_dd(cav, v, v), lambda: h.ddmkzeta(v), lambda: h.neighbours(),
+             lambda: h.guess_train(1)]
+    calls += [lambda a=a: h.get(a) for a in ("fi", "ui", "zi", "ccav")]
+    if not batch:
+        calls += [lambda: h.cosmo(False, phi=cav, psi=v), lambda: h.cosmo(True, psi=v),
+                  lambda: h.jacobi_diis(False, v, v)]
+    for call in calls:
+        with pytest.raises(DDXError) as e:
+            call()
+        assert e.value.code == 6 and "setup" in str(e.value)
+    with pytest.raises(DDXError) as e:   # sets up again, and meets the same error
+        h.energy_forces([q] * 2 if batch else q)
+    assert e.value.code == 4
+    h.stats()
+    for old, now in zip(before, h.result()):
+        assert np.array_equal(old, now)
+    assert np.array_equal(sigma, h.get("sigma"))
+    if batch:
+        off = np.zeros(3, dtype=np.int32)
+        h._check(h.L.ddx_batch_sizes(h.h, None, None, off.ctypes.data_as(C.POINTER(C.c_int))))
+        assert np.array_equal(off, h.cav_off)
+    upload(h, 1.01)
+    h.run()
+    f = new()
+    upload(f, 1.01)
+    f.run()
+    for a, b in zip(h.result(), f.result()):
+        assert np.array_equal(a, b)
+    assert np.array_equal(h.lx(v), f.lx(v))
