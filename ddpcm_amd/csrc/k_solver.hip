@@ -1719,9 +1719,11 @@ int solve_end(ddx_handle *h, Lane &ln, int *n_iter, int *ok, std::vector<double>
 }
 
 namespace {
+// (an acquire, against the device's fence ahead of its store: the record's
+// other values are read after it)
 bool lanes_done(Lane *const *lanes, int count) {
   for (int k = 0; k < count; ++k)
-    if (!*(volatile int *)&lanes[k]->h_diis->done) return false;
+    if (!__atomic_load_n(&lanes[k]->h_diis->done, __ATOMIC_ACQUIRE)) return false;
   return true;
 }
 

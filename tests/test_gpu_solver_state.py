@@ -11,6 +11,9 @@
   with more than 64 neighbours) every call that walks the setup's lists, which
   are half made then, is refused; the sizes and the last results stay; the next
   good geometry gives a fresh handle's results, bit for bit.
+* test_solve_records: solves of different lengths in turn on one handle, so that a
+  value read from the record of the solve before would show: iteration counts,
+  flags and all norms equal those of the same solve made first.
 """
 import ctypes as C
 
@@ -104,3 +107,27 @@ def test_failed_setup_is_refused(batch):
     for a, b in zip(h.result(), f.result()):
         assert np.array_equal(a, b)
     assert np.array_equal(h.lx(v), f.lx(v))
+
+
+def test_solve_records():
+    from ddpcm_amd.ddx import DDCosmo
+    from ddpcm_amd.inputs import synthetic_input
+    x, y, z, r = synthetic_input(20, 8, 2, 26).bohr()
+    h = DDCosmo(x, y, z, r, 2, 26)
+    rhs = np.random.default_rng(2).standard_normal((20, h.nylm))
+    x0 = h.get("facl")[None, :] * rhs
+
+    def solve(star, tol, cap):
+        _, it, ok = h.jacobi_diis(star, rhs, x0, tol=tol, n_iter=cap)
+        return it, ok, h.history(star)
+
+    kinds = [(star, tol, cap) for star in (0, 1)
+             for tol, cap in ((1e-12, 200), (1e-2, 200), (1e-12, 3), (1e-6, 200))]
+    first = [solve(*k) for k in kinds]
+    assert len({f[0] for f in first}) >= 4
+    for it, ok, hist in first:
+        assert hist.size == (it if ok else it - 1)
+    rng = np.random.default_rng(4)
+    for k in rng.integers(len(kinds), size=300):
+        it, ok, hist = solve(*kinds[k])
+        assert (it, ok) == first[k][:2] and np.array_equal(hist, first[k][2])
