@@ -14,6 +14,17 @@
 * test_solve_records: solves of different lengths in turn on one handle, so that a
   value read from the record of the solve before would show: iteration counts,
   flags and all norms equal those of the same solve made first.
+* test_two_launch_solver_equals_batch_of_two, test_two_launch_solver_short_histories:
+  single systems whose DIIS and extrapolation are two latency-ordered launches
+  (more spheres than two a compute unit; the extrapolation's launches are
+  counted, so that a size that takes another path fails).  Both solutions equal
+  the general kernels', which a batch takes, bit for bit (a sweep worker has at
+  most one unit at these sizes, so the operators' sums are split alike), at one
+  and several elements a thread.  14 points do not resolve lmax 6 and 16: there
+  the iteration, the reference's too, wanders on, and the iterates after all 200
+  steps are compared, past many drops of the oldest vectors.  Shorter histories, whose later slots do not
+  exist, give the same solution (1e-10 in the h^-1/2 norm for increments below
+  1e-12).
 """
 import ctypes as C
 
@@ -131,3 +142,52 @@ def test_solve_records():
     for k in rng.integers(len(kinds), size=300):
         it, ok, hist = solve(*kinds[k])
         assert (it, ok) == first[k][:2] and np.array_equal(hist, first[k][2])
+
+
+def _two_launches(h):
+    """Whether the solve just timed had launches of the extrapolation alone."""
+    return h.kernel_timer_read("extrap")[0] > 0
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+@pytest.mark.parametrize("n,lmax,ngrid", [(601, 0, 26), (600, 2, 26), (901, 6, 14), (700, 16, 14)])
+def test_two_launch_solver_equals_batch_of_two(n, lmax, ngrid, mixed):
+    from ddpcm_amd.ddx import DDCosmo, DDCosmoBatch, NotConverged
+    from ddpcm_amd.inputs import synthetic_input
+    d = synthetic_input(n, 77 + n, lmax, ngrid)
+    x, y, z, r = d.bohr()
+    h = DDCosmo(x, y, z, r, lmax, ngrid)
+    b = DDCosmoBatch([x, x], [y, y], [z, z], [r, r], lmax, ngrid)
+    for v in (h, b):
+        v.set_precision(mixed)
+    h.kernel_timer("extrap")
+    converged = lmax < 6
+    for v, q in ((h, d.charge), (b, [d.charge, d.charge])):
+        if converged:
+            v.energy_forces(q)
+        else:
+            with pytest.raises(NotConverged):
+                v.energy_forces(q)
+    assert _two_launches(h)
+    for name in ("sigma", "s"):
+        one, two = h.get(name), b.get(name)
+        assert np.all(np.isfinite(one))
+        assert np.array_equal(one, two[:n]) and np.array_equal(one, two[n:]), name
+
+
+@pytest.mark.parametrize("star", [False, True])
+@pytest.mark.parametrize("n,lmax,ngrid", [(600, 2, 26), (1300, 6, 110)])
+def test_two_launch_solver_short_histories(n, lmax, ngrid, star):
+    from ddpcm_amd.ddx import DDCosmo
+    from ddpcm_amd.inputs import synthetic_input
+    x, y, z, r = synthetic_input(n, 5 + n, lmax, ngrid).bohr()
+    h = DDCosmo(x, y, z, r, lmax, ngrid)
+    rhs = np.random.default_rng(n).standard_normal((n, h.nylm))
+    x0 = h.get("facl")[None, :] * rhs
+    ref, _, ok = h.jacobi_diis(star, rhs, x0, tol=1e-12)
+    assert ok
+    h.kernel_timer("extrap")
+    for m in (11, 12, 18, 24):
+        got, _, ok = h.jacobi_diis(star, rhs, x0, diis_max=m, tol=1e-12)
+        assert _two_launches(h)
+        assert ok and h.hnorm(got - ref) <= 1e-10, m
