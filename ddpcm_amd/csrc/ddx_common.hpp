@@ -316,7 +316,7 @@ struct ddx_handle {
   double *h_stage = nullptr, *d_stage = nullptr, *h_out = nullptr, *d_out = nullptr;
   bool stage_busy = false, results_ok = false;
   bool setup_timed = false;       // events 0 and 6 bracket a setup not yet read
-  hipEvent_t gev[2] = {};           // completion of a group's state copy
+  hipEvent_t gev[2] = {};           // the ends of the two groups of rounds in flight
   int tag_solve = -1, tag_round = 0;  // attached to timed launches
 
   // problem data / results

@@ -82,8 +82,8 @@ int seg_sum(ddx_handle *h, hipStream_t s, const double *yp, double *y, const Dii
 // k_solver.hip — Jacobi/DIIS (jacobi_diis.f90:43-438), RHS, norms
 // Solves on lanes: solve_begin sets one up (x holds the guess); solve_run
 // iterates one solve, or a direct (star 0) and an adjoint (star 1) solve in
-// lockstep on one stream, enqueueing groups of iterations and reading the
-// DIIS states back between groups; solve_end reports each.
+// lockstep on one stream, enqueueing groups of iterations until the lanes'
+// records in pinned memory say done; solve_end reports each.
 // solve_jacobi_diis runs the three for one solve.
 // the state that gates a lane's kernels: the instance's own for a plain
 // handle, the summary of a batch

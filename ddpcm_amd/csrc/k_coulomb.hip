@@ -48,8 +48,11 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
 // workgroup of four waves (two per thread) 642 atoms made 61 workgroups.  That
 // form -> this one, in us (lmax, grid): 60 atoms (6, 302) 9.5 -> 5.9; 259 (6,
 // 110) 30 -> 17; 642 (6, 110) 71 -> 39; 200 (10, 1202) 27.5 -> 24.0; 1000 (8,
-// 590) 202 -> 195; 2000 (8, 590) 614 -> 601.  Two targets per lane in one wave:
-// 70 us at 642 atoms, 755 at 2000.
+// 590) 202 -> 195; 2000 (8, 590) 614 -> 601.  From there on either form may win
+// by what its last workgroups leave idle: with the field 2000 -> 1850 us at 3500
+// atoms, 4970 -> 4740 at 6000, 5010 -> 5110 at 6400, 9600 -> 9160 at 12 000 (302
+// points); without 1434 -> 1345, 3676 -> 3610, 3855 -> 3950, 7050 -> 6925.  Two
+// targets per lane in one wave: 70 us at 642 atoms, 755 at 2000, 5000 at 6400.
 template <bool FIELD>
 __global__ __launch_bounds__(kFW) void k_potential(const int4 *__restrict__ tiles,
                                                    const double *__restrict__ q,

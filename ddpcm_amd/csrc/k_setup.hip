@@ -1,8 +1,9 @@
 // Device setup of one ddCOSMO system (the per-geometry part of ddinit,
 // ddcosmo.f90:308-468), plus the triple lists the sweeps run on.
 //
-//   neighbours  CSR, increasing j, |c_i - c_j| <= r_i + r_j (ddcosmo.f90:308-324),
-//               found through a spatial hash in O(n) instead of the O(n^2) scan
+//   neighbours  CSR, increasing j, |c_i - c_j| <= r_i + r_j (ddcosmo.f90:308-324):
+//               by the O(n^2) scan where no instance has more than 4096
+//               spheres, else through a spatial hash in O(n)
 //   per point   fi = sum_j chi(t_n^ij), ui = max(0, 1 - fi) when fi <= 1,
 //               zi in the switch region (ddcosmo.f90:359-411), plus a 64-bit
 //               mask of the neighbours j with t_n^ij < 1
@@ -23,7 +24,10 @@
 // leaves the offsets within a sphere's points, the sums over spheres are one
 // scan launch, and the host waits once, for the five totals that size the
 // triple arrays.  60 atoms: 290 us with 45 launches and copies and three waits,
-// now 77 us with 13 launches and one wait; 2000 atoms 490 -> 181 us.
+// now 77 us with 13 launches and one wait; 2000 atoms 490 -> 181 us.  (On a
+// geometry no larger than an earlier one of the handle: one with more triples or
+// exposed points than all before also frees and allocates their arrays, 0.3 to
+// 0.6 ms at 300 to 1000 atoms.)
 #include "ddx_device.hpp"
 #include "ddx_kernels.hpp"
 
@@ -221,6 +225,12 @@ __device__ __forceinline__ int pair_of(const int *__restrict__ inl, const int *_
 // A sphere's points are cut into `runs` (1 or kRuns) runs of whole 64-point
 // groups, one wave each: four where the spheres alone would leave most of the
 // chip's 1024 SIMDs idle.  Run r of sphere i is number i runs + r.
+//   Whole setup with one run -> four, us (points): 60 atoms 109 -> 69 (302), 642
+// 92 -> 74 (110), 1000 189 -> 123 (590), 2000 220 -> 174 (590), 4000 139 -> 140
+// (110) and 337 -> 283 (590).  Four is the faster beyond the line as well, on
+// large grids (6000 494 -> 411 at 590 points, 20 000 765 -> 714 at 302; 12 000 at
+// 110 points 292 -> 289): the line only bounds the arrays that hold 64 counts to
+// a run.
 constexpr int kRuns = 4;
 constexpr int kRunSpheres = 4096;   // fewer spheres than this: kRuns
 

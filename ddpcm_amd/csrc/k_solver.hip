@@ -7,12 +7,16 @@
 //          system by Gauss-Jordan with full pivoting; x_new = sum c_i x_i
 //          (diis/makeb/gjinv, jacobi_diis.f90:198-400, drop-10 rule included)
 //   norm   hnorm(x_new - x) (matvec.f90:281-323); converged when < tol
-// as four kernels: k_jacobi (update + Gram-row partial sums, fused),
-// k_diis_small (one wave: B update, Gauss-Jordan, coefficients),
-// k_extrap (extrapolation, increment norm partials, x <- x_new) and
-// k_norm.  Their bookkeeping lives in a device DiisState; once it says
-// done every later kernel returns at once, so the host can enqueue several
-// iterations before it looks at the state.
+// as three kernels: k_jacobi (update + Gram-row partial sums, fused),
+// k_diis_small (the previous norm's test, B update, Gauss-Jordan by one wave,
+// coefficients) and k_extrap (extrapolation, increment norm partials,
+// x <- x_new); without DIIS k_norm takes the second one's place.  Single
+// systems take forms arranged for latency: k_jacobi_two and k_extrap_one up to
+// 512 elements a workgroup, and up to one workgroup of both solves to a compute
+// unit k_diis_extrap, the last two kernels in one launch.  The bookkeeping
+// lives in a device DiisState; once it says done every later kernel returns
+// at once, so the host can enqueue iterations ahead.  The kernel that ends a
+// solve writes its results to a record in pinned memory, which the host polls.
 //
 // A handle may hold a batch of independent instances (molecules): each has
 // its own DiisState and converges on its own, exactly as if solved alone.
@@ -300,7 +304,9 @@ __device__ __forceinline__ void copy_state(DiisState *st) {
 //    the same bits) instead of one six-stage sum each.
 // Average launch of k_jacobi -> this kernel: 12.5 -> 5.8 us at 60 atoms, 18.9 ->
 // 7.7 us at 200 atoms and lmax 10, 12.1 -> 7.7 us at 1000, 14.8 -> 12.5 us at
-// 2000 atoms (lmax 8).
+// 2000, 31.2 -> 26.9 us at 4096, 40.5 -> 37.4 us at 6400 atoms (lmax 8, the last
+// size that it takes; FP32 history 35.9 -> 28.6); 36.0 in both at 20 000 atoms
+// and lmax 4.
 template <typename E>
 __global__ __launch_bounds__(kJThreads) void k_jacobi_two(unsigned nn, unsigned nylm,
                                                           int diis_max, unsigned nbj,
@@ -396,7 +402,7 @@ __device__ __forceinline__ double lane_value(double v, int src) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-constexpr int kSmallThreads = 256;       // 4 workgroup partials per thread
+constexpr int kSmallThreads = 256;
 
 // Tells the host, which polls the record, that the solve has ended.  Once per
 // solve: a copy of the state's header after every second round cost two
@@ -971,7 +977,7 @@ __device__ __forceinline__ double extrapolate(const double *__restrict__ xd, uns
 // each of 256 threads took 198 registers and two rounds of workgroups at 2000
 // atoms.  Average launch of k_extrap -> this kernel: 9.2 -> 4.6 us at 60 atoms,
 // 12.1 -> 6.9 us at 200 atoms and lmax 10, 13.2 -> 9.0 us at 1000, 15.7 -> 14.2
-// us at 2000 atoms (lmax 8; near its bytes there).
+// us at 2000 atoms (lmax 8; near its bytes there), 43.2 -> 37.5 us at 6400.
 constexpr int kExtrapThreads = 512;
 
 __global__ __launch_bounds__(kExtrapThreads) void k_extrap_one(
@@ -1745,8 +1751,8 @@ int run_groups(ddx_handle *h, Lane *const *lanes, int count) {
       continue;
     }
     if (queued == 0) break;
-    // poll the record beside the group's event for about a millisecond,
-    // then sleep on the event
+    // poll the record beside the group's event for about a millisecond (the
+    // calling thread is busy for that long), then sleep on the event
     hipError_t e = hipErrorNotReady;
     for (int spin = 0; spin < 1000 && e == hipErrorNotReady; ++spin) {
       if (lanes_done(lanes, count)) return DDX_OK;

@@ -15,7 +15,7 @@
 // cf = facs * 4pi/(2l+1) is applied outside the triple loop: L X contracts
 // with X' = cf X (16 values to a vector register, read by row broadcast),
 // L* S accumulates sum_t coef_t p~ trig in registers per lane and multiplies
-// by cf after one LDS transpose reduction per container.  When the direct
+// by cf after one register reduce-scatter per segment.  When the direct
 // and the adjoint solve run in lockstep a single pass over the triples
 // builds each basis once for both.
 // The basis follows ylmbas (ddcosmo.f90:830-895) with t^l folded into the
@@ -389,12 +389,12 @@ __device__ __forceinline__ void sweep_pass(
   R acc[NA];
 #pragma unroll
   for (int k = 0; k < NA; ++k) acc[k] = R(0);
-  // software pipeline, two triples deep: geometry, slot and owner point of
-  // triple k + 128 and xi of triple k + 64 load while triple k is evaluated
   typedef typename Geo<R>::G4 G4;
   typedef typename Geo<R>::G2 G2;
   int k = beg + lane_id();
   if constexpr (F) {
+    // Software pipeline, two triples deep: geometry, slot and owner point of
+    // triple k + 128 and xi of triple k + 64 load while triple k is evaluated.
     // Indices past the chunk read its last triple instead, so that no load
     // is conditional, and the loop is unrolled by three so that the three
     // stages rotate by name (a register copy of a load in flight waits for
@@ -574,7 +574,7 @@ __device__ __forceinline__ int xcd_block(int b, int n) {
 // sphere, gates: the summaries after ninst instance states) so is every
 // container of an instance that has converged.
 // (two waves per SIMD: the register budget that keeps a block of
-// accumulators and the two-deep load pipeline without spilling)
+// accumulators, X' and the loads ahead without spilling)
 template <typename R, int LMAX, bool DIR, bool ADJ>
 __global__ __launch_bounds__(kWave * kSweepWaves, 2) void k_sweep(
     int G, const int4 *__restrict__ wstart, const int *__restrict__ uoff,
