@@ -410,9 +410,10 @@ int create(ddx_handle **out, int n, int count, const int *nsph, const double *x,
     const size_t in = 5 * (size_t)n * sizeof(double);
     const size_t res = (3 * (size_t)n + count) * sizeof(double);
     char *hp = nullptr, *dp = nullptr;
-    // (coherent: the host polls the lanes' records while kernels run)
-    if (hipHostMalloc((void **)&hp, 2 * rec + cnt + in + res,
-                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    // (coherent: the host polls the lanes' records while kernels run; mapped
+    // and portable as by default)
+    const unsigned kind = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
+    if (hipHostMalloc((void **)&hp, 2 * rec + cnt + in + res, kind) != hipSuccess) {
       set_error("hipHostMalloc failed");
       return fail(DDX_ERR_ALLOC);
     }
